@@ -9,6 +9,7 @@
 #pragma clang fp contract(off)
 
 #include "hk_internal.h"
+#include "hk_mfma.h"
 #include "hk_synth.h"
 
 namespace hk {
@@ -159,59 +160,196 @@ struct SynthSrc {
 
 // ------------------------------------------------------------------ packers over f32 buffers
 
-__global__ void pack_q4_kernel(const float* __restrict__ w, size_t groups, int G,
-                               uint16_t* __restrict__ scales, uint8_t* __restrict__ codes,
-                               uint32_t* bad) {
-    for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups;
-         g += (size_t)gridDim.x * blockDim.x) {
-        uint32_t b = 0;
-        q4_pack_group(BufSrc{w + g * G}, G, scales + g, codes + g * (G / 2), &b);
-        if (b) atomicOr(bad, 1u);
+// A thread owns 8 consecutive weights and a group is G / 8 neighbouring lanes
+// (G <= 128: at most 16, inside one DPP row), so a wave reads 2 KiB of
+// consecutive bytes and its maximum, sum and codes need no LDS.  With one
+// thread per group (loads 4 G bytes apart, each line fetched again for every
+// element) a 2048 x 7168 Q4 pack took 490 us; it takes 15 us here, 4.3 TB/s of
+// the 4 bytes a weight read and the codes written.
+__device__ __forceinline__ void load8(const float* w, bool v4, float (&v)[8]) {
+    if (v4) {
+        const float4* p = reinterpret_cast<const float4*>(w);
+        const float4 a = ldg(p), b = ldg(p + 1);
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+        v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = ldg(w + k);
     }
 }
 
-__global__ void pack_bin_kernel(const float* __restrict__ w, size_t groups,
-                                uint16_t* __restrict__ scales, uint8_t* __restrict__ signs,
-                                uint32_t* bad) {
-    for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups;
-         g += (size_t)gridDim.x * blockDim.x) {
-        uint32_t b = 0;
-        bin_pack_group(BufSrc{w + g * 128}, scales + g, signs + g * 16, &b);
-        if (b) atomicOr(bad, 1u);
+// max |v| over the group's lanes (every lane gets it); *bad: a non-finite
+// value among this lane's.
+template <int NL>
+__device__ __forceinline__ float group_max_abs(const float (&v)[8], bool* bad) {
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        *bad |= !isfinite(v[k]);
+        m = fmaxf(m, fabsf(v[k]));
     }
+    return group_max<NL>(m);
 }
 
-__global__ void pack_q2_kernel(const float* __restrict__ w, size_t groups,
-                               uint16_t* __restrict__ scales, uint8_t* __restrict__ codes,
-                               uint32_t* bad) {
-    for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups;
-         g += (size_t)gridDim.x * blockDim.x) {
-        uint32_t b = 0;
-        q2_pack_group(BufSrc{w + g * 64}, scales + g, codes + g * 16, &b);
-        if (b) atomicOr(bad, 1u);
-    }
+// Chunks [0, n8) of 8 weights, whole groups of NL chunks each: the lanes of
+// a group are active together (the grid's stride is whole waves).
+template <class F>
+__device__ __forceinline__ void for_chunks(size_t n8, F f) {
+    for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < n8; c += (size_t)gridDim.x * blockDim.x) f(c);
 }
 
-__global__ void pack_q8_kernel(const float* __restrict__ w, size_t groups, uint16_t* __restrict__ scales,
-                               uint8_t* __restrict__ codes, uint32_t* bad) {
-    for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups;
-         g += (size_t)gridDim.x * blockDim.x) {
-        uint32_t b = 0;
-        q8_pack_group(BufSrc{w + g * 64}, scales + g, codes + g * 64, &b);
-        if (b) atomicOr(bad, 1u);
-    }
+template <int G>
+__global__ void __launch_bounds__(256) pack_q4_kernel(const float* __restrict__ w, size_t groups,
+                                                      uint16_t* __restrict__ scales, uint8_t* __restrict__ codes,
+                                                      uint32_t* flag, bool v4) {
+    constexpr int NL = G / 8;
+    for_chunks(groups * NL, [&](size_t c) {
+        float v[8];
+        load8(w + 8 * c, v4, v);
+        bool bad = false;
+        const uint16_t sb = f32_to_f16_bits(__fdiv_rn(group_max_abs<NL>(v, &bad), 7.0f));
+        bad |= (sb & 0x7C00u) == 0x7C00u;
+        const float rs = f16_bits_to_f32(sb);
+        uint32_t word = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            int q = 0;
+            if (rs != 0.0f) q = (int)fminf(fmaxf(rintf(__fdiv_rn(v[k], rs)), -8.0f), 7.0f);
+            word |= (uint32_t)(q + 8) << (4 * k);
+        }
+        reinterpret_cast<uint32_t*>(codes)[c] = word;
+        if (c % NL == 0) scales[c / NL] = sb;
+        if (bad) atomicOr(flag, 1u);
+    });
 }
 
-__global__ void pack_u3_kernel(const float* __restrict__ w, size_t count, uint16_t* __restrict__ scales,
-                               uint8_t* __restrict__ codes, uint32_t* bad) {
-    const size_t groups = (count + 63) / 64;
-    for (size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x; g < groups;
-         g += (size_t)gridDim.x * blockDim.x) {
+__device__ __forceinline__ double group_sum16(double v) {
+    auto step = [](double x, auto partner) {
+        const uint64_t b = __builtin_bit_cast(uint64_t, x);
+        const uint64_t o = (uint64_t)partner((uint32_t)b) | ((uint64_t)partner((uint32_t)(b >> 32)) << 32);
+        return x + __builtin_bit_cast(double, o);
+    };
+    v = step(v, [](uint32_t x) { return xor_partner<1>(x); });
+    v = step(v, [](uint32_t x) { return xor_partner<2>(x); });
+    v = step(v, [](uint32_t x) { return xor_partner<4>(x); });
+    return step(v, [](uint32_t x) { return xor_partner<8>(x); });
+}
+
+// The reference sums |w| in index order in f64.  When the group's nonzero
+// magnitudes span at most 2^21 every partial sum of any order is exact (a
+// multiple of 2^(e_min - 23) below 2^(e_max + 8): 53 bits), so the lanes' tree
+// gives the same bits; a wider group is summed in index order by one lane.
+__global__ void __launch_bounds__(256) pack_bin_kernel(const float* __restrict__ w, size_t groups,
+                                                       uint16_t* __restrict__ scales, uint8_t* __restrict__ signs,
+                                                       uint32_t* flag, bool v4) {
+    for_chunks(groups * 16, [&](size_t c) {
+        float v[8];
+        load8(w + 8 * c, v4, v);
+        bool bad = false;
+        uint32_t bits = 0, lo = 0xFFFFFFFFu, hi = 0;
+        double sum = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            bad |= !isfinite(v[k]);
+            const uint32_t m = __float_as_uint(v[k]) & 0x7FFFFFFFu;
+            lo = min(lo, m - 1u);  // zero wraps to the top: only nonzero magnitudes count
+            hi = max(hi, m);
+            sum += (double)fabsf(v[k]);
+            bits |= v[k] >= 0.0f ? 1u << k : 0u;
+        }
+        signs[c] = (uint8_t)bits;
+        lo = group_reduce<16>(lo, [](uint32_t a, uint32_t b) { return min(a, b); });
+        hi = group_reduce<16>(hi, [](uint32_t a, uint32_t b) { return max(a, b); });
+        sum = group_sum16(sum);
+        if (c % 16 == 0) {
+            const uint32_t e_min = max((lo + 1u) >> 23, 1u), e_max = hi >> 23;
+            if (hi != 0u && e_max > e_min + 21u) {
+                sum = 0.0;
+                for (int i = 0; i < 128; ++i) sum += (double)fabsf(w[8 * c + (size_t)i]);
+            }
+            scales[c / 16] = f32_to_f16_bits((float)(sum / 128.0));
+        }
+        if (bad) atomicOr(flag, 1u);
+    });
+}
+
+__global__ void __launch_bounds__(256) pack_q2_kernel(const float* __restrict__ w, size_t groups,
+                                                      uint16_t* __restrict__ scales, uint8_t* __restrict__ codes,
+                                                      uint32_t* flag, bool v4) {
+    for_chunks(groups * 8, [&](size_t c) {
+        float v[8];
+        load8(w + 8 * c, v4, v);
+        bool bad = false;
+        const uint16_t sb = f32_to_f16_bits(__fdiv_rn(group_max_abs<8>(v, &bad), 1.5f));
+        const float sf = f16_bits_to_f32(sb), denom = sf > 0.0f ? sf : 1.0f;
+        uint32_t word = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            word |= (uint32_t)fminf(fmaxf(rintf(__fdiv_rn(v[k], denom) + 1.5f), 0.0f), 3.0f) << (2 * k);
+        reinterpret_cast<uint16_t*>(codes)[c] = (uint16_t)word;
+        if (c % 8 == 0) scales[c / 8] = sb;
+        if (bad) atomicOr(flag, 1u);
+    });
+}
+
+// A uniform group of 64 (bound 127 or 3): the f16 scale, and this lane's 8
+// codes q + bound (the quantizer divides by the f32 scale).
+template <int BOUND>
+__device__ __forceinline__ uint16_t uniform_codes(const float (&v)[8], uint32_t (&code)[8], bool* bad) {
+    const float scale = __fdiv_rn(group_max_abs<8>(v, bad), (float)BOUND);
+    const uint16_t sb = f32_to_f16_bits(scale);
+    *bad |= (sb & 0x7C00u) == 0x7C00u;
+    const float denom = scale > 0.0f ? scale : 1.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        code[k] = (uint32_t)((int)fminf(fmaxf(roundf(__fdiv_rn(v[k], denom)), -(float)BOUND), (float)BOUND) + BOUND);
+    return sb;
+}
+
+__global__ void __launch_bounds__(256) pack_q8_kernel(const float* __restrict__ w, size_t groups,
+                                                      uint16_t* __restrict__ scales, uint8_t* __restrict__ codes,
+                                                      uint32_t* flag, bool v4) {
+    for_chunks(groups * 8, [&](size_t c) {
+        float v[8];
+        load8(w + 8 * c, v4, v);
+        bool bad = false;
+        uint32_t q[8];
+        const uint16_t sb = uniform_codes<127>(v, q, &bad);
+        reinterpret_cast<uint2*>(codes)[c] =
+            make_uint2(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24));
+        if (c % 8 == 0) scales[c / 8] = sb;
+        if (bad) atomicOr(flag, 1u);
+    });
+}
+
+// Values past `count` in the last group pack as 0.  A lane's 8 codes are 24
+// bits; the group's 8 lanes' 192 bits leave as the 6 words of lanes 0-5 (word
+// j starts in lane 4 j / 3 at bit 8 (4 j % 3)).
+__global__ void __launch_bounds__(256) pack_u3_kernel(const float* __restrict__ w, size_t count,
+                                                      uint16_t* __restrict__ scales, uint8_t* __restrict__ codes,
+                                                      uint32_t* flag, bool v4) {
+    for_chunks((count + 63) / 64 * 8, [&](size_t c) {
+        float v[8];
+        if (8 * c + 8 <= count) {
+            load8(w + 8 * c, v4, v);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = 8 * c + k < count ? w[8 * c + k] : 0.0f;
+        }
+        bool bad = false;
+        uint32_t q[8];
+        const uint16_t sb = uniform_codes<3>(v, q, &bad);
         uint32_t b = 0;
-        const uint32_t nv = (uint32_t)(count - g * 64 < 64 ? count - g * 64 : 64);
-        u3_pack_group(BufSrc{w + g * 64}, nv, scales + g, codes + g * 24, &b);
-        if (b) atomicOr(bad, 1u);
-    }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) b |= q[k] << (3 * k);
+        const uint32_t lane = threadIdx.x & 63u, j = lane & 7u, s = (lane & ~7u) + min(4u * j / 3u, 6u), off = 8u * (4u * j % 3u);
+        const uint32_t b0 = __shfl(b, (int)s, 64), b1 = __shfl(b, (int)(s + 1u), 64);
+        const uint64_t two = (uint64_t)b0 | ((uint64_t)b1 << 24);
+        // bits off .. off + 31 of lanes s and s + 1: off <= 16, so 48 bits suffice
+        if (j < 6u) reinterpret_cast<uint32_t*>(codes)[6 * (c / 8) + j] = (uint32_t)(two >> off);
+        if (j == 0u) scales[c / 8] = sb;
+        if (bad) atomicOr(flag, 1u);
+    });
 }
 
 __global__ void synth_normal_kernel(uint64_t key, uint64_t first, size_t count, float sigma,
@@ -227,37 +365,43 @@ static unsigned grid_for(size_t n, unsigned block) {
     return (unsigned)(b ? b : 1);
 }
 
-hipError_t launch_pack_q4(const float* w, size_t groups, int G, uint16_t* scales, uint8_t* codes,
-                          uint32_t* bad, hipStream_t s) {
-    hipLaunchKernelGGL(pack_q4_kernel, dim3(grid_for(groups, 256)), dim3(256), 0, s, w, groups, G,
-                       scales, codes, bad);
+// 256 threads of 8 weights a block, and whether the weights allow 16-byte loads.
+static unsigned pack_grid(size_t chunks) { return grid_for(chunks, 256); }
+static bool vec4(const float* w) { return (reinterpret_cast<uintptr_t>(w) & 15u) == 0; }
+
+hipError_t launch_pack_q4(const float* w, size_t groups, int G, uint16_t* scales, uint8_t* codes, uint32_t* bad,
+                          hipStream_t s) {
+    const dim3 grid(pack_grid(groups * (size_t)(G / 8)));
+    auto* k = G == 32 ? pack_q4_kernel<32> : G == 64 ? pack_q4_kernel<64> : pack_q4_kernel<128>;
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, s, w, groups, scales, codes, bad, vec4(w));
     return hipGetLastError();
 }
 
-hipError_t launch_pack_bin(const float* w, size_t groups, uint16_t* scales, uint8_t* signs,
-                           uint32_t* bad, hipStream_t s) {
-    hipLaunchKernelGGL(pack_bin_kernel, dim3(grid_for(groups, 256)), dim3(256), 0, s, w, groups,
-                       scales, signs, bad);
+hipError_t launch_pack_bin(const float* w, size_t groups, uint16_t* scales, uint8_t* signs, uint32_t* bad,
+                           hipStream_t s) {
+    hipLaunchKernelGGL(pack_bin_kernel, dim3(pack_grid(groups * 16)), dim3(256), 0, s, w, groups, scales, signs, bad,
+                       vec4(w));
     return hipGetLastError();
 }
 
 hipError_t launch_pack_q8(const float* w, size_t groups, uint16_t* scales, uint8_t* codes, uint32_t* bad,
                           hipStream_t s) {
-    hipLaunchKernelGGL(pack_q8_kernel, dim3(grid_for(groups, 256)), dim3(256), 0, s, w, groups, scales, codes, bad);
+    hipLaunchKernelGGL(pack_q8_kernel, dim3(pack_grid(groups * 8)), dim3(256), 0, s, w, groups, scales, codes, bad,
+                       vec4(w));
     return hipGetLastError();
 }
 
 hipError_t launch_pack_u3(const float* w, size_t count, uint16_t* scales, uint8_t* codes, uint32_t* bad,
                           hipStream_t s) {
-    hipLaunchKernelGGL(pack_u3_kernel, dim3(grid_for((count + 63) / 64, 256)), dim3(256), 0, s, w, count, scales,
-                       codes, bad);
+    hipLaunchKernelGGL(pack_u3_kernel, dim3(pack_grid((count + 63) / 64 * 8)), dim3(256), 0, s, w, count, scales, codes,
+                       bad, vec4(w));
     return hipGetLastError();
 }
 
-hipError_t launch_pack_q2(const float* w, size_t groups, uint16_t* scales, uint8_t* codes,
-                          uint32_t* bad, hipStream_t s) {
-    hipLaunchKernelGGL(pack_q2_kernel, dim3(grid_for(groups, 256)), dim3(256), 0, s, w, groups,
-                       scales, codes, bad);
+hipError_t launch_pack_q2(const float* w, size_t groups, uint16_t* scales, uint8_t* codes, uint32_t* bad,
+                          hipStream_t s) {
+    hipLaunchKernelGGL(pack_q2_kernel, dim3(pack_grid(groups * 8)), dim3(256), 0, s, w, groups, scales, codes, bad,
+                       vec4(w));
     return hipGetLastError();
 }
 
