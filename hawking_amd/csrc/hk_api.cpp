@@ -319,7 +319,14 @@ extern "C" int hk_ctx_create(int device, hk_ctx** out) {
     }
     (void)hipMemset(st, 0, 512);
     ctx->dev_status = static_cast<uint32_t*>(st);
-    ctx->pack_flag = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(st) + 256);
+    ctx->mixed_words = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(st) + 256);
+    void* flag = nullptr;
+    if (hipHostMalloc(&flag, 256, hipHostMallocDefault) != hipSuccess) {
+        (void)hipFree(st);
+        delete ctx;
+        return HK_E_NOMEM;
+    }
+    ctx->pack_flag = static_cast<uint32_t*>(flag);
     *out = ctx;
     return HK_OK;
 }
@@ -329,6 +336,7 @@ extern "C" void hk_ctx_destroy(hk_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipDeviceSynchronize();
     if (ctx->dev_status) (void)hipFree(ctx->dev_status);
+    if (ctx->pack_flag) (void)hipHostFree(const_cast<uint32_t*>(ctx->pack_flag));
     delete ctx;
 }
 
@@ -1053,20 +1061,21 @@ extern "C" int hk_decode_rows(hk_ctx* ctx, const hk_organ* o, uint32_t row0, uin
 
 // ====================================================================== packers / generator
 
-static int finish_pack(hk_ctx* ctx, hipStream_t st, uint32_t* bad_dev, hipError_t launch) {
-    int rc = check_hip(ctx, launch, "pack launch");
-    if (rc) return rc;
-    uint32_t bad = 0;
-    rc = check_hip(ctx, hipMemcpyAsync(&bad, bad_dev, 4, hipMemcpyDeviceToHost, st), "pack status read");
-    if (!rc) rc = check_hip(ctx, hipStreamSynchronize(st), "hipStreamSynchronize (pack)");
-    if (rc) return rc;
-    if (bad) return set_error(ctx, HK_E_NONFINITE, "source tensor contains a non-finite value or scale");
-    return HK_OK;
+static int pack_verdict(hk_ctx* ctx, uint32_t bad) {
+    return bad ? set_error(ctx, HK_E_NONFINITE, "source tensor contains a non-finite value or scale") : HK_OK;
 }
 
-static int pack_prologue(hk_ctx* ctx, hipStream_t st, uint32_t** bad) {
-    *bad = ctx->pack_flag;
-    return check_hip(ctx, hipMemsetAsync(ctx->pack_flag, 0, 4, st), "hipMemsetAsync (pack flag)");
+// Waits for a packer launched after `*ctx->pack_flag = 0` and reads its flag.
+static int finish_pack(hk_ctx* ctx, hipStream_t st, hipError_t launch) {
+    int rc = check_hip(ctx, launch, "pack launch");
+    if (!rc) rc = check_hip(ctx, hipStreamSynchronize(st), "hipStreamSynchronize (pack)");
+    return rc ? rc : pack_verdict(ctx, *ctx->pack_flag);
+}
+
+// The flag of a call's launch, cleared.
+static uint32_t* pack_flag(hk_ctx* ctx) {
+    *ctx->pack_flag = 0u;
+    return const_cast<uint32_t*>(ctx->pack_flag);
 }
 
 extern "C" int hk_pack_q4(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t cols, int32_t group,
@@ -1077,10 +1086,8 @@ extern "C" int hk_pack_q4(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t c
     if (!w || !scales || !codes || !aligned16(codes) || !aligned16(w))
         return set_error(ctx, HK_E_INVALID_ARG, "hk_pack_q4: NULL or misaligned pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* bad;
-    if ((rc = pack_prologue(ctx, st, &bad))) return rc;
     const size_t groups = (size_t)rows * cols / (size_t)group;
-    return finish_pack(ctx, st, bad, launch_pack_q4(w, groups, group, scales, codes, bad, st));
+    return finish_pack(ctx, st, launch_pack_q4(w, groups, group, scales, codes, pack_flag(ctx), st));
 }
 
 extern "C" int hk_pack_bin(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t cols, uint16_t* scales,
@@ -1091,9 +1098,7 @@ extern "C" int hk_pack_bin(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t 
     if (!w || !scales || !signs || !aligned16(signs))
         return set_error(ctx, HK_E_INVALID_ARG, "hk_pack_bin: NULL or misaligned pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* bad;
-    if ((rc = pack_prologue(ctx, st, &bad))) return rc;
-    return finish_pack(ctx, st, bad, launch_pack_bin(w, (size_t)rows * cols / 128, scales, signs, bad, st));
+    return finish_pack(ctx, st, launch_pack_bin(w, (size_t)rows * cols / 128, scales, signs, pack_flag(ctx), st));
 }
 
 extern "C" int hk_pack_q8(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t cols, uint16_t* scales,
@@ -1104,9 +1109,7 @@ extern "C" int hk_pack_q8(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t c
     if (!w || !scales || !codes || !aligned16(codes))
         return set_error(ctx, HK_E_INVALID_ARG, "hk_pack_q8: NULL or misaligned pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* bad;
-    if ((rc = pack_prologue(ctx, st, &bad))) return rc;
-    return finish_pack(ctx, st, bad, launch_pack_q8(w, (size_t)rows * cols / 64, scales, codes, bad, st));
+    return finish_pack(ctx, st, launch_pack_q8(w, (size_t)rows * cols / 64, scales, codes, pack_flag(ctx), st));
 }
 
 extern "C" int hk_pack_u3(hk_ctx* ctx, const float* w, size_t count, uint16_t* scales, uint8_t* codes,
@@ -1116,10 +1119,7 @@ extern "C" int hk_pack_u3(hk_ctx* ctx, const float* w, size_t count, uint16_t* s
     if (!w || !scales || !codes || !aligned16(codes))
         return set_error(ctx, HK_E_INVALID_ARG, "hk_pack_u3: NULL or misaligned pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* bad;
-    int rc;
-    if ((rc = pack_prologue(ctx, st, &bad))) return rc;
-    return finish_pack(ctx, st, bad, launch_pack_u3(w, count, scales, codes, bad, st));
+    return finish_pack(ctx, st, launch_pack_u3(w, count, scales, codes, pack_flag(ctx), st));
 }
 
 extern "C" int hk_pack_binary_rice(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t cols, double ratio,
@@ -1166,10 +1166,7 @@ extern "C" int hk_pack_q2(hk_ctx* ctx, const float* w, size_t count, uint16_t* s
     if (!w || !scales || !codes || !aligned16(codes))
         return set_error(ctx, HK_E_INVALID_ARG, "hk_pack_q2: NULL or misaligned pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* bad;
-    int rc;
-    if ((rc = pack_prologue(ctx, st, &bad))) return rc;
-    return finish_pack(ctx, st, bad, launch_pack_q2(w, count / 64, scales, codes, bad, st));
+    return finish_pack(ctx, st, launch_pack_q2(w, count / 64, scales, codes, pack_flag(ctx), st));
 }
 
 extern "C" int hk_pack_mixed(hk_ctx* ctx, const float* w, uint32_t rows, uint32_t cols, const uint8_t* is_binary,
@@ -1188,12 +1185,10 @@ extern "C" int hk_pack_mixed(hk_ctx* ctx, const float* w, uint32_t rows, uint32_
     const size_t groups = (size_t)rows * cols / 128;
     if (groups > 0xFFFFFFFFull) return set_error(ctx, HK_E_GEOMETRY, "hk_pack_mixed: more than 2^32 groups");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // pass 1: tags and the binary count (into the packer flag's neighbour word)
-    uint32_t* bad;
-    if ((rc = pack_prologue(ctx, st, &bad))) return rc;
-    uint32_t* count = ctx->pack_flag + 1;
-    uint32_t nb = 0;
-    rc = check_hip(ctx, hipMemsetAsync(count, 0, 4, st), "hipMemsetAsync (mixed count)");
+    // pass 1: tags and the binary count
+    uint32_t *bad = ctx->mixed_words, *count = bad + 1;
+    uint32_t nb = 0, bad_host = 0;
+    rc = check_hip(ctx, hipMemsetAsync(bad, 0, 8, st), "hipMemsetAsync (mixed flag and count)");
     if (!rc) rc = check_hip(ctx, launch_mixed_tags_from_sel(is_binary, groups, tags, count, st), "mixed tags");
     if (!rc) rc = check_hip(ctx, hipMemcpyAsync(&nb, count, 4, hipMemcpyDeviceToHost, st), "mixed count read");
     if (!rc) rc = check_hip(ctx, hipStreamSynchronize(st), "hipStreamSynchronize (mixed count)");
@@ -1222,10 +1217,11 @@ extern "C" int hk_pack_mixed(hk_ctx* ctx, const float* w, uint32_t rows, uint32_
     j.row_q2 = reinterpret_cast<uint32_t*>(tp + align256(sizeof(SynthJob)) + align256(((size_t)rows + 1) * 4));
     j.w = w;
     rc = check_hip(ctx, hipMemcpyAsync(tmp, &j, sizeof(j), hipMemcpyHostToDevice, st), "mixed job upload");
-    if (!rc) rc = finish_pack(ctx, st, bad, launch_mixed_pack_buffer(static_cast<SynthJob*>(tmp), groups, bad, st));
+    if (!rc) rc = check_hip(ctx, launch_mixed_pack_buffer(static_cast<SynthJob*>(tmp), groups, bad, st), "pack launch");
+    if (!rc) rc = check_hip(ctx, hipMemcpyAsync(&bad_host, bad, 4, hipMemcpyDeviceToHost, st), "pack status read");
     (void)hipStreamSynchronize(st);
     (void)hipFree(tmp);
-    return rc;
+    return rc ? rc : pack_verdict(ctx, bad_host);
 }
 
 extern "C" uint64_t hk_stream_key(uint64_t seed, uint64_t stream_id) { return hk::stream_key(seed, stream_id); }

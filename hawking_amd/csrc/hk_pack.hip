@@ -178,6 +178,10 @@ __device__ __forceinline__ void load8(const float* w, bool v4, float (&v)[8]) {
     }
 }
 
+// The packers' non-finite flag, which may be host memory (no atomics there;
+// every writer stores the same word).
+__device__ __forceinline__ void raise(uint32_t* flag) { *const_cast<volatile uint32_t*>(flag) = 1u; }
+
 // max |v| over the group's lanes (every lane gets it); *bad: a non-finite
 // value among this lane's.
 template <int NL>
@@ -219,7 +223,7 @@ __global__ void __launch_bounds__(256) pack_q4_kernel(const float* __restrict__ 
         }
         reinterpret_cast<uint32_t*>(codes)[c] = word;
         if (c % NL == 0) scales[c / NL] = sb;
-        if (bad) atomicOr(flag, 1u);
+        if (bad) raise(flag);
     });
 }
 
@@ -269,7 +273,7 @@ __global__ void __launch_bounds__(256) pack_bin_kernel(const float* __restrict__
             }
             scales[c / 16] = f32_to_f16_bits((float)(sum / 128.0));
         }
-        if (bad) atomicOr(flag, 1u);
+        if (bad) raise(flag);
     });
 }
 
@@ -288,7 +292,7 @@ __global__ void __launch_bounds__(256) pack_q2_kernel(const float* __restrict__ 
             word |= (uint32_t)fminf(fmaxf(rintf(__fdiv_rn(v[k], denom) + 1.5f), 0.0f), 3.0f) << (2 * k);
         reinterpret_cast<uint16_t*>(codes)[c] = (uint16_t)word;
         if (c % 8 == 0) scales[c / 8] = sb;
-        if (bad) atomicOr(flag, 1u);
+        if (bad) raise(flag);
     });
 }
 
@@ -318,7 +322,7 @@ __global__ void __launch_bounds__(256) pack_q8_kernel(const float* __restrict__ 
         reinterpret_cast<uint2*>(codes)[c] =
             make_uint2(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24));
         if (c % 8 == 0) scales[c / 8] = sb;
-        if (bad) atomicOr(flag, 1u);
+        if (bad) raise(flag);
     });
 }
 
@@ -348,7 +352,7 @@ __global__ void __launch_bounds__(256) pack_u3_kernel(const float* __restrict__ 
         // bits off .. off + 31 of lanes s and s + 1: off <= 16, so 48 bits suffice
         if (j < 6u) reinterpret_cast<uint32_t*>(codes)[6 * (c / 8) + j] = (uint32_t)(two >> off);
         if (j == 0u) scales[c / 8] = sb;
-        if (bad) atomicOr(flag, 1u);
+        if (bad) raise(flag);
     });
 }
 
