@@ -579,8 +579,14 @@ extern "C" int hk_gemv(hk_ctx* ctx, const hk_organ* o, const float* x, float* y,
     if (rc) return rc;
     // the single-organ descriptor was uploaded with the organ
     hipStream_t st = static_cast<hipStream_t>(stream);
-    rc = check_hip(ctx, launch_gemv_tiled(static_cast<const OrganView*>(o->view_dev), 1, o->view, x, 0, y, 0, st),
-                   "gemv launch");
+    const OrganView* dev = static_cast<const OrganView*>(o->view_dev);
+    bool fused = false;
+    if (o->res_dev)
+        rc = check_hip(ctx, launch_gemv_rice(dev, o->res_dev, &o->res, 1, o->view, o->res8_pieces_256, o->res8_pieces, x, 0,
+                                             y, 0, st, &fused),
+                       "gemv launch");
+    if (rc || fused) return rc;
+    rc = check_hip(ctx, launch_gemv_tiled(dev, 1, o->view, x, 0, y, 0, st), "gemv launch");
     if (!rc && o->res_dev)
         rc = check_hip(ctx, launch_rice_apply(o->res_dev, 1, o->view.rows, o->view.cols, o->res_pieces, x, 0, y, 0, st),
                        "rice apply");
@@ -702,7 +708,7 @@ extern "C" int hk_gemv_set(hk_ctx* ctx, const hk_organ_set* set, const float* x,
     bool fused = false;
     if (set->res_dev)
         rc = check_hip(ctx,
-                       launch_gemv_rice(set->dev, set->res_dev, set->n, set->first, set->res8_pieces_256,
+                       launch_gemv_rice(set->dev, set->res_dev, nullptr, set->n, set->first, set->res8_pieces_256,
                                         set->res8_pieces, x, x_stride, y, y_stride, st, &fused),
                        "gemv_set launch");
     if (!rc && !fused)

@@ -8,6 +8,7 @@
 // tiles' MFMAs and the next step's weight loads are in flight while the
 // current step computes.
 #include "hk_mfma.h"
+#include "hk_rice.h"
 
 namespace hk {
 
@@ -647,6 +648,221 @@ static hipError_t launch_kind(const OrganView* organs, uint32_t n, const OrganVi
     return hipGetLastError();
 }
 
+// ------------------------------------------------------------------ small launches
+//
+// One organ, or a set with too few row tiles to fill the chip: the time is a
+// chain of memory round trips, not bandwidth.  gemv_split_kernel splits each
+// row tile's steps over KS waves of its workgroup (TS = waves / KS tiles side
+// by side), so a tile's weights are all in flight at once instead of two
+// steps at a time in one wave, and every thread of the workgroup builds its
+// part of the x image.  A single organ's view comes with the kernel
+// arguments (one round trip fewer than a descriptor load).
+struct SplitArgs {
+    OrganView one;            // n = 1: the organ
+    const OrganView* organs;  // else the set's table
+    ResView res_one;          // RES, the same way
+    const ResView* res;
+    const float* x;
+    float* y;
+    size_t x_stride, y_stride;
+    uint32_t n, parts;        // organs, workgroups per organ
+    uint32_t tpw;             // tiles per workgroup, a multiple of TS
+    uint32_t ks_log, ts_log;  // log2 KS, log2 TS
+};
+
+// LDS: the x image, then (RES) a copy of x and the residual's products, then
+// the terms of every (tile, step) {scale, v} (ORD with KS > 1) or one partial
+// row sum per (K slice, row), then (RES) the rows' base sums.
+template <int KIND, bool ORD, bool RES>
+struct SplitLds {
+    size_t xs, vals, terms, ysh, total;
+    __host__ __device__ SplitLds(uint32_t S, uint32_t cols, uint32_t tpw, uint32_t ks) {
+        constexpr size_t TERM = KIND == HK_MIXED ? 16 : 8;
+        xs = (x_lds_bytes<KIND>(S) + 15u) & ~(size_t)15;
+        vals = xs + (RES ? (size_t)cols * 4u : 0);
+        terms = vals + (RES ? (size_t)RICE_BATCH * 4u : 0);
+        ysh = terms + (ORD && ks > 1 ? (size_t)tpw * S * 64u * TERM : (size_t)ks * tpw * 64u);
+        total = ysh + (RES ? (size_t)tpw * 64u : 0);
+    }
+};
+
+constexpr size_t SPLIT_LDS_LIMIT = 96 * 1024;
+
+// ORD: a row's terms are added in step order whatever KS is: the waves leave
+// each lane's {scale, v} in LDS and one wave per tile runs the same chain of
+// fused multiply-adds that one wave walking the tile would, so the sums are
+// the streamed launches' to the bit.  Otherwise (Q4, Q8: 16 to 128 steps) each
+// wave sums its own slice and the slices are added in order.
+// RES: the HGRAVR02 residual added to the base sums in the same launch (256
+// threads; records loaded before the image build).
+template <int KIND, int D, bool ORD, bool RES>
+__global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs a) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    uint32_t oi, part;
+    organ_part(blockIdx.x, a.parts, a.n, &oi, &part);
+    OrganView o = a.one;
+    ResView rv = a.res_one;
+    if (a.organs) {
+        o = a.organs[oi];
+        if constexpr (RES) rv = a.res[oi];
+    }
+    const float* __restrict__ x = a.x + (size_t)oi * a.x_stride;
+    float* __restrict__ y = a.y + (size_t)oi * a.y_stride;
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nthr = blockDim.x;
+    const uint32_t S = o.steps, KS = 1u << a.ks_log, TS = 1u << a.ts_log;
+    const uint32_t ksl = wave & (KS - 1u), tsl = wave >> a.ks_log;
+    const uint32_t per = (S + KS - 1u) >> a.ks_log, s0 = min(ksl * per, S), ns = min(per, S - s0);
+    const uint32_t t0 = part * a.tpw, t1 = min(t0 + a.tpw, o.n_tiles), tf = t0 + tsl;
+    const uint32_t n = tf < t1 ? ((t1 - tf + TS - 1u) >> a.ts_log) * ns : 0u;  // this wave's (tile, step) items
+    const SplitLds<KIND, ORD, RES> M(S, o.cols, a.tpw, KS);
+
+    constexpr int NC = 2;
+    XChunks<NC> xc;
+    load_x<NC>(BlockTeam{}, x, o.cols, xc);
+    RiceTile rt;
+    const uint32_t r0 = t0 * 16u, r1 = min(t1 * 16u, o.rows);
+    if constexpr (RES) rice_ranges(rv, r0, r1, rt);
+    // the first D items, unconditionally (a wave with fewer re-reads its last)
+    uint32_t fT = n ? tf : t0, fs = n ? s0 : 0u, fi = 0;
+    auto step_on = [&]() {
+        if (++fi < n) {
+            ++fs;
+            if (fs == s0 + ns) {
+                fs = s0;
+                fT += TS;
+            }
+        }
+    };
+    Frag<KIND, 1> f[D];
+    if constexpr (KIND == HK_MIXED) {
+        uint4 h[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            h[d] = ldg(o.hdr + (fT * S + fs));
+            step_on();
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) fetch_mixed<1>(o, h[d], lane, f[d], 0);
+    } else {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            fetch_one<KIND, 1, false>(o, fT, fs, lane, f[d], 0);
+            step_on();
+        }
+    }
+    if constexpr (RES) rice_first_records(rv, rt);
+
+    const uint32_t nch = S * (uint32_t)Kcfg<KIND>::STEP_COLS / 8u;
+    float* sx = reinterpret_cast<float*>(lds + (size_t)S * Kcfg<KIND>::P * A_TILE_STRIDE);
+    float* xs = reinterpret_cast<float*>(lds + M.xs);
+    for (uint32_t i = threadIdx.x; i < S * (uint32_t)Kcfg<KIND>::P; i += nthr)
+        *reinterpret_cast<uint4*>(lds + (size_t)i * A_TILE_STRIDE + 256u) = make_uint4(0u, 0u, 0u, 0u);
+    auto image = [&](uint32_t ch, float4 (&v)[2]) {
+        if constexpr (RES) {
+            if (8u * ch < o.cols) {
+                reinterpret_cast<float4*>(xs)[2u * ch] = v[0];
+                reinterpret_cast<float4*>(xs)[2u * ch + 1u] = v[1];
+            }
+        }
+        (void)image_chunk<KIND>(ch, v, lds, sx, 0u, 0u);
+    };
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const uint32_t ch = threadIdx.x + nthr * (uint32_t)j;
+        if (ch < nch) image(ch, xc.v[j]);
+    }
+    for (uint32_t ch = threadIdx.x + nthr * NC; ch < nch; ch += nthr) {
+        float4 v[2];
+        load_chunk(x, 8u * ch, o.cols, v);
+        image(ch, v);
+    }
+    __syncthreads();
+
+    const ImageA A{lds, a_lane_offset(lane)};
+    float* terms = reinterpret_cast<float*>(lds + M.terms);
+    const bool split = ORD && KS > 1u;
+    float acc = 0.0f;
+    uint32_t cT = tf, cs = s0;
+    auto consume = [&](const Frag<KIND, 1>& fr) {
+        if (split) {
+            constexpr uint32_t NT = KIND == HK_MIXED ? 2u : 1u;
+            float2* o2 = reinterpret_cast<float2*>(terms) + ((cT - t0) * S + cs) * 64u * NT + (uint32_t)lane * NT;
+            uint32_t k = 0;
+            compute_terms<KIND, 1>(fr, cs, A, sx, q, [&](int, float s, float v) { o2[k++] = make_float2(s, v); });
+        } else {
+            compute_step<KIND, 1>(fr, cs, A, sx, q, &acc);
+            if (cs + 1u == s0 + ns) {
+                const float v = tile_row_sum(acc);
+                if (lane < 16) terms[(ksl * a.tpw + cT - t0) * 16u + (uint32_t)lane] = v;
+                acc = 0.0f;
+            }
+        }
+        ++cs;
+        if (cs == s0 + ns) {
+            cs = s0;
+            cT += TS;
+        }
+    };
+    uint32_t it = 0;
+    for (; it + D < n; it += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            consume(f[d]);
+            fetch_one<KIND, 1, false>(o, fT, fs, lane, f[d], 0);
+            step_on();
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (it + (uint32_t)d < n) consume(f[d]);
+    __syncthreads();
+
+    float* ysh = reinterpret_cast<float*>(lds + M.ysh);
+    auto put = [&](uint32_t i, float v) {  // row i of the workgroup
+        if constexpr (RES) ysh[i] = v;
+        else if (r0 + i < o.rows) y[r0 + i] = v;
+    };
+    if (split) {
+        constexpr uint32_t NT = KIND == HK_MIXED ? 2u : 1u;
+        for (uint32_t T = wave; T < t1 - t0; T += nthr >> 6) {
+            const float2* t2 = reinterpret_cast<const float2*>(terms) + T * S * 64u * NT + (uint32_t)lane * NT;
+            float v = 0.0f;
+#pragma unroll 4
+            for (uint32_t s = 0; s < S; ++s)
+#pragma unroll
+                for (uint32_t h = 0; h < NT; ++h) {
+                    const float2 e = t2[s * 64u * NT + h];
+                    v = __builtin_fmaf(e.x, e.y, v);
+                }
+            v = tile_row_sum(v);
+            if (lane < 16) put(T * 16u + (uint32_t)lane, v);
+        }
+    } else {
+        for (uint32_t i = threadIdx.x; i < (t1 - t0) * 16u; i += nthr) {
+            float v = terms[i];
+            // (slices past the last step hold no sums)
+            for (uint32_t k = 1; k * per < S && k < KS; ++k) v += terms[k * a.tpw * 16u + i];
+            put(i, v);
+        }
+    }
+    if constexpr (RES) {
+        __syncthreads();
+        float racc[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t i = threadIdx.x + 256u * (uint32_t)h;
+            racc[h] = r0 + i < r1 ? ysh[i] : 0.0f;
+        }
+        rice_batches_from(rv, rt, rt.e0 & ~7u, racc, xs, reinterpret_cast<float*>(lds + M.vals));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t row = r0 + threadIdx.x + 256u * (uint32_t)h;
+            if (row < r1) y[row] = racc[h];
+        }
+    }
+}
+
 // Launch shape (R tiles per wave group, D steps in flight, tiles per
 // workgroup) by kind and size, from sweeps over the streamed workloads:
 // binary 2-tile groups 5 deep, over 16 tiles when the organ has >= 4 steps
@@ -692,10 +908,97 @@ static hipError_t launch_kind(const OrganView* organs, uint32_t n, const OrganVi
 #define HK_MIX_D 3
 #define HK_MIX_TPW 16
 #endif
+struct SplitShape {
+    uint32_t waves, ks, tpw;  // waves 0: the launch is not split
+};
+
+static uint32_t pow2_ceil(uint32_t v) {
+    uint32_t p = 1;
+    while (p < v) p *= 2u;
+    return p;
+}
+
+// Where the split pays and its shape (us per launch in a graph of one launch,
+// split against the walk of gemv_tiled_kernel; organs of 512 x 2048 unless
+// stated):
+//   * one step (<= 512 binary columns): nothing to split (2.92 against 2.89);
+//   * up to 2,048 row tiles the workgroups are what is scarce: about one per
+//     CU, so tpw = tiles / 256 rounded up to a power of two, and as many waves
+//     as the steps and the image (one chunk of 8 columns a thread) employ.
+//     One Q4 2048 x 7168: 15.2 -> 5.0, q8 4096 x 2048: 7.6 -> 3.5, binary:
+//     3.74 -> 3.11, mixed: 4.4 -> 3.2; 20 mixed organs (640 tiles): 5.3 -> 3.9;
+//     40 Q4 organs: 7.3 -> 4.8;
+//   * up to 4,096 tiles Q4 and q8 (long rows) still gain from four slices (80
+//     Q4 organs: 9.7 -> 9.4, with 7168 columns 30.8 -> 24.7), the short kinds
+//     from one wave per tile without slices (mixed 6.05 -> 5.63, binary 5.07 ->
+//     4.88);
+//   * beyond, q8 (160 organs: 29.1 -> 26.0; 320: 60.2 -> 54.4) and mixed
+//     (8.9 -> 8.05) up to the streamed shapes; the others' walk is faster
+//     (binary 320 organs: 9.7 against 10.8; Q4 with 7168 columns 99 against 107).
+// RES (256 threads, at most 4 tiles a workgroup: a row's records are one
+// thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8 ->
+// 6.7, 512 x 7168: 35.4 -> 8.9; above 4,096 tiles the two launches are faster
+// (160 organs: 11.0 against 11.8).
+static SplitShape split_shape(int kind, bool res, uint64_t tiles, uint32_t S, uint32_t cols) {
+    if (tiles >= 16384) return {0, 0, 0};
+    const uint32_t s2 = pow2_ceil(S);
+    uint32_t tpw = std::min(pow2_ceil((uint32_t)((tiles + 255) / 256)), 8u);
+    if (res) {
+        if (tiles > 4096) return {0, 0, 0};
+        tpw = std::min(tpw, 4u);
+        const uint32_t ks = std::min(std::max(4u / tpw, 1u), s2);
+        return {4, ks, std::max(tpw, 4u / ks)};
+    }
+    if (S == 1) return {0, 0, 0};
+    const bool wide = kind == HK_Q4 || kind == HK_Q8;
+    if (tiles <= 2048) {
+        const uint32_t w = cols > 4096 ? 16u : S >= 16 ? (tpw >= 4 ? 16u : 8u) : tpw == 1 ? 4u : 8u;
+        const uint32_t ks = std::min(std::max(w / tpw, 1u), s2);
+        return {w, ks, std::max(tpw, w / ks)};
+    }
+    if (wide && S >= 16 && (tiles <= 4096 || kind == HK_Q8)) return {8, kind == HK_Q8 ? 8u : 4u, 2};
+    if (!wide && (tiles <= 4096 || kind == HK_MIXED)) return {4, 1, 4};
+    return {0, 0, 0};
+}
+
+template <int KIND, bool RES>
+static hipError_t launch_split(const OrganView* organs, const ResView* res, const ResView* res_one, uint32_t n,
+                               const OrganView& sh, const float* x, size_t xs, float* y, size_t ys, hipStream_t s,
+                               bool* done) {
+    constexpr bool ORD = KIND != HK_Q4 && KIND != HK_Q8;
+    constexpr int D = KIND == HK_MIXED ? 2 : 4;
+    *done = false;
+    SplitShape c = split_shape(KIND, RES, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
+    if (!c.waves) return hipSuccess;
+    const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw;
+    const size_t lds = SplitLds<KIND, ORD, RES>(sh.steps, sh.cols, tpw, ks).total;
+    if (lds > SPLIT_LDS_LIMIT) return hipSuccess;
+    *done = true;
+    SplitArgs a{};
+    a.ks_log = (uint32_t)__builtin_ctz(ks);
+    a.ts_log = (uint32_t)__builtin_ctz(waves / ks);
+    a.one = sh;
+    a.organs = n > 1 ? organs : nullptr;
+    if (res_one) a.res_one = *res_one;
+    a.res = res;
+    a.x = x;
+    a.y = y;
+    a.x_stride = xs;
+    a.y_stride = ys;
+    a.n = n;
+    a.parts = (sh.n_tiles + tpw - 1) / tpw;
+    a.tpw = tpw;
+    hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES>), dim3(a.parts * n), dim3(64u * waves), lds, s, a);
+    return hipGetLastError();
+}
+
 template <int KIND>
 static hipError_t launch_r(const OrganView* organs, uint32_t n, const OrganView& sh, const float* x, size_t xs,
                            float* y, size_t ys, hipStream_t s) {
     const uint64_t tiles = (uint64_t)n * sh.n_tiles;
+    bool done = false;
+    const hipError_t e = launch_split<KIND, false>(organs, nullptr, nullptr, n, sh, x, xs, y, ys, s, &done);
+    if (e != hipSuccess || done) return e;
     if (tiles >= 16384) {
         if constexpr (KIND == HK_BIN) {
             if (sh.steps >= 4)
@@ -755,10 +1058,15 @@ hipError_t launch_head_fused(const OrganView* organ_dev, const OrganView& sh, co
     return hipGetLastError();
 }
 
-hipError_t launch_gemv_rice(const OrganView* organs_dev, const ResView* res_dev, uint32_t n, const OrganView& sh,
-                            uint32_t pieces256, uint32_t pieces512, const float* x, size_t x_stride, float* y,
-                            size_t y_stride, hipStream_t s, bool* fused) {
+hipError_t launch_gemv_rice(const OrganView* organs_dev, const ResView* res_dev, const ResView* res_one, uint32_t n,
+                            const OrganView& sh, uint32_t pieces256, uint32_t pieces512, const float* x,
+                            size_t x_stride, float* y, size_t y_stride, hipStream_t s, bool* fused) {
     *fused = false;
+    if (sh.kind == HK_BIN) {
+        const hipError_t e = launch_split<HK_BIN, true>(organs_dev, res_dev, res_one, n, sh, x, x_stride, y, y_stride, s,
+                                                        fused);
+        if (e != hipSuccess || *fused) return e;
+    }
     // the streamed binary shapes (launch_r), with x in one register chunk
     if (sh.kind != HK_BIN || (uint64_t)n * sh.n_tiles < 16384 || x_image_cols<HK_BIN>(sh.steps) > 2048u)
         return hipSuccess;

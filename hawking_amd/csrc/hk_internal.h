@@ -303,13 +303,14 @@ int check_hip(hk_ctx* ctx, hipError_t e, const char* what);
 size_t gemv_lds_bytes(int kind, uint32_t cols);
 constexpr size_t GEMV_LDS_LIMIT = 64 * 1024;
 struct ResView;
-// The binary GEMV of HGRAVR02 organs with the residual added in its
-// epilogue (the bits of launch_gemv_tiled then launch_rice_apply); pieces256
-// / pieces512: rice_part_pieces of the organs for 256- and 512-row parts.
+// The binary GEMV of HGRAVR02 organs with the residual added in the same
+// launch (the bits of launch_gemv_tiled then launch_rice_apply); res_one: a
+// host copy of the residual's view for n = 1 (else null); pieces256 /
+// pieces512: rice_part_pieces8 of the organs for 256- and 512-row parts.
 // *fused = false (nothing launched) when the launch shape has no fused form.
-hipError_t launch_gemv_rice(const OrganView* organs_dev, const ResView* res_dev, uint32_t n, const OrganView& sh,
-                            uint32_t pieces256, uint32_t pieces512, const float* x, size_t x_stride, float* y,
-                            size_t y_stride, hipStream_t s, bool* fused);
+hipError_t launch_gemv_rice(const OrganView* organs_dev, const ResView* res_dev, const ResView* res_one, uint32_t n,
+                            const OrganView& sh, uint32_t pieces256, uint32_t pieces512, const float* x,
+                            size_t x_stride, float* y, size_t y_stride, hipStream_t s, bool* fused);
 // The read-only bandwidth control (hk_control.hip).
 hipError_t launch_stream_control(const void* data, size_t nbytes, float* out, uint32_t workgroups, hipStream_t s);
 hipError_t launch_gemv_tiled(const OrganView* organs_dev, uint32_t n, const OrganView& shape,

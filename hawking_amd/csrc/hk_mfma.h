@@ -691,12 +691,13 @@ __device__ __forceinline__ void fetch_step(const OrganView& o, const uint32_t* T
     for (int r = 0; r < R; ++r) fetch_one<KIND, R, NT>(o, r < nvalid ? T[r] : T[0], t, lane, f, r);
 }
 
-// Consume one fetched step: acc[r] += this lane's partial dot, in units of
-// 2^-E (slots fetched for aliased tiles accumulate junk the caller drops).
-// A(tau) yields this lane's A operand of x-image tile tau.
-template <int KIND, int R, class ASrc>
-__device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t, const ASrc& A, const float* SX,
-                                             int q, float* acc) {
+// Consume one fetched step: emit(r, scale, v) for each of this lane's terms
+// scale * v of the dot, in order (one per step; a mixed step has two, one per
+// 64-column half), in units of 2^-E.  A(tau) yields this lane's A operand of
+// x-image tile tau.
+template <int KIND, int R, class ASrc, class Emit>
+__device__ __forceinline__ void compute_terms(const Frag<KIND, R>& f, uint32_t t, const ASrc& A, const float* SX,
+                                              int q, const Emit& emit) {
     v4i c[R];
     if constexpr (KIND == HK_BIN) {
 #pragma unroll
@@ -714,7 +715,7 @@ __device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t,
         }
         const float2 u = reinterpret_cast<const float2*>(SX)[4 * t + q];
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += f16_bits_to_f32(f.s[r]) * (combine_limbs(c[r]) * u.x - u.y);
+        for (int r = 0; r < R; ++r) emit(r, f16_bits_to_f32(f.s[r]), __builtin_fmaf(combine_limbs(c[r]), u.x, -u.y));
     } else if constexpr (KIND == HK_Q4) {
         const uint32_t m = 0x0F0F0F0Fu;
         const v4i alo = A(t * 2), ahi = A(t * 2 + 1);
@@ -728,7 +729,7 @@ __device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t,
         }
         const float2 u = reinterpret_cast<const float2*>(SX)[4 * t + q];
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += f16_bits_to_f32(f.s[r]) * (combine_limbs(c[r]) * u.x - u.y);
+        for (int r = 0; r < R; ++r) emit(r, f16_bits_to_f32(f.s[r]), __builtin_fmaf(combine_limbs(c[r]), u.x, -u.y));
     } else if constexpr (KIND == HK_Q8) {
         // code - 127 = (code ^ 0x80 as a signed byte) + 1: the B bytes are the
         // codes with the top bit flipped and the +1 is the slot's sum of X
@@ -741,7 +742,7 @@ __device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t,
         }
         const float2 u = reinterpret_cast<const float2*>(SX)[4 * t + q];
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += f16_bits_to_f32(f.s[r]) * (combine_limbs(c[r]) * u.x - u.y);
+        for (int r = 0; r < R; ++r) emit(r, f16_bits_to_f32(f.s[r]), __builtin_fmaf(combine_limbs(c[r]), u.x, -u.y));
     } else if constexpr (KIND == HK_U3) {
 #pragma unroll
         for (int r = 0; r < R; ++r) c[r] = v4i{0, 0, 0, 0};
@@ -759,7 +760,7 @@ __device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t,
         }
         const float2 u = reinterpret_cast<const float2*>(SX)[4 * t + q];
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] += f16_bits_to_f32(f.s[r]) * (combine_limbs(c[r]) * u.x - u.y);
+        for (int r = 0; r < R; ++r) emit(r, f16_bits_to_f32(f.s[r]), __builtin_fmaf(combine_limbs(c[r]), u.x, -u.y));
     } else {
         // field u of a byte is bits 2u..2u+1 (binary: bit 2u; the odd bits come
         // from the copy shifted down by one).  A Q2 item's bit 7 is stored
@@ -807,9 +808,18 @@ __device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t,
             }
 #pragma unroll
             for (int r = 0; r < R; ++r)
-                acc[r] += f16_bits_to_f32(h ? f.s1[r] : f.s0[r]) * (combine_limbs(c[r]) * uh[h][r].x - uh[h][r].y);
+                emit(r, f16_bits_to_f32(h ? f.s1[r] : f.s0[r]),
+                     __builtin_fmaf(combine_limbs(c[r]), uh[h][r].x, -uh[h][r].y));
         }
     }
+}
+
+// Consume one fetched step: acc[r] += this lane's partial dot, in units of
+// 2^-E (slots fetched for aliased tiles accumulate junk the caller drops).
+template <int KIND, int R, class ASrc>
+__device__ __forceinline__ void compute_step(const Frag<KIND, R>& f, uint32_t t, const ASrc& A, const float* SX,
+                                             int q, float* acc) {
+    compute_terms<KIND, R>(f, t, A, SX, q, [&](int r, float s, float v) { acc[r] = __builtin_fmaf(s, v, acc[r]); });
 }
 
 // Sum the four column-slot partials of a tile: every lane gets its row's total.
