@@ -1243,14 +1243,16 @@ extern "C" int hk_synth_normal(hk_ctx* ctx, uint64_t key, uint64_t first, size_t
 
 // ====================================================================== terminal head
 
-// The head's launches: fused for a q8 lm_head the fused GEMV takes, else norm,
+// The head's launches: fused for an lm_head the fused GEMV takes, else norm,
 // GEMV and pick.  `pick` holds 16 zero bytes and is left zeroed.
 static int head_greedy(hk_ctx* ctx, const float* hidden, const float* norm_w, float eps, const hk_organ* lm_head,
                        uint32_t n_valid, float* xn, float* logits, uint64_t* pick, int32_t* token, hipStream_t st) {
-    if (head_gemv_fusable(lm_head->view) && aligned16(norm_w) && aligned16(xn))
+    // (a residual is not part of the fused GEMV, and kinds other than q8 keep
+    // hk_gemv's alignment rule for the logits)
+    if (head_gemv_fusable(lm_head->view) && !lm_head->res_dev && aligned16(norm_w) && aligned16(xn) &&
+        (lm_head->view.kind == HK_Q8 || aligned16(logits)))
         return check_hip(ctx,
-                         launch_head_fused(static_cast<const OrganView*>(lm_head->view_dev), lm_head->view, hidden,
-                                           norm_w, eps, xn, logits, n_valid, pick, token, ctx->dev_status, st),
+                         launch_head_fused(lm_head->view, hidden, norm_w, eps, xn, logits, n_valid, pick, token, ctx->dev_status, st),
                          "terminal head");
     int rc = check_hip(ctx, launch_head_norm(hidden, norm_w, lm_head->view.cols, eps, xn, token, pick,
                                              ctx->dev_status, st),

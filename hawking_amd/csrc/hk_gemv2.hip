@@ -108,6 +108,18 @@ __device__ __forceinline__ uint64_t greedy_key(float v, uint32_t i) {
     return ((uint64_t)ord << 32) | (uint64_t)(~i);
 }
 
+// The block's largest key into key[0], one atomic (every thread calls this;
+// kred: one word per wave).
+__device__ __forceinline__ void fold_key(uint64_t best, uint64_t* kred, uint64_t* key) {
+    for (int off = 32; off; off >>= 1) best = max(best, (uint64_t)__shfl_xor((unsigned long long)best, off, 64));
+    if ((threadIdx.x & 63) == 0) kred[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (uint32_t w = 1; w < (blockDim.x >> 6); ++w) best = max(best, kred[w]);
+        if (best) atomicMax(reinterpret_cast<unsigned long long*>(key), (unsigned long long)best);
+    }
+}
+
 // Block-wide sum (every thread gets it); red: one float per wave.
 __device__ __forceinline__ float block_sum_f(float v, float* red) {
     v = wave_sum(v);
@@ -123,7 +135,7 @@ __device__ __forceinline__ float block_sum_f(float v, float* red) {
 // xn = h * (1 / sqrt(mean(h^2) + eps)) * (1 + w) on this thread's register
 // chunks of h (source_qwen80_residual_rms_norm,
 // model/qwen80_complete_runtime.rs:6778-6797); every chunk of h must be in
-// registers (cols <= 8 * 256 * NC), and gw holds the same chunks of w
+// registers (cols <= 8 * block size * NC), and gw holds the same chunks of w
 // (loaded with h, before the first weight steps: vector loads retire in
 // issue order, so a w load issued after them would hold the norm until the
 // weights land).
@@ -142,7 +154,7 @@ __device__ __forceinline__ void head_norm_chunks(XChunks<NC>& xc, const XChunks<
     const float inv = 1.0f / sqrtf(sum / (float)cols + ha.eps);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
-        const uint32_t c0 = 8u * (threadIdx.x + 256u * (uint32_t)j);
+        const uint32_t c0 = 8u * (threadIdx.x + blockDim.x * (uint32_t)j);
         if (c0 < cols) {
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
@@ -209,15 +221,13 @@ __device__ __forceinline__ void fetch_step_or_dummy(const OrganView& o, const ui
     fetch_step<KIND, R, NT>(op, Tz, nvalid, past ? 0u : t, lane, f);
 }
 
-template <int KIND, int R, int D, int NC, bool HEAD, bool RES = false>
+template <int KIND, int R, int D, int NC, bool RES = false>
 __global__ void __launch_bounds__(256)
 gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const float* __restrict__ xall,
                   size_t x_stride, float* __restrict__ yall, size_t y_stride, uint32_t tiles_per_wg, uint32_t parts,
-                  uint32_t* status, HeadArgs ha, ResArgs ra) {
-    static_assert(!RES || (KIND == HK_BIN && NC == 1 && !HEAD), "the fused residual is for binary organs");
+                  ResArgs ra) {
+    static_assert(!RES || (KIND == HK_BIN && NC == 1), "the fused residual is for binary organs");
     extern __shared__ __align__(16) uint8_t lds[];
-    __shared__ float red[4];
-    __shared__ uint64_t kred[HEAD ? 4 : 1];
     uint32_t oi, part;
     organ_part(blockIdx.x, parts, n_organs, &oi, &part);
     const OrganView o = organs[oi];
@@ -230,13 +240,11 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
     W.n = W.g0 < t1 ? ((t1 - W.g0 + W.gstride - 1) / W.gstride) * o.steps : 0;
     const uint32_t last = W.n ? W.n - 1u : 0u;
 
-    // x (and for HEAD the norm weight) first, then (mixed) this workgroup's
+    // x first, then (mixed) this workgroup's
     // step headers, then the first D steps' weight loads, all before the
     // image build
     XChunks<NC> xc;
     load_x<NC>(BlockTeam{}, x, o.cols, xc);
-    XChunks<HEAD ? NC : 1> gw;  // HEAD: the norm weight's chunks, with x
-    if constexpr (HEAD) load_x<NC>(BlockTeam{}, ha.norm_w, o.cols, gw);
     const uint32_t nh = (t1 - t0) * o.steps;
     uint4 hreg[GEMV_HDR_PER_THREAD];
     uint4* hsh = reinterpret_cast<uint4*>(lds + gemv_hdr_offset<KIND>(o.steps));
@@ -258,8 +266,8 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             P.at(min((uint32_t)d, last), T[d], R, &nv[d], &ts[d]);
-            if constexpr (KIND == HK_MIXED) fetch_step<KIND, R, !HEAD>(o, T[d], nv[d], ts[d], lane, f[d]);
-            else fetch_step_or_dummy<KIND, R, !HEAD>(o, T[d], nv[d], ts[d], lane, f[d], (uint32_t)d > last);
+            if constexpr (KIND == HK_MIXED) fetch_step<KIND, R, true>(o, T[d], nv[d], ts[d], lane, f[d]);
+            else fetch_step_or_dummy<KIND, R, true>(o, T[d], nv[d], ts[d], lane, f[d], (uint32_t)d > last);
         }
     }
     if constexpr (KIND == HK_MIXED) {
@@ -284,11 +292,9 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
             my1[h] = ldg(rv.row_ptr8 + min(row + 1u, r1));
         }
     }
-    if constexpr (HEAD) head_norm_chunks<NC>(xc, gw, o.cols, ha, red);
     // the x image with E = 0: every thread scatters its own chunks (no
     // block-wide maximum, no gather pass); a unit's chunks are consecutive
     // threads, active together
-    bool bad = false;
     {
         const uint32_t nch = o.steps * (uint32_t)Kcfg<KIND>::STEP_COLS / 8u;
         float* sxw = reinterpret_cast<float*>(lds + (size_t)o.steps * Kcfg<KIND>::P * A_TILE_STRIDE);
@@ -296,19 +302,16 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
             const uint32_t ch = threadIdx.x + 256u * (uint32_t)j;
-            if (ch < nch) bad |= image_chunk<KIND>(ch, xc.v[j], lds, sxw, 0u, 0u);
+            if (ch < nch) (void)image_chunk<KIND>(ch, xc.v[j], lds, sxw, 0u, 0u);
         }
         for (uint32_t ch = threadIdx.x + 256u * NC; ch < nch; ch += 256u) {
             float4 v[2];
             load_chunk(x, 8u * ch, o.cols, v);
-            bad |= image_chunk<KIND>(ch, v, lds, sxw, 0u, 0u);
+            (void)image_chunk<KIND>(ch, v, lds, sxw, 0u, 0u);
         }
         __syncthreads();
     }
     const int E = 0;
-    if (bad && status) atomicOr(status, 1u);
-    if constexpr (HEAD)
-        if (bad) atomicOr(reinterpret_cast<uint32_t*>(ha.key + 1), 1u);
 
     const ImageA A{lds, a_lane_offset(lane)};
     const float* SX = reinterpret_cast<const float*>(lds + (size_t)o.steps * Kcfg<KIND>::P * A_TILE_STRIDE);
@@ -334,7 +337,7 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
                     fetch_mixed<R>(o, hsh[(Tr - t0) * o.steps + ts[d]], lane, f[d], r);
                 }
             } else {
-                fetch_step_or_dummy<KIND, R, !HEAD>(o, T[d], nv[d], ts[d], lane, f[d], it + D + d > last);
+                fetch_step_or_dummy<KIND, R, true>(o, T[d], nv[d], ts[d], lane, f[d], it + D + d > last);
             }
         }
     }
@@ -400,24 +403,9 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
         }
         return;
     }
-    uint64_t best = 0;
     for (uint32_t i = threadIdx.x; i < nrows; i += blockDim.x) {
         const uint32_t row = t0 * 16u + i;
-        if (row < o.rows) {
-            const float v = ldexpf(ysh[i], -E);
-            y[row] = v;
-            if constexpr (HEAD)
-                if (row < ha.n_valid) best = max(best, greedy_key(v, row));
-        }
-    }
-    if constexpr (HEAD) {
-        for (int off = 32; off; off >>= 1) best = max(best, (uint64_t)__shfl_xor((unsigned long long)best, off, 64));
-        if ((threadIdx.x & 63) == 0) kred[threadIdx.x >> 6] = best;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            best = max(max(kred[0], kred[1]), max(kred[2], kred[3]));
-            if (best) atomicMax(reinterpret_cast<unsigned long long*>(ha.key), (unsigned long long)best);
-        }
+        if (row < o.rows) y[row] = ldexpf(ysh[i], -E);
     }
 }
 
@@ -629,10 +617,9 @@ size_t gemv_lds_bytes(int kind, uint32_t cols) {
     return gemv_hdr_offset<HK_MIXED>(S) + (size_t)GEMV_MAX_MIXED_TILES_PER_WG * S * sizeof(uint4) + ysh;
 }
 
-template <int KIND, int R, int D, bool HEAD = false, bool RES = false>
+template <int KIND, int R, int D, bool RES = false>
 static hipError_t launch_kind(const OrganView* organs, uint32_t n, const OrganView& sh, const float* x,
-                              size_t xs, float* y, size_t ys, uint32_t tpw, hipStream_t s, const HeadArgs& ha = {},
-                              uint32_t* status = nullptr, const ResArgs& ra = {}) {
+                              size_t xs, float* y, size_t ys, uint32_t tpw, hipStream_t s, const ResArgs& ra = {}) {
     const uint32_t parts = (sh.n_tiles + tpw - 1) / tpw;
     const dim3 grid(parts * n);
     // image + one quantization window (2048 columns); x chunks held in
@@ -640,11 +627,11 @@ static hipError_t launch_kind(const OrganView* organs, uint32_t n, const OrganVi
     const uint32_t kc = x_image_cols<KIND>(sh.steps);
     const size_t lds = gemv_ysh_offset<KIND, RES>(sh.steps, tpw, sh.cols, ra.pieces) + (size_t)tpw * 16u * sizeof(float);
     if (kc <= 2048u)
-        hipLaunchKernelGGL((gemv_tiled_kernel<KIND, R, D, 1, HEAD, RES>), grid, dim3(256), lds, s, organs, n, x, xs, y,
-                           ys, tpw, parts, status, ha, ra);
+        hipLaunchKernelGGL((gemv_tiled_kernel<KIND, R, D, 1, RES>), grid, dim3(256), lds, s, organs, n, x, xs, y, ys,
+                           tpw, parts, ra);
     else if constexpr (!RES)
-        hipLaunchKernelGGL((gemv_tiled_kernel<KIND, R, D, 4, HEAD>), grid, dim3(256), lds, s, organs, n, x, xs, y, ys,
-                           tpw, parts, status, ha, ra);
+        hipLaunchKernelGGL((gemv_tiled_kernel<KIND, R, D, 4>), grid, dim3(256), lds, s, organs, n, x, xs, y, ys, tpw,
+                           parts, ra);
     return hipGetLastError();
 }
 
@@ -668,6 +655,8 @@ struct SplitArgs {
     uint32_t n, parts;        // organs, workgroups per organ
     uint32_t tpw;             // tiles per workgroup, a multiple of TS
     uint32_t ks_log, ts_log;  // log2 KS, log2 TS
+    HeadArgs ha;              // HEAD: the terminal head's prologue and epilogue
+    uint32_t* status;
 };
 
 // LDS: the x image, then (RES) a copy of x and the residual's products, then
@@ -695,9 +684,14 @@ constexpr size_t SPLIT_LDS_LIMIT = 96 * 1024;
 // wave sums its own slice and the slices are added in order.
 // RES: the HGRAVR02 residual added to the base sums in the same launch (256
 // threads; records loaded before the image build).
-template <int KIND, int D, bool ORD, bool RES>
+// HEAD: x is the hidden state; the prologue forms RMSNorm(1+w) of it and the
+// epilogue folds the rows' greedy keys (HeadArgs; cols <= 8192, 512 threads).
+template <int KIND, int D, bool ORD, bool RES, bool HEAD>
 __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs a) {
+    static_assert(!(RES && HEAD), "an lm_head has no fused residual");
     extern __shared__ __align__(16) uint8_t lds[];
+    __shared__ float red[HEAD ? 16 : 1];
+    __shared__ uint64_t kred[HEAD ? 16 : 1];
     uint32_t oi, part;
     organ_part(blockIdx.x, a.parts, a.n, &oi, &part);
     OrganView o = a.one;
@@ -717,9 +711,11 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     const uint32_t n = tf < t1 ? ((t1 - tf + TS - 1u) >> a.ts_log) * ns : 0u;  // this wave's (tile, step) items
     const SplitLds<KIND, ORD, RES> M(S, o.cols, a.tpw, KS);
 
-    constexpr int NC = 2;
+    constexpr int NC = 2;  // (HEAD: 512 threads x 2 chunks = 8192 columns, all in registers)
     XChunks<NC> xc;
     load_x<NC>(BlockTeam{}, x, o.cols, xc);
+    XChunks<HEAD ? NC : 1> gw;
+    if constexpr (HEAD) load_x<NC>(BlockTeam{}, a.ha.norm_w, o.cols, gw);
     RiceTile rt;
     const uint32_t r0 = t0 * 16u, r1 = min(t1 * 16u, o.rows);
     if constexpr (RES) rice_ranges(rv, r0, r1, rt);
@@ -752,12 +748,14 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
         }
     }
     if constexpr (RES) rice_first_records(rv, rt);
+    if constexpr (HEAD) head_norm_chunks<NC>(xc, gw, o.cols, a.ha, red);
 
     const uint32_t nch = S * (uint32_t)Kcfg<KIND>::STEP_COLS / 8u;
     float* sx = reinterpret_cast<float*>(lds + (size_t)S * Kcfg<KIND>::P * A_TILE_STRIDE);
     float* xs = reinterpret_cast<float*>(lds + M.xs);
     for (uint32_t i = threadIdx.x; i < S * (uint32_t)Kcfg<KIND>::P; i += nthr)
         *reinterpret_cast<uint4*>(lds + (size_t)i * A_TILE_STRIDE + 256u) = make_uint4(0u, 0u, 0u, 0u);
+    bool bad = false;  // (a plain GEMV's non-finite x gives zeroed units and no flag)
     auto image = [&](uint32_t ch, float4 (&v)[2]) {
         if constexpr (RES) {
             if (8u * ch < o.cols) {
@@ -765,19 +763,25 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
                 reinterpret_cast<float4*>(xs)[2u * ch + 1u] = v[1];
             }
         }
-        (void)image_chunk<KIND>(ch, v, lds, sx, 0u, 0u);
+        bad |= image_chunk<KIND>(ch, v, lds, sx, 0u, 0u);
     };
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
         const uint32_t ch = threadIdx.x + nthr * (uint32_t)j;
         if (ch < nch) image(ch, xc.v[j]);
     }
-    for (uint32_t ch = threadIdx.x + nthr * NC; ch < nch; ch += nthr) {
+    if constexpr (!HEAD) for (uint32_t ch = threadIdx.x + nthr * NC; ch < nch; ch += nthr) {
         float4 v[2];
         load_chunk(x, 8u * ch, o.cols, v);
         image(ch, v);
     }
     __syncthreads();
+    if constexpr (HEAD) {
+        if (bad) {
+            if (a.status) atomicOr(a.status, 1u);
+            atomicOr(reinterpret_cast<uint32_t*>(a.ha.key + 1), 1u);
+        }
+    }
 
     const ImageA A{lds, a_lane_offset(lane)};
     float* terms = reinterpret_cast<float*>(lds + M.terms);
@@ -819,9 +823,15 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     __syncthreads();
 
     float* ysh = reinterpret_cast<float*>(lds + M.ysh);
+    uint64_t best = 0;
     auto put = [&](uint32_t i, float v) {  // row i of the workgroup
-        if constexpr (RES) ysh[i] = v;
-        else if (r0 + i < o.rows) y[r0 + i] = v;
+        if constexpr (RES) {
+            ysh[i] = v;
+        } else if (r0 + i < o.rows) {
+            y[r0 + i] = v;
+            if constexpr (HEAD)
+                if (r0 + i < a.ha.n_valid) best = max(best, greedy_key(v, r0 + i));
+        }
     };
     if (split) {
         constexpr uint32_t NT = KIND == HK_MIXED ? 2u : 1u;
@@ -861,6 +871,7 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
             if (row < r1) y[row] = racc[h];
         }
     }
+    if constexpr (HEAD) fold_key(best, kred, a.ha.key);
 }
 
 // Launch shape (R tiles per wave group, D steps in flight, tiles per
@@ -898,11 +909,6 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
 #ifndef HK_Q_TPW
 #define HK_Q_TPW 32
 #endif
-#ifndef HK_HEAD_R
-#define HK_HEAD_R 2
-#define HK_HEAD_D 3
-#define HK_HEAD_TPW 5
-#endif
 #ifndef HK_MIX_R
 #define HK_MIX_R 1
 #define HK_MIX_D 3
@@ -935,13 +941,27 @@ static uint32_t pow2_ceil(uint32_t v) {
 //   * beyond, q8 (160 organs: 29.1 -> 26.0; 320: 60.2 -> 54.4) and mixed
 //     (8.9 -> 8.05) up to the streamed shapes; the others' walk is faster
 //     (binary 320 organs: 9.7 against 10.8; Q4 with 7168 columns 99 against 107).
+// HEAD: every workgroup ends in one atomic max on the same word, which the
+// memory side takes at about 12 ns each (a binary 151,936 x 2048 lm_head over
+// 1,900 workgroups: 30 us for 44 MB), so one or two balanced workgroups per
+// CU, 8 waves each: binary 16.8 us (one wave per tile, one workgroup per CU),
+// Q4 40.0 -> 30.4, q8 56.3 -> 55 (four slices, two workgroups per CU above
+// 4,096 tiles); q8 65,000 rows 29.8 -> 25.5, 11,409 rows 13.0 -> 10.8; tile
+// counts that leave a nearly empty last round cost up to 30 % (q8 151,936 over
+// 32 tiles: 69.7).
 // RES (256 threads, at most 4 tiles a workgroup: a row's records are one
 // thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8 ->
 // 6.7, 512 x 7168: 35.4 -> 8.9; above 4,096 tiles the two launches are faster
 // (160 organs: 11.0 against 11.8).
-static SplitShape split_shape(int kind, bool res, uint64_t tiles, uint32_t S, uint32_t cols) {
-    if (tiles >= 16384) return {0, 0, 0};
+static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uint32_t S, uint32_t cols) {
     const uint32_t s2 = pow2_ceil(S);
+    if (head) {
+        const uint32_t ks = kind == HK_BIN ? 1u : std::min(4u, s2), ts = 8u / ks;
+        const uint32_t wgs = kind == HK_BIN || tiles <= 4096 ? 256u : 512u;
+        const uint32_t even = (uint32_t)((tiles + wgs - 1u) / wgs);
+        return {8, ks, std::min((even + ts - 1u) / ts * ts, 64u)};
+    }
+    if (tiles >= 16384) return {0, 0, 0};
     uint32_t tpw = std::min(pow2_ceil((uint32_t)((tiles + 255) / 256)), 8u);
     if (res) {
         if (tiles > 4096) return {0, 0, 0};
@@ -961,14 +981,15 @@ static SplitShape split_shape(int kind, bool res, uint64_t tiles, uint32_t S, ui
     return {0, 0, 0};
 }
 
-template <int KIND, bool RES>
+template <int KIND, bool RES, bool HEAD = false>
 static hipError_t launch_split(const OrganView* organs, const ResView* res, const ResView* res_one, uint32_t n,
                                const OrganView& sh, const float* x, size_t xs, float* y, size_t ys, hipStream_t s,
-                               bool* done) {
+                               bool* done, const HeadArgs& ha = {}, uint32_t* status = nullptr) {
     constexpr bool ORD = KIND != HK_Q4 && KIND != HK_Q8;
     constexpr int D = KIND == HK_MIXED ? 2 : 4;
     *done = false;
-    SplitShape c = split_shape(KIND, RES, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
+    SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
+//SWEEP
     if (!c.waves) return hipSuccess;
     const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw;
     const size_t lds = SplitLds<KIND, ORD, RES>(sh.steps, sh.cols, tpw, ks).total;
@@ -988,7 +1009,9 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     a.n = n;
     a.parts = (sh.n_tiles + tpw - 1) / tpw;
     a.tpw = tpw;
-    hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES>), dim3(a.parts * n), dim3(64u * waves), lds, s, a);
+    a.ha = ha;
+    a.status = status;
+    hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES, HEAD>), dim3(a.parts * n), dim3(64u * waves), lds, s, a);
     return hipGetLastError();
 }
 
@@ -1017,13 +1040,10 @@ static hipError_t launch_r(const OrganView* organs, uint32_t n, const OrganView&
     return launch_kind<KIND, 1, 2>(organs, n, sh, x, xs, y, ys, tpw, s);
 }
 
-// The terminal head on a q8 lm_head (cols <= 8192): one GEMV launch with the
-// norm prologue and the greedy-key epilogue, then the one-thread pick (which
-// also clears the key for the next call).  Launch shapes as for one q8 organ,
-// except 4,096-16,383 tiles (a 65k-262k vocabulary), where 2-tile groups, 3
-// steps in flight, over 5 tiles per workgroup measured fastest (151,936 x
-// 2048: 1,900 workgroups, under the 2,048 resident at once; 56.5 us against
-// 57.6 for 6 tiles, 59.3 for 8, 64.0 for 4).
+// The terminal head on a packed lm_head of at most 8192 columns: one GEMV
+// launch with the norm prologue and the greedy-key epilogue, then the
+// one-thread pick (which also clears the key for the next call), against four
+// launches of its parts.
 __global__ void head_pick_fused_kernel(uint64_t* __restrict__ key, int32_t* __restrict__ token, uint32_t* status) {
     if (threadIdx.x == 0) {
         const uint64_t best = key[0];
@@ -1038,21 +1058,28 @@ __global__ void head_pick_fused_kernel(uint64_t* __restrict__ key, int32_t* __re
     }
 }
 
-bool head_gemv_fusable(const OrganView& sh) { return sh.kind == HK_Q8 && x_image_cols<HK_Q8>(sh.steps) <= 8192u; }
+bool head_gemv_fusable(const OrganView& sh) {
+    return (sh.kind == HK_Q8 || sh.kind == HK_Q4 || sh.kind == HK_BIN) &&
+           sh.steps * tile_step_cols(sh.kind) <= 8192u;
+}
 
-hipError_t launch_head_fused(const OrganView* organ_dev, const OrganView& sh, const float* h, const float* norm_w,
+template <int KIND>
+static hipError_t launch_head_gemv(const OrganView& sh, const float* h, float* logits, const HeadArgs& ha,
+                                   uint32_t* status, hipStream_t s) {
+    bool done = false;
+    const hipError_t e = launch_split<KIND, false, true>(nullptr, nullptr, nullptr, 1, sh, h, 0, logits, 0, s, &done, ha,
+                                                         status);
+    return e != hipSuccess || done ? e : hipErrorInvalidValue;  // (at most 55 KB of LDS: always done)
+}
+
+hipError_t launch_head_fused(const OrganView& sh, const float* h, const float* norm_w,
                              float eps, float* xn, float* logits, uint32_t n_valid, uint64_t* key, int32_t* token,
                              uint32_t* status, hipStream_t s) {
     if (!head_gemv_fusable(sh)) return hipErrorInvalidValue;
     const HeadArgs ha{norm_w, eps, xn, n_valid, key};
-    hipError_t e;
-    if (sh.n_tiles >= 16384u)
-        e = launch_kind<HK_Q8, 2, 3, true>(organ_dev, 1, sh, h, 0, logits, 0, 16, s, ha, status);
-    else if (sh.n_tiles >= 4096u)
-        e = launch_kind<HK_Q8, HK_HEAD_R, HK_HEAD_D, true>(organ_dev, 1, sh, h, 0, logits, 0, HK_HEAD_TPW, s, ha, status);
-    else
-        e = launch_kind<HK_Q8, 1, 2, true>(organ_dev, 1, sh, h, 0, logits, 0, (sh.n_tiles + 3) / 4 >= 256 ? 4 : 1, s,
-                                          ha, status);
+    const hipError_t e = sh.kind == HK_Q8   ? launch_head_gemv<HK_Q8>(sh, h, logits, ha, status, s)
+                         : sh.kind == HK_Q4 ? launch_head_gemv<HK_Q4>(sh, h, logits, ha, status, s)
+                                            : launch_head_gemv<HK_BIN>(sh, h, logits, ha, status, s);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(head_pick_fused_kernel, dim3(1), dim3(64), 0, s, key, token, status);
     return hipGetLastError();
@@ -1081,10 +1108,8 @@ hipError_t launch_gemv_rice(const OrganView* organs_dev, const ResView* res_dev,
     const ResArgs ra{res_dev, pieces};
     *fused = true;
     if (wide)
-        return launch_kind<HK_BIN, HK_RES_R, HK_RES_D, false, true>(organs_dev, n, sh, x, x_stride, y, y_stride, tpw, s, {},
-                                                                   nullptr, ra);
-    return launch_kind<HK_BIN, HK_BIN_NARROW_R, HK_BIN_NARROW_D, false, true>(organs_dev, n, sh, x, x_stride, y,
-                                                                              y_stride, tpw, s, {}, nullptr, ra);
+        return launch_kind<HK_BIN, HK_RES_R, HK_RES_D, true>(organs_dev, n, sh, x, x_stride, y, y_stride, tpw, s, ra);
+    return launch_kind<HK_BIN, HK_BIN_NARROW_R, HK_BIN_NARROW_D, true>(organs_dev, n, sh, x, x_stride, y, y_stride, tpw, s, ra);
 }
 
 hipError_t launch_gemv_tiled(const OrganView* organs_dev, uint32_t n, const OrganView& sh, const float* x,

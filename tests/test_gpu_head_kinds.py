@@ -1,0 +1,68 @@
+"""The fused terminal head over the lm_head kinds it takes (q8, Q4, binary)
+and one it must leave to the separate launches (a binary lm_head with a
+residual), at small and ragged vocabularies and its widest hidden size."""
+from __future__ import annotations
+
+import sys
+
+import numpy as np
+import pytest
+
+from tests import hk_testutil as U
+
+pytestmark = pytest.mark.gpu
+KIND = {"q4": U.HK_Q4, "bin": U.HK_BIN, "q8": 4, "rice": 6}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from hawking_amd.runtime import Context
+    return Context(0)
+
+
+def _organ(ctx, oracle, kind, rows, cols):
+    from hawking_amd.organs import SyntheticOrgan
+    return SyntheticOrgan(ctx, KIND[kind], rows, cols, oracle.stream_key(U.SEED, (0x4EAD << 32) + rows * 8 + cols),
+                          0, group={"q4": 32, "q8": 64}.get(kind, 128))
+
+
+@pytest.mark.parametrize("kind", sorted(KIND))
+@pytest.mark.parametrize("vocab,hidden,cut", [(1, 128, 0), (15, 640, 3), (257, 8192, 1), (4101, 1024, 100),
+                                              (70000, 512, 331)])
+def test_head_kinds(ctx, oracle, kind, vocab, hidden, cut):
+    from hawking_amd.head import TerminalHead
+    print("[gpu-case] head", kind, vocab, hidden, flush=True)
+    sys.stdout.flush()
+    lm = _organ(ctx, oracle, kind, vocab, hidden)
+    rng = np.random.default_rng(vocab + hidden)
+    h = rng.standard_normal(hidden).astype(np.float32)
+    nw = (rng.standard_normal(hidden) * 0.02).astype(np.float32)
+    head = TerminalHead(ctx, nw, lm, vocab - cut)
+    for _ in range(2):  # the second call finds the key cleared
+        tok = head.greedy(h)
+        logits, xn = head.logits.download(), head.xn.download()
+        assert tok == oracle.argmax_greedy(logits, vocab - cut)
+    # each xn to a few roundings, the logits to the engine's bound on it
+    assert np.all(np.abs(xn - oracle.rmsnorm_1p(h, nw, 1e-6)) <= 2e-6 * np.abs(xn) + 1e-30)
+    w, x64 = lm.decode(0, min(vocab, 300)).astype(np.float64), xn.astype(np.float64)
+    terms = hidden // 16 + 20 + (2 * int(0.1 * hidden) if kind == "rice" else 0)
+    bound = 2.0 ** -23 * np.abs(x64).max() * np.abs(w).sum(1) + terms * 2.0 ** -24 * (np.abs(w) @ np.abs(x64))
+    assert np.all(np.abs(logits[:300] - w @ x64) <= bound)
+    assert head.pick.download().tolist() == [0, 0]
+
+
+@pytest.mark.parametrize("kind", ["q4", "bin"])
+def test_head_kinds_flag_nonfinite(ctx, oracle, kind):
+    from hawking_amd._lib import HawkingError
+    from hawking_amd.head import TerminalHead
+    print("[gpu-case] head non-finite", kind, flush=True)
+    sys.stdout.flush()
+    head = TerminalHead(ctx, np.zeros(512, np.float32), _organ(ctx, oracle, kind, 300, 512))
+    h = np.ones(512, np.float32)
+    for value in (np.inf, np.nan):
+        bad = h.copy()
+        bad[511] = value
+        with pytest.raises(HawkingError):
+            head.greedy(bad)
+        assert int(head.token.download()[0]) == -1
+    assert head.greedy(h) == oracle.argmax_greedy(head.logits.download())
