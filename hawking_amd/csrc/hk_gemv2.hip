@@ -686,7 +686,8 @@ constexpr size_t SPLIT_LDS_LIMIT = 96 * 1024;
 // threads; records loaded before the image build).
 // HEAD: x is the hidden state; the prologue forms RMSNorm(1+w) of it and the
 // epilogue folds the rows' greedy keys (HeadArgs; cols <= 8192, 512 threads).
-template <int KIND, int D, bool ORD, bool RES, bool HEAD>
+// NT: the weight loads carry the non-temporal hint.
+template <int KIND, int D, bool ORD, bool RES, bool HEAD, bool NT = false>
 __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs a) {
     static_assert(!(RES && HEAD), "an lm_head has no fused residual");
     extern __shared__ __align__(16) uint8_t lds[];
@@ -743,7 +744,7 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     } else {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            fetch_one<KIND, 1, false>(o, fT, fs, lane, f[d], 0);
+            fetch_one<KIND, 1, NT>(o, fT, fs, lane, f[d], 0);
             step_on();
         }
     }
@@ -790,8 +791,8 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     uint32_t cT = tf, cs = s0;
     auto consume = [&](const Frag<KIND, 1>& fr) {
         if (split) {
-            constexpr uint32_t NT = KIND == HK_MIXED ? 2u : 1u;
-            float2* o2 = reinterpret_cast<float2*>(terms) + ((cT - t0) * S + cs) * 64u * NT + (uint32_t)lane * NT;
+            constexpr uint32_t TERMS = KIND == HK_MIXED ? 2u : 1u;
+            float2* o2 = reinterpret_cast<float2*>(terms) + ((cT - t0) * S + cs) * 64u * TERMS + (uint32_t)lane * TERMS;
             uint32_t k = 0;
             compute_terms<KIND, 1>(fr, cs, A, sx, q, [&](int, float s, float v) { o2[k++] = make_float2(s, v); });
         } else {
@@ -813,7 +814,7 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             consume(f[d]);
-            fetch_one<KIND, 1, false>(o, fT, fs, lane, f[d], 0);
+            fetch_one<KIND, 1, NT>(o, fT, fs, lane, f[d], 0);
             step_on();
         }
     }
@@ -834,15 +835,15 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
         }
     };
     if (split) {
-        constexpr uint32_t NT = KIND == HK_MIXED ? 2u : 1u;
+        constexpr uint32_t TERMS = KIND == HK_MIXED ? 2u : 1u;
         for (uint32_t T = wave; T < t1 - t0; T += nthr >> 6) {
-            const float2* t2 = reinterpret_cast<const float2*>(terms) + T * S * 64u * NT + (uint32_t)lane * NT;
+            const float2* t2 = reinterpret_cast<const float2*>(terms) + T * S * 64u * TERMS + (uint32_t)lane * TERMS;
             float v = 0.0f;
 #pragma unroll 4
             for (uint32_t s = 0; s < S; ++s)
 #pragma unroll
-                for (uint32_t h = 0; h < NT; ++h) {
-                    const float2 e = t2[s * 64u * NT + h];
+                for (uint32_t h = 0; h < TERMS; ++h) {
+                    const float2 e = t2[s * 64u * TERMS + h];
                     v = __builtin_fmaf(e.x, e.y, v);
                 }
             v = tile_row_sum(v);
@@ -914,6 +915,8 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
 #define HK_MIX_D 3
 #define HK_MIX_TPW 16
 #endif
+constexpr uint64_t MALL_BYTES = 256ull << 20;  // the Infinity Cache
+
 struct SplitShape {
     uint32_t waves, ks, tpw;  // waves 0: the launch is not split
 };
@@ -946,7 +949,11 @@ static uint32_t pow2_ceil(uint32_t v) {
 // 1,900 workgroups: 30 us for 44 MB), so one or two balanced workgroups per
 // CU, 8 waves each: binary 16.8 us (one wave per tile, one workgroup per CU),
 // Q4 40.0 -> 30.4, q8 56.3 -> 55 (four slices, two workgroups per CU above
-// 4,096 tiles); q8 65,000 rows 29.8 -> 25.5, 11,409 rows 13.0 -> 10.8; tile
+// 4,096 tiles); q8 65,000 rows 29.8 -> 25.5, 11,409 rows 13.0 -> 10.8; a q8
+// lm_head larger than the Infinity Cache loads non-temporally with one
+// workgroup per CU (151,936 x 2048: 53.4 -> 51.4, 128,256 x 4096: 96.2 -> 84;
+// below, the hint and the fewer loads in flight cost: 65,000 rows 25.9 -> 34.8;
+// Q4 of these sizes fits and gains nothing from it); tile
 // counts that leave a nearly empty last round cost up to 30 % (q8 151,936 over
 // 32 tiles: 69.7).
 // RES (256 threads, at most 4 tiles a workgroup: a row's records are one
@@ -957,7 +964,8 @@ static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uin
     const uint32_t s2 = pow2_ceil(S);
     if (head) {
         const uint32_t ks = kind == HK_BIN ? 1u : std::min(4u, s2), ts = 8u / ks;
-        const uint32_t wgs = kind == HK_BIN || tiles <= 4096 ? 256u : 512u;
+        const bool past_mall = kind == HK_Q8 && tiles * 16u * cols > MALL_BYTES;
+        const uint32_t wgs = kind == HK_BIN || tiles <= 4096 || past_mall ? 256u : 512u;
         const uint32_t even = (uint32_t)((tiles + wgs - 1u) / wgs);
         return {8, ks, std::min((even + ts - 1u) / ts * ts, 64u)};
     }
@@ -1011,7 +1019,11 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     a.tpw = tpw;
     a.ha = ha;
     a.status = status;
-    hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES, HEAD>), dim3(a.parts * n), dim3(64u * waves), lds, s, a);
+    if (HEAD && KIND == HK_Q8 && (uint64_t)sh.rows * sh.cols > MALL_BYTES)
+        hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES, HEAD, HEAD && KIND == HK_Q8>), dim3(a.parts * n),
+                           dim3(64u * waves), lds, s, a);
+    else
+        hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES, HEAD>), dim3(a.parts * n), dim3(64u * waves), lds, s, a);
     return hipGetLastError();
 }
 

@@ -26,9 +26,12 @@ def _organ(ctx, oracle, kind, rows, cols):
                           0, group={"q4": 32, "q8": 64}.get(kind, 128))
 
 
-@pytest.mark.parametrize("kind", sorted(KIND))
-@pytest.mark.parametrize("vocab,hidden,cut", [(1, 128, 0), (15, 640, 3), (257, 8192, 1), (4101, 1024, 100),
-                                              (70000, 512, 331)])
+CASES = [(k, v, h, c) for k in sorted(KIND)
+         for v, h, c in ((1, 128, 0), (15, 640, 3), (257, 8192, 1), (4101, 1024, 100), (70000, 512, 331))]
+CASES.append(("q8", 140001, 2048, 7))  # weights larger than the Infinity Cache
+
+
+@pytest.mark.parametrize("kind,vocab,hidden,cut", CASES)
 def test_head_kinds(ctx, oracle, kind, vocab, hidden, cut):
     from hawking_amd.head import TerminalHead
     print("[gpu-case] head", kind, vocab, hidden, flush=True)
