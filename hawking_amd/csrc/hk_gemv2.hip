@@ -67,6 +67,8 @@ __device__ __forceinline__ void flush_group(float* acc, const uint32_t* T, int n
     }
 }
 
+constexpr size_t SPLIT_LDS_LIMIT = 96 * 1024;  // of the small launches (one workgroup per CU)
+
 // Mixed step headers staged per workgroup: tiles x steps <= 32 x 24.
 constexpr uint32_t GEMV_MAX_MIXED_TILES_PER_WG = 32;
 constexpr int GEMV_HDR_PER_THREAD = 3;
@@ -568,6 +570,191 @@ lowrank_kernel(const OrganView* __restrict__ lefts, const OrganView* __restrict_
     if (bad && status) atomicOr(status, 1u);
 }
 
+// The same pairs when there are too few of them for one workgroup each to
+// fill the chip: P workgroups of 16 waves share a pair's left factor, each
+// forming the whole mid itself (the right factor is the smaller one, and its
+// re-reads are cache hits).  The right tiles go in rounds of at most 16: four
+// waves split a tile's steps and leave their terms in LDS, then one wave per
+// tile adds them in step order (the bits of a walk); the left tiles are one
+// wave each, their first steps in flight while mid's image is built.
+constexpr uint32_t LOWRANK_WAVES = 16, LOWRANK_ROUND = 16;
+struct LowrankArgs {
+    OrganView left, right;                // n = 1: the pair
+    const OrganView *lefts, *rights;      // else the tables
+    const float* x;
+    float *mid, *y;                       // mid may be null
+    size_t x_stride, mid_stride, y_stride;
+    uint32_t n, parts;                    // pairs, workgroups per pair
+    uint32_t tpw, round;                  // left tiles per workgroup, right tiles per round
+};
+struct LowrankSplitLds {
+    size_t terms, mid, img_l, total;
+    __host__ __device__ LowrankSplitLds(const OrganView& l, const OrganView& r, uint32_t round) {
+        terms = (x_lds_bytes<HK_U3>(r.steps) + 15u) & ~(size_t)15;
+        mid = terms + (size_t)round * r.steps * 512u;
+        img_l = mid + (size_t)r.n_tiles * 64u;
+        total = img_l + x_lds_bytes<HK_U3>(l.steps);
+    }
+};
+__global__ void __launch_bounds__(64 * LOWRANK_WAVES) lowrank_split_kernel(LowrankArgs a) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    constexpr int D = 4;
+    constexpr uint32_t P3 = Kcfg<HK_U3>::P, KS = 4, TS = LOWRANK_WAVES / KS;
+    uint32_t oi, part;
+    organ_part(blockIdx.x, a.parts, a.n, &oi, &part);
+    OrganView lv = a.left, rv = a.right;
+    if (a.lefts) {
+        lv = a.lefts[oi];
+        rv = a.rights[oi];
+    }
+    const float* __restrict__ x = a.x + (size_t)oi * a.x_stride;
+    float* __restrict__ y = a.y + (size_t)oi * a.y_stride;
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nthr = blockDim.x;
+    const LowrankSplitLds M(lv, rv, a.round);
+    float* mid = reinterpret_cast<float*>(lds + M.mid);
+    float2* terms = reinterpret_cast<float2*>(lds + M.terms) + lane;
+    const uint32_t S = rv.steps, ksl = wave & (KS - 1u), tsl = wave / KS;
+    const uint32_t per = (S + KS - 1u) / KS, s0 = min(ksl * per, S), ns = min(per, S - s0);
+
+    XChunks<1> xc;
+    load_x<1>(BlockTeam{}, x, rv.cols, xc);  // cols <= 8192: one chunk a thread
+    // this wave's items of the round of right tiles from b on
+    uint32_t fT = 0, fs = 0, fi = 0, fn = 0;
+    Frag<HK_U3, 1> f[D];
+    auto next = [&]() {
+        if (++fi < fn) {
+            ++fs;
+            if (fs == s0 + ns) {
+                fs = s0;
+                fT += TS;
+            }
+        }
+    };
+    auto start = [&](uint32_t b) {
+        const uint32_t e = min(b + a.round, rv.n_tiles), t = b + tsl;
+        fn = t < e ? (e - t + TS - 1u) / TS * ns : 0u;
+        fT = fn ? t : b;
+        fs = fn ? s0 : 0u;
+        fi = 0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            fetch_one<HK_U3, 1>(rv, fT, fs, lane, f[d], 0);
+            next();
+        }
+        return fn;
+    };
+    uint32_t n = start(0);
+    auto image = [&](uint8_t* img, const OrganView& o, float4 (&v)[2], uint32_t ch) {
+        float* sx = reinterpret_cast<float*>(img + (size_t)o.steps * P3 * A_TILE_STRIDE);
+        if (ch < o.steps * 16u) (void)image_chunk<HK_U3>(ch, v, img, sx, 0u, 0u);
+    };
+    auto zero = [&](uint8_t* img, uint32_t steps) {
+        for (uint32_t i = threadIdx.x; i < steps * P3; i += nthr)
+            *reinterpret_cast<uint4*>(img + (size_t)i * A_TILE_STRIDE + 256u) = make_uint4(0u, 0u, 0u, 0u);
+    };
+    zero(lds, S);
+    zero(lds + M.img_l, lv.steps);
+    image(lds, rv, xc.v[0], threadIdx.x);
+    __syncthreads();
+
+    const ImageA AR{lds, a_lane_offset(lane)};
+    const float* sxr = reinterpret_cast<const float*>(lds + (size_t)S * P3 * A_TILE_STRIDE);
+    for (uint32_t b = 0; b < rv.n_tiles; b += a.round) {
+        uint32_t cT = b + tsl, cs = s0;
+        auto consume = [&](const Frag<HK_U3, 1>& fr) {
+            float2* o = terms + ((cT - b) * S + cs) * 64u;
+            compute_terms<HK_U3, 1>(fr, cs, AR, sxr, q, [&](int, float s, float v) { *o = make_float2(s, v); });
+            ++cs;
+            if (cs == s0 + ns) {
+                cs = s0;
+                cT += TS;
+            }
+        };
+        uint32_t it = 0;
+        for (; it + D < n; it += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                consume(f[d]);
+                fetch_one<HK_U3, 1>(rv, fT, fs, lane, f[d], 0);
+                next();
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (it + (uint32_t)d < n) consume(f[d]);
+        if (b + a.round < rv.n_tiles) n = start(b + a.round);
+        __syncthreads();
+        if (b + wave < min(b + a.round, rv.n_tiles)) {
+            float v = 0.0f;
+#pragma unroll 4
+            for (uint32_t s = 0; s < S; ++s) {
+                const float2 e = terms[(wave * S + s) * 64u];
+                v = __builtin_fmaf(e.x, e.y, v);
+            }
+            v = tile_row_sum(v);
+            if (lane < 16) mid[(b + wave) * 16u + (uint32_t)lane] = v;
+        }
+        __syncthreads();
+    }
+
+    // the left tiles: wave w takes t0 + w, t0 + w + 16, ..., every step
+    const uint32_t t0 = part * a.tpw, t1 = min(t0 + a.tpw, lv.n_tiles), S2 = lv.steps;
+    n = t0 + wave < t1 ? (t1 - t0 - wave + LOWRANK_WAVES - 1u) / LOWRANK_WAVES * S2 : 0u;
+    fT = n ? t0 + wave : 0u;
+    fs = 0;
+    fi = 0;
+    auto next_l = [&]() {
+        if (++fi < n) {
+            ++fs;
+            if (fs == S2) {
+                fs = 0;
+                fT += LOWRANK_WAVES;
+            }
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        fetch_one<HK_U3, 1>(lv, fT, fs, lane, f[d], 0);
+        next_l();
+    }
+    if (a.mid && part == 0)
+        for (uint32_t i = threadIdx.x; i < rv.rows; i += nthr) a.mid[(size_t)oi * a.mid_stride + i] = mid[i];
+    {
+        float4 v[2];
+        load_chunk(mid, 8u * threadIdx.x, rv.rows, v);
+        image(lds + M.img_l, lv, v, threadIdx.x);
+    }
+    __syncthreads();
+    const ImageA AL{lds + M.img_l, a_lane_offset(lane)};
+    const float* sxl = reinterpret_cast<const float*>(lds + M.img_l + (size_t)S2 * P3 * A_TILE_STRIDE);
+    uint32_t cT = t0 + wave, cs = 0;
+    float acc = 0.0f;
+    auto consume = [&](const Frag<HK_U3, 1>& fr) {
+        compute_step<HK_U3, 1>(fr, cs, AL, sxl, q, &acc);
+        if (++cs == S2) {
+            const float v = tile_row_sum(acc);
+            const uint32_t row = cT * 16u + (uint32_t)lane;
+            if (lane < 16 && row < lv.rows) y[row] = v;
+            acc = 0.0f;
+            cs = 0;
+            cT += LOWRANK_WAVES;
+        }
+    };
+    uint32_t it = 0;
+    for (; it + D < n; it += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            consume(f[d]);
+            fetch_one<HK_U3, 1>(lv, fT, fs, lane, f[d], 0);
+            next_l();
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (it + (uint32_t)d < n) consume(f[d]);
+}
+
 bool lowrank_fusable(const OrganView& l, const OrganView& r) {
     return l.kind == HK_U3 && r.kind == HK_U3 && r.rows == l.cols && r.cols <= 8192u && r.rows <= 2048u &&
            lowrank_lds(l, r).total <= GEMV_LDS_LIMIT;
@@ -577,6 +764,37 @@ hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint3
                           const OrganView& r, const float* x, size_t x_stride, float* mid, size_t mid_stride, float* y,
                           size_t y_stride, uint32_t* status, hipStream_t s) {
     if (!lowrank_fusable(l, r)) return hipErrorInvalidValue;
+    // One workgroup per CU over all pairs, at least 16 left tiles each (us in a
+    // graph of one launch, against one 4-wave workgroup per pair): r160 2048 x
+    // 768, 1 pair 17.9 -> 6.4, 64 pairs 18.3 -> 7.3, 256 pairs 18.8 -> 12.8, 512
+    // pairs 23.3 -> 20.1, 1,024 pairs 34.7 against 37.7; r64 512 x 512, 1 pair
+    // 6.2 -> 4.8, 256 pairs 6.6 -> 5.6, 512 pairs 7.5 against 7.8; r384 4096 x
+    // 2048, 1 pair 53 -> 15.
+    const uint32_t few = l.n_tiles >= 64u ? 512u : 256u;
+    const uint32_t parts = n > few ? 0u
+                                   : std::min(std::max(256u / n, 1u), (l.n_tiles + LOWRANK_WAVES - 1u) / LOWRANK_WAVES);
+    if (parts) {
+        LowrankArgs a{};
+        a.tpw = (l.n_tiles + parts - 1u) / parts;
+        a.parts = (l.n_tiles + a.tpw - 1u) / a.tpw;
+        a.round = std::min(std::min(LOWRANK_ROUND, r.n_tiles), 128u / r.steps);
+        const size_t sl = LowrankSplitLds(l, r, a.round).total;
+        if (a.round && sl <= SPLIT_LDS_LIMIT) {
+            a.left = l;
+            a.right = r;
+            a.lefts = n > 1 ? lefts : nullptr;
+            a.rights = rights;
+            a.x = x;
+            a.mid = mid;
+            a.y = y;
+            a.x_stride = x_stride;
+            a.mid_stride = mid_stride;
+            a.y_stride = y_stride;
+            a.n = n;
+            hipLaunchKernelGGL(lowrank_split_kernel, dim3(a.parts * n), dim3(64u * LOWRANK_WAVES), sl, s, a);
+            return hipGetLastError();
+        }
+    }
     const size_t lds = lowrank_lds(l, r).total;
     if (x_image_cols<HK_U3>(r.steps) <= 2048u)
         hipLaunchKernelGGL(lowrank_kernel<1>, dim3(n), dim3(256), lds, s, lefts, rights, n, x, x_stride, mid,
@@ -674,8 +892,6 @@ struct SplitLds {
         total = ysh + (RES ? (size_t)tpw * 64u : 0);
     }
 };
-
-constexpr size_t SPLIT_LDS_LIMIT = 96 * 1024;
 
 // ORD: a row's terms are added in step order whatever KS is: the waves leave
 // each lane's {scale, v} in LDS and one wave per tile runs the same chain of
@@ -1040,7 +1256,10 @@ static hipError_t launch_r(const OrganView* organs, uint32_t n, const OrganView&
                 return launch_kind<KIND, HK_BIN_WIDE_R, HK_BIN_WIDE_D>(organs, n, sh, x, xs, y, ys, HK_BIN_WIDE_TPW, s);
             return launch_kind<KIND, HK_BIN_NARROW_R, HK_BIN_NARROW_D>(organs, n, sh, x, xs, y, ys, HK_BIN_NARROW_TPW, s);
         } else if constexpr (KIND == HK_U3) {
-            return launch_kind<KIND, 2, 3>(organs, n, sh, x, xs, y, ys, gemv_max_tiles(KIND, sh.steps) == 128u ? 128 : 16, s);
+            // narrow factors: up to 128 tiles share an image, as long as 1,024
+            // workgroups remain
+            const uint32_t share = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tiles / 1024u, 16u), 128u) & ~7u;
+            return launch_kind<KIND, 2, 3>(organs, n, sh, x, xs, y, ys, gemv_max_tiles(KIND, sh.steps) == 128u ? share : 16, s);
         } else if constexpr (KIND == HK_Q4 || KIND == HK_Q8) {
             return launch_kind<KIND, HK_Q_R, HK_Q_D>(organs, n, sh, x, xs, y, ys, HK_Q_TPW, s);
         } else {
