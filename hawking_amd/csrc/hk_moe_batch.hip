@@ -20,6 +20,8 @@
 //   6. act image: the x image of every (token, expert) activation row
 //   7. down:     per (active expert, 8 row tiles): w * (down . act) per member
 //   8. combine:  y_t = sum over t's experts in ascending id, then + shared
+#include <type_traits>
+
 #include "hk_internal.h"
 #include "hk_mfma.h"
 #include "hk_moe.h"
@@ -527,21 +529,22 @@ __device__ __forceinline__ void stage_images(uint8_t* lds, const uint8_t* src, u
 // member groups find them in that XCD's L2.  Slots past the last tile group
 // (tile groups rounded up to a multiple of 8) are empty items.
 constexpr uint32_t MOE_BATCH_XCDS = 8;
-__host__ __device__ inline uint32_t moe_batch_items(uint32_t gpe, uint32_t ngs, uint32_t n_routed) {
-    return (gpe + MOE_BATCH_XCDS - 1u) / MOE_BATCH_XCDS * MOE_BATCH_XCDS * ngs + n_routed * gpe;
+__host__ __device__ inline uint32_t moe_batch_items(uint32_t gps, uint32_t ngs, uint32_t gpe, uint32_t n_routed) {
+    return (gps + MOE_BATCH_XCDS - 1u) / MOE_BATCH_XCDS * MOE_BATCH_XCDS * ngs + n_routed * gpe;
 }
 struct ItemMap {
-    uint32_t gpe, ngs, nsh, n_items;
-    __device__ ItemMap(const MoeBatchDims& d, uint32_t gpe_, uint32_t n_active, uint32_t TB) : gpe(gpe_) {
+    uint32_t gps, gpe, ngs, nsh;  // tile groups (shared, routed), the shared expert's member groups, its items
+    __device__ ItemMap(const MoeBatchDims& d, uint32_t gps_, uint32_t gpe_, uint32_t TB) : gps(gps_), gpe(gpe_) {
         ngs = d.SI ? (d.T + TB - 1) / TB : 0u;
-        nsh = moe_batch_items(gpe, ngs, 0u);
-        n_items = moe_batch_items(gpe, ngs, n_active - (ngs ? 1u : 0u));
+        nsh = moe_batch_items(gps, ngs, 0u, 0u);
     }
+    // The item's active entry (the caller checks it against n_active: entries
+    // past it are stale), tile group and member groups.
     __device__ void at(uint32_t item, uint32_t* a, uint32_t* tg, uint32_t* m_lo, uint32_t* m_hi) const {
         if (item < nsh) {
             const uint32_t x = item % MOE_BATCH_XCDS, s = item / MOE_BATCH_XCDS;
             *a = 0;
-            *tg = x + MOE_BATCH_XCDS * (s / ngs);  // >= gpe: an empty slot
+            *tg = x + MOE_BATCH_XCDS * (s / ngs);  // >= gps: an empty slot
             *m_lo = s % ngs;
             *m_hi = *m_lo + 1u;
             return;
@@ -554,69 +557,88 @@ struct ItemMap {
     }
 };
 
+// One work item as the workgroup runs it.  Every load is independent of the
+// others: the entry and the active count together, and the entry's organ from
+// the views of expert 0 and the shared expert (routed experts sit at a uniform
+// stride), so an item's weights start one memory round trip after its index
+// instead of three.
+struct BatchItem {
+    uint4 ent;  // {expert, first member, members}
+    uint32_t tg, m0, m_end;
+    bool on;
+};
+__device__ __forceinline__ BatchItem batch_item(const MoeBatchDims& d, const MoeBatchWs& ws, const ItemMap& im,
+                                                uint32_t item, uint32_t TB) {
+    BatchItem w;
+    uint32_t a, lo, hi;
+    im.at(item, &a, &w.tg, &lo, &hi);
+    w.ent = ws.active[min(a, d.E)];
+    w.on = a < __builtin_amdgcn_readfirstlane(*ws.n_active);
+    w.m0 = lo * TB;
+    w.m_end = hi == 0xFFFFFFFFu ? w.ent.z : min(w.ent.z, hi * TB);
+    return w;
+}
+
 // ------------------------------------------------------------------ 5. gate/up (grouped)
 
 // An item covers TPI row tiles; a workgroup of TPI / TPW waves, each wave
 // runs TPW row tiles (gate and up of each) for the item's member tokens.
-template <int TB, int D, int TPW, int TPI>
-__global__ void __launch_bounds__(64 * TPI / TPW)
-moe_batch_gate_up_kernel(MoeBatchDims d, const OrganView* __restrict__ table, MoeBatchWs ws) {
+// WPE: waves per SIMD the registers must allow.
+template <int TB, int D, int TPW, int TPI, int PT, int WPE>
+__global__ void __launch_bounds__(64 * TPI / TPW, WPE)
+moe_batch_gate_up_kernel(MoeBatchDims d, MoeLayerDev L, MoeBatchWs ws) {
     extern __shared__ __align__(16) uint8_t lds[];  // TB x images of H columns
     const int lane = threadIdx.x & 63, q = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t aoff = a_lane_offset(lane);
-    const uint32_t tiles = n_tiles_for(max(d.I, d.SI)), gpe = (tiles + TPI - 1) / TPI;
+    const ItemMap im(d, (n_tiles_for(d.SI) + TPI - 1) / TPI, (n_tiles_for(d.I) + TPI - 1) / TPI, TB);
     const uint32_t S = n_steps_for(HK_Q4, d.H);
     const uint32_t img_bytes = (uint32_t)x_lds_bytes<HK_Q4>(S);
-    const ItemMap im(d, gpe, __builtin_amdgcn_readfirstlane(*ws.n_active), TB);
-    for (uint32_t item = blockIdx.x; item < im.n_items; item += gridDim.x) {
-        uint32_t a, tg, mg_lo, mg_hi;
-        im.at(item, &a, &tg, &mg_lo, &mg_hi);
-        const uint4 ent = ws.active[a];
-        const OrganView g = table[ent.x * 3u + 0u], u = table[ent.x * 3u + 1u];
-        if (tg * TPI >= g.n_tiles) continue;
-        // this wave's tiles (past the end they alias the first)
-        const uint32_t Tb = tg * TPI + TPW * wave;
-        bool vw[TPW];
-        const uint8_t* bd[2 * TPW];
-        const uint16_t* bs[2 * TPW];
+    const bool shared = blockIdx.x < im.nsh;
+    const OrganView g0 = L.table[shared ? d.E * 3u : 0u], u0 = L.table[shared ? d.E * 3u + 1u : 1u];
+    const BatchItem it = batch_item(d, ws, im, blockIdx.x, TB);
+    const OrganView g = advance_view(g0, shared ? 0u : it.ent.x, L.stride), u = advance_view(u0, shared ? 0u : it.ent.x, L.stride);
+    if (!it.on || it.tg * TPI >= g.n_tiles) return;
+    // this wave's tiles (past the end they alias the first)
+    const uint32_t Tb = it.tg * TPI + TPW * wave;
+    bool vw[TPW];
+    const uint8_t* bd[2 * TPW];
+    const uint16_t* bs[2 * TPW];
 #pragma unroll
-        for (int h = 0; h < TPW; ++h) {
-            vw[h] = Tb + h < g.n_tiles;
-            const size_t Tc = vw[h] ? Tb + h : Tb;
-            bd[2 * h] = g.data + Tc * S * 1024u + 16u * lane;
-            bd[2 * h + 1] = u.data + Tc * S * 1024u + 16u * lane;
-            bs[2 * h] = g.scales + Tc * S * 64u + lane;
-            bs[2 * h + 1] = u.scales + Tc * S * 64u + lane;
+    for (int h = 0; h < TPW; ++h) {
+        vw[h] = Tb + h < g.n_tiles;
+        const size_t Tc = vw[h] ? Tb + h : Tb;
+        bd[2 * h] = g.data + Tc * S * 1024u + 16u * lane;
+        bd[2 * h + 1] = u.data + Tc * S * 1024u + 16u * lane;
+        bs[2 * h] = g.scales + Tc * S * 64u + lane;
+        bs[2 * h + 1] = u.scales + Tc * S * 64u + lane;
+    }
+    for (uint32_t m0 = it.m0; m0 < it.m_end; m0 += TB) {
+        const uint32_t nm = min((uint32_t)TB, it.ent.z - m0);
+        uint32_t pair[TB], tok[TB];
+#pragma unroll
+        for (int j = 0; j < TB; ++j) {
+            pair[j] = ws.members[it.ent.y + m0 + min((uint32_t)j, nm - 1u)];
+            tok[j] = pair_token(d, pair[j]);
         }
-        const uint32_t m_end = mg_hi == 0xFFFFFFFFu ? ent.z : min(ent.z, mg_hi * (uint32_t)TB);
-        for (uint32_t m0 = mg_lo * TB; m0 < m_end; m0 += TB) {
-            const uint32_t nm = min((uint32_t)TB, ent.z - m0);
-            uint32_t pair[TB], tok[TB];
+        Frag<HK_Q4, 2 * TPW> f[D];
+        if (vw[0]) tiles_fetch_first<2 * TPW, D>(bd, bs, S, f);
+        __syncthreads();
+        stage_images<TB, PT>(lds, ws.ximg, ws.ximg_stride, tok, nm, img_bytes);
+        __syncthreads();
+        if (!vw[0]) continue;
+        float acc[TB][2 * TPW] = {};
+        tiles_x_tokens<2 * TPW, TB, D>(bd, bs, S, lds, img_bytes, nm, aoff, q, acc, f);
 #pragma unroll
-            for (int j = 0; j < TB; ++j) {
-                pair[j] = ws.members[ent.y + m0 + min((uint32_t)j, nm - 1u)];
-                tok[j] = pair_token(d, pair[j]);
-            }
-            Frag<HK_Q4, 2 * TPW> f[D];
-            if (vw[0]) tiles_fetch_first<2 * TPW, D>(bd, bs, S, f);
-            __syncthreads();
-            stage_images<TB, 4>(lds, ws.ximg, ws.ximg_stride, tok, nm, img_bytes);
-            __syncthreads();
-            if (!vw[0]) continue;
-            float acc[TB][2 * TPW] = {};
-            tiles_x_tokens<2 * TPW, TB, D>(bd, bs, S, lds, img_bytes, nm, aoff, q, acc, f);
+        for (int j = 0; j < TB; ++j) {
+            if ((uint32_t)j >= nm) break;
+            const int E = ws.ximg_e[tok[j]];
 #pragma unroll
-            for (int j = 0; j < TB; ++j) {
-                if ((uint32_t)j >= nm) break;
-                const int E = ws.ximg_e[tok[j]];
-#pragma unroll
-                for (int h = 0; h < TPW; ++h) {
-                    const float gs = ldexpf(tile_row_sum(acc[j][2 * h]), -E), us = ldexpf(tile_row_sum(acc[j][2 * h + 1]), -E);
-                    const uint32_t row = (Tb + h) * 16u + (uint32_t)(lane & 15);
-                    if (lane < 16 && vw[h] && row < g.rows)
-                        ws.act[(size_t)pair[j] * d.Imax + row] = (gs / (1.0f + expf(-gs))) * us;
-                }
+            for (int h = 0; h < TPW; ++h) {
+                const float gs = ldexpf(tile_row_sum(acc[j][2 * h]), -E), us = ldexpf(tile_row_sum(acc[j][2 * h + 1]), -E);
+                const uint32_t row = (Tb + h) * 16u + (uint32_t)(lane & 15);
+                if (lane < 16 && vw[h] && row < g.rows)
+                    ws.act[(size_t)pair[j] * d.Imax + row] = (gs / (1.0f + expf(-gs))) * us;
             }
         }
     }
@@ -643,61 +665,85 @@ __global__ void __launch_bounds__(256) moe_batch_act_image_kernel(MoeBatchDims d
 
 // ------------------------------------------------------------------ 7. down (grouped)
 
-template <int TB, int D, int TPW, int TPI>
+// OWN: the workgroup builds its members' activation images itself (E = 0: the
+// image launch's bits, its exponent aside), for batches of few items, where
+// the image launch costs more than the repeated builds.
+template <int TB, int D, int TPW, int TPI, bool OWN>
 __global__ void __launch_bounds__(64 * TPI / TPW)
-moe_batch_down_kernel(MoeBatchDims d, const OrganView* __restrict__ table, MoeBatchWs ws) {
+moe_batch_down_kernel(MoeBatchDims d, MoeLayerDev L, MoeBatchWs ws) {
     extern __shared__ __align__(16) uint8_t lds[];  // TB activation images
     const int lane = threadIdx.x & 63, q = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t aoff = a_lane_offset(lane);
-    const uint32_t tiles = n_tiles_for(d.H), gpe = (tiles + TPI - 1) / TPI;
-    const ItemMap im(d, gpe, __builtin_amdgcn_readfirstlane(*ws.n_active), TB);
-    const uint32_t np = d.T * d.K;
-    for (uint32_t item = blockIdx.x; item < im.n_items; item += gridDim.x) {
-        uint32_t a, tg, mg_lo, mg_hi;
-        im.at(item, &a, &tg, &mg_lo, &mg_hi);
-        const uint4 ent = ws.active[a];
-        const OrganView o = table[ent.x * 3u + 2u];
-        const uint32_t S = o.steps, img_bytes = (uint32_t)x_lds_bytes<HK_Q4>(S);
-        const uint32_t Tb = tg * TPI + TPW * wave;
-        bool vw[TPW];
-        const uint8_t* bd[TPW];
-        const uint16_t* bs[TPW];
+    const uint32_t tiles = n_tiles_for(d.H), gpe = (tiles + TPI - 1) / TPI, np = d.T * d.K;
+    const ItemMap im(d, gpe, gpe, TB);
+    const bool shared = blockIdx.x < im.nsh;
+    const OrganView o0 = L.table[shared ? d.E * 3u + 2u : 2u];
+    const BatchItem it = batch_item(d, ws, im, blockIdx.x, TB);
+    const OrganView o = advance_view(o0, shared ? 0u : it.ent.x, L.stride);
+    if (!it.on || it.tg * TPI >= o.n_tiles) return;
+    const uint32_t S = o.steps, img_bytes = (uint32_t)x_lds_bytes<HK_Q4>(S);
+    const uint32_t Tb = it.tg * TPI + TPW * wave;
+    bool vw[TPW];
+    const uint8_t* bd[TPW];
+    const uint16_t* bs[TPW];
 #pragma unroll
-        for (int h = 0; h < TPW; ++h) {
-            vw[h] = Tb + h < o.n_tiles;
-            const size_t Tc = vw[h] ? Tb + h : Tb;
-            bd[h] = o.data + Tc * S * 1024u + 16u * lane;
-            bs[h] = o.scales + Tc * S * 64u + lane;
-        }
-        const uint32_t m_end = mg_hi == 0xFFFFFFFFu ? ent.z : min(ent.z, mg_hi * (uint32_t)TB);
-        for (uint32_t m0 = mg_lo * TB; m0 < m_end; m0 += TB) {
-            const uint32_t nm = min((uint32_t)TB, ent.z - m0);
-            uint32_t pair[TB];
+    for (int h = 0; h < TPW; ++h) {
+        vw[h] = Tb + h < o.n_tiles;
+        const size_t Tc = vw[h] ? Tb + h : Tb;
+        bd[h] = o.data + Tc * S * 1024u + 16u * lane;
+        bs[h] = o.scales + Tc * S * 64u + lane;
+    }
+    for (uint32_t m0 = it.m0; m0 < it.m_end; m0 += TB) {
+        const uint32_t nm = min((uint32_t)TB, it.ent.z - m0);
+        uint32_t pair[TB];
 #pragma unroll
-            for (int j = 0; j < TB; ++j) pair[j] = ws.members[ent.y + m0 + min((uint32_t)j, nm - 1u)];
-            Frag<HK_Q4, TPW> f[D];
+        for (int j = 0; j < TB; ++j) pair[j] = ws.members[it.ent.y + m0 + min((uint32_t)j, nm - 1u)];
+        Frag<HK_Q4, TPW> f[D];
+        if constexpr (OWN) {
+            const uint32_t nch = S * tile_step_cols(HK_Q4) / 8u;
+            float4 v[TB][2];  // the first chunk of each, before the weights
+#pragma unroll
+            for (int j = 0; j < TB; ++j) load_chunk(ws.act + (size_t)pair[j] * d.Imax, 8u * threadIdx.x, o.cols, v[j]);
             if (vw[0]) tiles_fetch_first<TPW, D>(bd, bs, S, f);
             __syncthreads();
-            stage_images<TB, 2>(lds, ws.aimg, ws.aimg_stride, pair, nm, img_bytes);
-            __syncthreads();
-            if (!vw[0]) continue;
-            float acc[TB][TPW] = {};
-            tiles_x_tokens<TPW, TB, D>(bd, bs, S, lds, img_bytes, nm, aoff, q, acc, f);
+            bool bad = false;
 #pragma unroll
             for (int j = 0; j < TB; ++j) {
                 if ((uint32_t)j >= nm) break;
-                const int E = ws.aimg_e[pair[j]];
-                const bool routed = pair[j] < np;
-                const float w = routed ? ws.w[pair[j]] : 1.0f;
-                // a routed pair's output goes to its token's row of its rank in expert order
-                const uint32_t dst = routed ? pair[j] - pair[j] % d.K + (uint32_t)ws.rank[pair[j]] : pair[j];
-#pragma unroll
-                for (int h = 0; h < TPW; ++h) {
-                    const float y = ldexpf(tile_row_sum(acc[j][h]), -E);
-                    const uint32_t row = (Tb + h) * 16u + (uint32_t)(lane & 15);
-                    if (lane < 16 && vw[h] && row < d.H) ws.ybuf[(size_t)dst * d.H + row] = y * w;
+                uint8_t* img = lds + (size_t)j * img_bytes;
+                float* sx = reinterpret_cast<float*>(img + (size_t)S * Kcfg<HK_Q4>::P * A_TILE_STRIDE);
+                if (threadIdx.x < 64u) image_zero_blocks<HK_Q4>(threadIdx.x, img, S);
+                if (threadIdx.x < nch) bad |= image_chunk<HK_Q4>(threadIdx.x, v[j], img, sx, 0u, 0u);
+                for (uint32_t ch = threadIdx.x + blockDim.x; ch < nch; ch += blockDim.x) {
+                    float4 c[2];
+                    load_chunk(ws.act + (size_t)pair[j] * d.Imax, 8u * ch, o.cols, c);
+                    bad |= image_chunk<HK_Q4>(ch, c, img, sx, 0u, 0u);
                 }
+            }
+            if (bad) atomicOr(ws.status, HK_DEVERR_NONFINITE);
+        } else {
+            if (vw[0]) tiles_fetch_first<TPW, D>(bd, bs, S, f);
+            __syncthreads();
+            stage_images<TB, 2>(lds, ws.aimg, ws.aimg_stride, pair, nm, img_bytes);
+        }
+        __syncthreads();
+        if (!vw[0]) continue;
+        float acc[TB][TPW] = {};
+        tiles_x_tokens<TPW, TB, D>(bd, bs, S, lds, img_bytes, nm, aoff, q, acc, f);
+#pragma unroll
+        for (int j = 0; j < TB; ++j) {
+            if ((uint32_t)j >= nm) break;
+            const int E = OWN ? 0 : ws.aimg_e[pair[j]];
+            const bool routed = pair[j] < np;
+            const float w = routed ? ws.w[pair[j]] : 1.0f;
+            // a routed pair's output goes to its token's row of its rank in expert order
+            const uint32_t dst = routed ? pair[j] - pair[j] % d.K + (uint32_t)ws.rank[pair[j]] : pair[j];
+#pragma unroll
+            for (int h = 0; h < TPW; ++h) {
+                const float y = ldexpf(tile_row_sum(acc[j][h]), -E);
+                const uint32_t row = (Tb + h) * 16u + (uint32_t)(lane & 15);
+                if (lane < 16 && vw[h] && row < d.H) ws.ybuf[(size_t)dst * d.H + row] = y * w;
             }
         }
     }
@@ -740,6 +786,20 @@ static uint32_t tokens_per_group(uint32_t img_bytes, uint32_t cap, uint32_t budg
     return min(cap, budget / img_bytes);
 }
 
+// Calls f with the member tokens per group as a constant.
+template <class F>
+static void by_tokens(uint32_t tb, F f) {
+    if (tb >= 4) f(std::integral_constant<int, 4>{});
+    else if (tb >= 2) f(std::integral_constant<int, 2>{});
+    else f(std::integral_constant<int, 1>{});
+}
+
+// Down items up to which the down kernel builds its activation images itself:
+// hidden 4096 x 1024, 2 tokens (416 items) 49.2 -> 47.2 us a step, 7168 x 2048,
+// 1 token (504) 69.7 -> 66.7, 2176 x 256, 1 token (51) 33.9 -> 31.1; 4096 x 1024,
+// 8 tokens (1,600) 88.2 against 90.6.
+constexpr uint32_t OWN_IMAGE_ITEMS = 512;
+
 hipError_t launch_moe_batch(const MoeBatchDims& d, const MoeLayerDev& L, const float* bias, const uint16_t* x_bf16,
                             float* y, const MoeBatchWs& ws, int32_t* ids_out, float* w_out, hipStream_t s) {
     const uint32_t pairs = d.T * d.K + (d.SI ? d.T : 0u);
@@ -757,7 +817,7 @@ hipError_t launch_moe_batch(const MoeBatchDims& d, const MoeLayerDev& L, const f
 #define HK_BATCH_GU_TBMAX 4
 #endif
     constexpr int GU_TPI = HK_BATCH_GU_TPI, GU_TPW = 1, GU_D = HK_BATCH_GU_D, DN_TPI = 8, DN_TPW = 2, DN_D = HK_BATCH_DN_D;
-    const uint32_t gpe_gu = (n_tiles_for(max(d.I, d.SI)) + GU_TPI - 1) / GU_TPI;
+    const uint32_t gpe_gu = (n_tiles_for(d.I) + GU_TPI - 1) / GU_TPI, gps_gu = (n_tiles_for(d.SI) + GU_TPI - 1) / GU_TPI;
     const uint32_t gpe_dn = (n_tiles_for(d.H) + DN_TPI - 1) / DN_TPI;
     const uint32_t ximg = (uint32_t)moe_batch_img_bytes(d.H), aimg = (uint32_t)moe_batch_img_bytes(d.Imax);
     const uint32_t budget = image_lds_budget();
@@ -769,8 +829,8 @@ hipError_t launch_moe_batch(const MoeBatchDims& d, const MoeLayerDev& L, const f
     const uint32_t tbg = tb_gu >= 4 ? 4u : tb_gu >= 2 ? 2u : 1u;
     const uint32_t tbd = tb_dn >= 4 ? 4u : tb_dn >= 2 ? 2u : 1u;
     const uint32_t n_routed = min(d.E, d.T * d.K);
-    const uint32_t gu_items = moe_batch_items(gpe_gu, d.SI ? (d.T + tbg - 1) / tbg : 0u, n_routed);
-    const uint32_t dn_items = moe_batch_items(gpe_dn, d.SI ? (d.T + tbd - 1) / tbd : 0u, n_routed);
+    const uint32_t gu_items = moe_batch_items(gps_gu, d.SI ? (d.T + tbg - 1) / tbg : 0u, gpe_gu, n_routed);
+    const uint32_t dn_items = moe_batch_items(gpe_dn, d.SI ? (d.T + tbd - 1) / tbd : 0u, gpe_dn, n_routed);
     const uint32_t n_prep = (d.E + 15u) / 16u * d.S + d.T * ((d.H + XPART_COLS - 1) / XPART_COLS);
     hipLaunchKernelGGL(moe_batch_prep_kernel, dim3(n_prep), dim3(64 * RT_WAVES), (size_t)q4_stage_floats(d.H) * sizeof(float),
                        s, d, x_bf16, L.router_w, ws);
@@ -779,26 +839,36 @@ hipError_t launch_moe_batch(const MoeBatchDims& d, const MoeLayerDev& L, const f
     // one workgroup per item (the item count is an upper bound; the device
     // count decides): the dispatcher then balances ~1 MB items across the CUs
     // better than a persistent grid (measured: 862 vs 910 us per step)
-    const dim3 ggu(gu_items), gdn(dn_items);
-    // one tile per wave, 8 waves sharing the staged images
-    const dim3 bgu(64 * GU_TPI / GU_TPW), bdn(64 * DN_TPI / DN_TPW);
-    if (tb_gu >= 4)
-        hipLaunchKernelGGL((moe_batch_gate_up_kernel<4, GU_D, GU_TPW, GU_TPI>), ggu, bgu, (size_t)4 * ximg, s, d, L.table, ws);
-    else if (tb_gu >= 2)
-        hipLaunchKernelGGL((moe_batch_gate_up_kernel<2, GU_D, GU_TPW, GU_TPI>), ggu, bgu, (size_t)2 * ximg, s, d, L.table, ws);
+    const size_t lgu = (size_t)tbg * ximg, ldn = (size_t)tbd * aimg;
+    // where four tokens' images leave room for a second workgroup on the CU
+    // (hidden <= 4,480), 128 registers and 2 steps in flight allow it: one's
+    // weights stream while the other stages images or writes results (us per
+    // step, 60 tokens: hidden 4096, 128 experts top 6, 261 -> 238; hidden 1024, 32
+    // experts top 8, 210 -> 173; 33 tokens, hidden 768, 136 experts top 2, 70.6 ->
+    // 56.6).  With at most one item per CU there is no second workgroup and 6
+    // steps in flight are better (4 tokens, hidden 4480: 64.9 against 65.7).
+    if (2 * lgu <= 160u * 1024u && tbg == 4u && gu_items > 256u)
+        hipLaunchKernelGGL((moe_batch_gate_up_kernel<4, 2, GU_TPW, GU_TPI, 2, 4>), dim3(gu_items),
+                           dim3(64 * GU_TPI / GU_TPW), lgu, s, d, L, ws);
     else
-        hipLaunchKernelGGL((moe_batch_gate_up_kernel<1, GU_D, GU_TPW, GU_TPI>), ggu, bgu, (size_t)ximg, s, d, L.table, ws);
+        by_tokens(tbg, [&](auto tb) {
+            constexpr int TB = decltype(tb)::value;
+            hipLaunchKernelGGL((moe_batch_gate_up_kernel<TB, GU_D, GU_TPW, GU_TPI, 4, 1>), dim3(gu_items),
+                               dim3(64 * GU_TPI / GU_TPW), lgu, s, d, L, ws);
+        });
 #ifndef HK_BATCH_AIMG_COLS
 #define HK_BATCH_AIMG_COLS 2048  // activation image columns per block (512: +0.4 us; build-time override)
 #endif
-    hipLaunchKernelGGL(moe_batch_act_image_kernel, dim3(pairs, (d.Imax + HK_BATCH_AIMG_COLS - 1) / HK_BATCH_AIMG_COLS), dim3(256),
-                       (size_t)q4_stage_floats(d.Imax) * sizeof(float), s, d, ws);
-    if (tb_dn >= 4)
-        hipLaunchKernelGGL((moe_batch_down_kernel<4, DN_D, DN_TPW, DN_TPI>), gdn, bdn, (size_t)4 * aimg, s, d, L.table, ws);
-    else if (tb_dn >= 2)
-        hipLaunchKernelGGL((moe_batch_down_kernel<2, DN_D, DN_TPW, DN_TPI>), gdn, bdn, (size_t)2 * aimg, s, d, L.table, ws);
-    else
-        hipLaunchKernelGGL((moe_batch_down_kernel<1, DN_D, DN_TPW, DN_TPI>), gdn, bdn, (size_t)aimg, s, d, L.table, ws);
+    const bool own = dn_items <= OWN_IMAGE_ITEMS;
+    if (!own)
+        hipLaunchKernelGGL(moe_batch_act_image_kernel, dim3(pairs, (d.Imax + HK_BATCH_AIMG_COLS - 1) / HK_BATCH_AIMG_COLS),
+                           dim3(256), (size_t)q4_stage_floats(d.Imax) * sizeof(float), s, d, ws);
+    by_tokens(tbd, [&](auto tb) {
+        constexpr int TB = decltype(tb)::value;
+        const dim3 grid(dn_items), block(64 * DN_TPI / DN_TPW);
+        if (own) hipLaunchKernelGGL((moe_batch_down_kernel<TB, DN_D, DN_TPW, DN_TPI, true>), grid, block, ldn, s, d, L, ws);
+        else hipLaunchKernelGGL((moe_batch_down_kernel<TB, DN_D, DN_TPW, DN_TPI, false>), grid, block, ldn, s, d, L, ws);
+    });
     hipLaunchKernelGGL(moe_batch_combine_kernel, dim3(d.T, (d.H + 255u) / 256u), dim3(256), 0, s, d, ws, y);
     return hipGetLastError();
 }
