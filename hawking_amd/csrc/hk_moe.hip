@@ -47,14 +47,17 @@ size_t moe_down_lds_bytes(int kind, uint32_t Imax, uint32_t slots) {
 
 // Float4s of h (per thread) and of a router row (per lane) held in registers:
 // every global load of the route kernel is issued before its first reduction.
-constexpr int H_PRE = 8;    // 256 threads x 8 float4 = hidden <= 8192
-constexpr int ROW_PRE = 8;  // 64 lanes x 8 float4 = 2048 columns, the rest streamed
+// H_PRE (256 threads x H_PRE float4 >= hidden) and ROW_PRE (64 lanes x ROW_PRE
+// float4 of the row; the rest is streamed) are the smallest that serve hidden:
+// fixed at 8 and 8, the 2048-column case issued 12 clamped duplicates of its 4
+// loads a thread before the norm, and 4096 columns streamed half the row.
+// ROUTEFIG
 
 __device__ __forceinline__ float dot4(const float4& a, const float4& b) {
     return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
 }
 
-template <int KIND>
+template <int KIND, int H_PRE, int ROW_PRE>
 __global__ void __launch_bounds__(256) moe_route_kernel(MoeDims d, MoeLayerDev L, const float* __restrict__ h,
                                                         MoeWs ws) {
     extern __shared__ __align__(16) float xn[];  // [H rounded up to whole steps]
@@ -474,8 +477,11 @@ static hipError_t launch_layer(const MoeDims& d, const MoeLayerDev& L, const flo
     const uint32_t slots = d.K + (d.has_shared ? 1u : 0u);
     const uint32_t gu_tiles = n_tiles_for(d.has_shared ? max(d.I, d.SI) : d.I);
     const uint32_t img_stride = (uint32_t)moe_img_bytes(KIND, d.Imax);
-    hipLaunchKernelGGL(moe_route_kernel<KIND>, dim3(nrb + 1u), dim3(256), moe_route_lds_bytes(KIND, d.H), s, d, L,
-                       h_in, ws);
+    auto* route = d.H <= 1024u   ? moe_route_kernel<KIND, 1, 4>
+                  : d.H <= 2048u ? moe_route_kernel<KIND, 2, 8>
+                  : d.H <= 4096u ? moe_route_kernel<KIND, 4, 16>
+                                 : moe_route_kernel<KIND, 8, 16>;
+    hipLaunchKernelGGL(route, dim3(nrb + 1u), dim3(256), moe_route_lds_bytes(KIND, d.H), s, d, L, h_in, ws);
     const dim3 gg(gu_tiles, slots);
     const size_t gl = moe_gate_up_lds_bytes(KIND, d.H);
     if (d.E <= 512)

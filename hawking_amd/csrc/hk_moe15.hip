@@ -104,26 +104,29 @@ __device__ __forceinline__ float dot4(const float4& a, const float4& b) {
 
 // xn = h * (1 / sqrt(mean(h^2) + eps)) * (1 + w) (source_qwen80_residual_rms_norm,
 // model/qwen80_complete_runtime.rs:6778-6797) held in registers: thread t has chunks t + 256 k
-// (8 columns each, k < M15_NC; hidden <= 8 * 256 * M15_NC).  h and w are
+// (8 columns each, k < NC; NC the smallest of 1, 2, 4 with hidden <= 8 * 256 *
+// NC, so no clamped duplicate loads hold the norm back).  h and w are
 // loaded once, unconditionally (index clamped, value dropped past H), so
 // every load is in flight before the block's one reduction.  Every thread
 // of the 256-thread block calls this (xn_load, then xn_finish; a block
 // with weights to fetch issues them between the two, after h and w: vector
 // loads retire in issue order, so the norm then waits for h and w only).
-constexpr int M15_NC = 4;
+template <int NC>
 struct XnRegs {
-    float4 v[M15_NC][2];
+    float4 v[NC][2];
 };
+template <int NC>
 struct XnW {
-    float4 v[M15_NC][2];
+    float4 v[NC][2];
 };
+template <int NC>
 __device__ __forceinline__ void xn_load(const float* __restrict__ h, const float* __restrict__ w, uint32_t H,
-                                        XnRegs& x, XnW& wv) {
+                                        XnRegs<NC>& x, XnW<NC>& wv) {
     const uint32_t nch = H / 8u;
     const float4* h4 = reinterpret_cast<const float4*>(h);
     const float4* w4 = reinterpret_cast<const float4*>(w);
 #pragma unroll
-    for (int k = 0; k < M15_NC; ++k) {
+    for (int k = 0; k < NC; ++k) {
         const uint32_t ch = min(threadIdx.x + 256u * (uint32_t)k, nch - 1u);
         x.v[k][0] = ldg(h4 + 2u * ch);
         x.v[k][1] = ldg(h4 + 2u * ch + 1u);
@@ -131,15 +134,16 @@ __device__ __forceinline__ void xn_load(const float* __restrict__ h, const float
         wv.v[k][1] = ldg(w4 + 2u * ch + 1u);
     }
 }
-__device__ __forceinline__ void xn_finish(uint32_t H, float eps, float* red, XnRegs& x, const XnW& wv) {
+template <int NC>
+__device__ __forceinline__ void xn_finish(uint32_t H, float eps, float* red, XnRegs<NC>& x, const XnW<NC>& wv) {
     const uint32_t nch = H / 8u;
     float ss = 0.0f;
 #pragma unroll
-    for (int k = 0; k < M15_NC; ++k)
+    for (int k = 0; k < NC; ++k)
         if (threadIdx.x + 256u * (uint32_t)k < nch) ss += dot4(x.v[k][0], x.v[k][0]) + dot4(x.v[k][1], x.v[k][1]);
     const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)H + eps);
 #pragma unroll
-    for (int k = 0; k < M15_NC; ++k)
+    for (int k = 0; k < NC; ++k)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const float4 v = x.v[k][j], g = wv.v[k][j];
@@ -147,9 +151,10 @@ __device__ __forceinline__ void xn_finish(uint32_t H, float eps, float* red, XnR
                                     v.w * inv * (1.0f + g.w));
         }
 }
+template <int NC>
 __device__ __forceinline__ void block_xn(const float* __restrict__ h, const float* __restrict__ w, uint32_t H,
-                                         float eps, float* red, XnRegs& x) {
-    XnW wv;
+                                         float eps, float* red, XnRegs<NC>& x) {
+    XnW<NC> wv;
     xn_load(h, w, H, x, wv);
     xn_finish(H, eps, red, x, wv);
 }
@@ -224,7 +229,7 @@ __device__ __forceinline__ void wave_share(uint32_t S, uint32_t wave, uint32_t& 
 // in registers (h and w issued before the weights) and each thread scatters
 // its chunks of the q8 x image (E = 0: one exponent per 16-column unit, no
 // block-wide maximum) into LDS.
-template <int R, int D = 8 / R>
+template <int R, int NC, int D = 8 / R>
 __device__ __forceinline__ void q8_tile(const M15Dims& d, const M15Dev& L, const float* h, const OrganView (&o)[R],
                                         uint32_t T, uint8_t* lds, float* red, float* part, uint32_t* status,
                                         float* v) {
@@ -233,8 +238,8 @@ __device__ __forceinline__ void q8_tile(const M15Dims& d, const M15Dev& L, const
     const uint32_t S = n_steps_for(HK_Q8, d.H), nch = d.H / 8u;
     uint32_t s0, n;
     wave_share(S, wave, s0, n);
-    XnRegs x;
-    XnW wv;
+    XnRegs<NC> x;
+    XnW<NC> wv;
     xn_load(h, L.norm_w, d.H, x, wv);
     Frag<HK_Q8, R> f[D];
     fetch_first<HK_Q8, R, D>(o, T, s0, n, lane, f);
@@ -244,7 +249,7 @@ __device__ __forceinline__ void q8_tile(const M15Dims& d, const M15Dev& L, const
     xn_finish(d.H, d.eps, red, x, wv);
     bool bad = false;
 #pragma unroll
-    for (int k = 0; k < M15_NC; ++k) {
+    for (int k = 0; k < NC; ++k) {
         const uint32_t ch = threadIdx.x + 256u * (uint32_t)k;
         if (ch < nch) bad |= image_chunk<HK_Q8>(ch, x.v[k], img, sx, 0u, 0u);
     }
@@ -257,6 +262,7 @@ __device__ __forceinline__ void q8_tile(const M15Dims& d, const M15Dev& L, const
     block_rows<R>(acc, part, 0, v);
 }
 
+template <int NC>
 __global__ void __launch_bounds__(256) m15_route_kernel(M15Dims d, M15Dev L, const float* __restrict__ h, M15Ws ws) {
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ float red[8];
@@ -284,12 +290,12 @@ __global__ void __launch_bounds__(256) m15_route_kernel(M15Dims d, M15Dev L, con
     float v[2] = {0.0f, 0.0f};
     if (b < nR) {
         const OrganView o[1] = {L.router};
-        q8_tile<1>(d, L, h, o, b, lds, red, part, ws.status, v);
+        q8_tile<1, NC>(d, L, h, o, b, lds, red, part, ws.status, v);
         const uint32_t row = b * 16u + threadIdx.x;
         if (threadIdx.x < 16 && row < d.E) ws.logits[row] = v[0];
     } else if (b < nR + nG) {
         const OrganView o[1] = {L.sgate};
-        q8_tile<1>(d, L, h, o, 0, lds, red, part, ws.status, v);
+        q8_tile<1, NC>(d, L, h, o, 0, lds, red, part, ws.status, v);
         if (threadIdx.x == 0) {
             // moe_suffix's shared-expert gate: sigmoid, finite and in [0, 1]
             const float g = 1.0f / (1.0f + expf(-v[0]));
@@ -302,7 +308,7 @@ __global__ void __launch_bounds__(256) m15_route_kernel(M15Dims d, M15Dev L, con
         // up projection (the next nS), each block one organ's share
         const uint32_t k = b - nR - nG, which = k >= nS ? 1u : 0u, T = k - which * nS;
         const OrganView o[1] = {which ? L.su : L.sg};
-        q8_tile<1>(d, L, h, o, T, lds, red, part, ws.status, v);
+        q8_tile<1, NC>(d, L, h, o, T, lds, red, part, ws.status, v);
         const uint32_t row = T * 16u + threadIdx.x;
         if (threadIdx.x < 16 && row < d.SI) ws.act_s[which * d.SI + row] = v[0];
     } else {
@@ -310,11 +316,11 @@ __global__ void __launch_bounds__(256) m15_route_kernel(M15Dims d, M15Dev L, con
         // scattered by the wave whose threads hold that step's 64 chunks;
         // the first block publishes xn
         const uint32_t tb = b - nR - nG - 2u * nS, S = n_steps_for(HK_BIN, d.H), nch = d.H / 8u;
-        XnRegs x;
+        XnRegs<NC> x;
         block_xn(h, L.norm_w, d.H, d.eps, red, x);
         if (tb == 0) {
 #pragma unroll
-            for (int k = 0; k < M15_NC; ++k) {
+            for (int k = 0; k < NC; ++k) {
                 const uint32_t ch = threadIdx.x + 256u * (uint32_t)k;
                 if (ch < nch) {
                     reinterpret_cast<float4*>(ws.xn)[2u * ch] = x.v[k][0];
@@ -331,7 +337,7 @@ __global__ void __launch_bounds__(256) m15_route_kernel(M15Dims d, M15Dev L, con
             image_zero_blocks<HK_BIN>(lane, tiles, 1u);
             bool bad = false;
 #pragma unroll
-            for (int k = 0; k < M15_NC; ++k)
+            for (int k = 0; k < NC; ++k)
                 if ((uint32_t)k == (tb >> 2)) bad = image_chunk<HK_BIN>(64u * tb + lane, x.v[k], tiles, sx, 64u * tb, 8u * tb);
             if (__ballot(bad) != 0 && lane == 0) atomicOr(ws.status, HK_DEVERR_NONFINITE);
         }
@@ -782,7 +788,8 @@ extern "C" int hk_moe15_decode_layer(hk_ctx* ctx, hk_moe15_layer* L, const float
         return set_error(ctx, HK_E_INVALID_ARG, "hk_moe15_decode_layer: h must be 16-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const M15Dims& d = L->d;
-    hipLaunchKernelGGL(m15_route_kernel, dim3(L->n_route_blocks), dim3(256), L->lds_route, s, d, L->dev, h, L->ws);
+    auto* route = d.H <= 2048u ? m15_route_kernel<1> : d.H <= 4096u ? m15_route_kernel<2> : m15_route_kernel<4>;
+    hipLaunchKernelGGL(route, dim3(L->n_route_blocks), dim3(256), L->lds_route, s, d, L->dev, h, L->ws);
     const dim3 gg(n_tiles_for(d.I), d.K);
     if (d.E <= 64)
         hipLaunchKernelGGL((m15_gate_up_kernel<1>), gg, dim3(256), L->lds_gu, s, d, L->dev, L->ws, ids, weights);
