@@ -1213,7 +1213,6 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     constexpr int D = KIND == HK_MIXED ? 2 : 4;
     *done = false;
     SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
-//SWEEP
     if (!c.waves) return hipSuccess;
     const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw;
     const size_t lds = SplitLds<KIND, ORD, RES>(sh.steps, sh.cols, tpw, ks).total;

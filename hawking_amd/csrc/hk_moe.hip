@@ -53,8 +53,10 @@ size_t moe_down_lds_bytes(int kind, uint32_t Imax, uint32_t slots) {
 // loads a thread before the norm, and 4096 columns streamed half the row.
 // 48-layer mixed token 826 -> 817 us.
 
+// Explicit fused steps: left to contraction, the first pair's order (and so the
+// bits) depends on the instantiation.
 __device__ __forceinline__ float dot4(const float4& a, const float4& b) {
-    return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
+    return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.x, b.x, a.y * b.y)));
 }
 
 template <int KIND, int H_PRE, int ROW_PRE>

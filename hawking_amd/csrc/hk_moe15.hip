@@ -98,8 +98,10 @@ struct M15Ws {
     uint32_t* status;
 };
 
+// Explicit fused steps: left to contraction, the first pair's order (and so the
+// bits) depends on the instantiation.
 __device__ __forceinline__ float dot4(const float4& a, const float4& b) {
-    return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
+    return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.x, b.x, a.y * b.y)));
 }
 
 // xn = h * (1 / sqrt(mean(h^2) + eps)) * (1 + w) (source_qwen80_residual_rms_norm,

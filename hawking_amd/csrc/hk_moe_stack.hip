@@ -161,8 +161,10 @@ __device__ __forceinline__ uint32_t fresh_tid() {
     return t;
 }
 
+// Explicit fused steps: left to contraction, the first pair's order (and so the
+// bits) depends on the instantiation.
 __device__ __forceinline__ float dot4s(const float4& a, const float4& b) {
-    return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
+    return fmaf(a.w, b.w, fmaf(a.z, b.z, fmaf(a.x, b.x, a.y * b.y)));
 }
 
 // Waits (one wave) until the n <= 64 NR ready words rdy[] carry `tag`; the
