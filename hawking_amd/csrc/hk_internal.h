@@ -392,7 +392,7 @@ hipError_t launch_head_norm(const float* h, const float* w, uint32_t n, float ep
 hipError_t launch_head_argmax(const float* logits, uint32_t n_valid, uint64_t* key, int32_t* token, uint32_t* status,
                               hipStream_t s);
 // HGRAVS01 pairs y_i = L_i (R_i x_i) (3-bit factors, right rows = left cols)
-// in one launch, one workgroup per pair; mid (may be null) receives R_i x_i.
+// in one launch, mid kept on chip; mid (may be null) receives R_i x_i.
 // lowrank_fusable: the shapes this kernel takes (right cols <= 8192, rank <=
 // 2048, LDS within the cap); launch_lowrank returns hipErrorInvalidValue
 // otherwise.

@@ -17,7 +17,8 @@
 //   5. gate/up:  per (active expert, 8 row tiles): the member tokens' x images
 //                in LDS, each wave runs two gate+up tile pairs over all columns
 //                and applies SwiGLU
-//   6. act image: the x image of every (token, expert) activation row
+//   6. act image: the x image of every (token, expert) activation row (batches
+//                of few down items build theirs in step 7 instead)
 //   7. down:     per (active expert, 8 row tiles): w * (down . act) per member
 //   8. combine:  y_t = sum over t's experts in ascending id, then + shared
 #include <type_traits>

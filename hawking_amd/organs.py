@@ -173,7 +173,7 @@ class UniformFactor3(PackedOrgan):
 
 class HgravS01LowRank:
     """W ~= L R with L rows x rank and R rank x cols (HGRAVS01): y = L (R x)
-    as two launches through a device mid vector of `rank` floats."""
+    (hk_gemv_lowrank), with a device mid vector of `rank` floats."""
 
     def __init__(self, left: UniformFactor3, right: UniformFactor3):
         if right.rows != left.cols:

@@ -218,7 +218,7 @@ int hk_gemv_lowrank(hk_ctx* ctx, const hk_organ* left, const hk_organ* right, co
                     float* mid, float* y, hk_stream stream);
 /* y_i = L_i (R_i x_i) for the n HGRAVS01 pairs of two organ sets (left set of
  * HK_U3 rows x rank, right set of HK_U3 rank x cols, the same n), streamed in
- * ONE launch (one workgroup per pair, mid kept on chip) for the shapes
+ * ONE launch (mid kept on chip) for the shapes
  * hk_gemv_lowrank fuses, else two set launches ordered on `stream` through
  * mid.  mid (device, mid_i = mid + i*mid_stride, 16-byte aligned) may be
  * NULL when the pair is fused; when given it receives R_i x_i; the two-launch
