@@ -17,8 +17,7 @@
 //   5. gate/up:  per (active expert, 8 row tiles): the member tokens' x images
 //                in LDS, each wave runs two gate+up tile pairs over all columns
 //                and applies SwiGLU
-//   6. act image: the x image of every (token, expert) activation row (batches
-//                of few down items build theirs in step 7 instead)
+//   6. act image: the x image of every (token, expert) activation row
 //   7. down:     per (active expert, 8 row tiles): w * (down . act) per member
 //   8. combine:  y_t = sum over t's experts in ascending id, then + shared
 #include <type_traits>
@@ -666,10 +665,7 @@ __global__ void __launch_bounds__(256) moe_batch_act_image_kernel(MoeBatchDims d
 
 // ------------------------------------------------------------------ 7. down (grouped)
 
-// OWN: the workgroup builds its members' activation images itself (E = 0: the
-// image launch's bits, its exponent aside), for batches of few items, where
-// the image launch costs more than the repeated builds.
-template <int TB, int D, int TPW, int TPI, bool OWN>
+template <int TB, int D, int TPW, int TPI>
 __global__ void __launch_bounds__(64 * TPI / TPW)
 moe_batch_down_kernel(MoeBatchDims d, MoeLayerDev L, MoeBatchWs ws) {
     extern __shared__ __align__(16) uint8_t lds[];  // TB activation images
@@ -701,33 +697,9 @@ moe_batch_down_kernel(MoeBatchDims d, MoeLayerDev L, MoeBatchWs ws) {
 #pragma unroll
         for (int j = 0; j < TB; ++j) pair[j] = ws.members[it.ent.y + m0 + min((uint32_t)j, nm - 1u)];
         Frag<HK_Q4, TPW> f[D];
-        if constexpr (OWN) {
-            const uint32_t nch = S * tile_step_cols(HK_Q4) / 8u;
-            float4 v[TB][2];  // the first chunk of each, before the weights
-#pragma unroll
-            for (int j = 0; j < TB; ++j) load_chunk(ws.act + (size_t)pair[j] * d.Imax, 8u * threadIdx.x, o.cols, v[j]);
-            if (vw[0]) tiles_fetch_first<TPW, D>(bd, bs, S, f);
-            __syncthreads();
-            bool bad = false;
-#pragma unroll
-            for (int j = 0; j < TB; ++j) {
-                if ((uint32_t)j >= nm) break;
-                uint8_t* img = lds + (size_t)j * img_bytes;
-                float* sx = reinterpret_cast<float*>(img + (size_t)S * Kcfg<HK_Q4>::P * A_TILE_STRIDE);
-                if (threadIdx.x < 64u) image_zero_blocks<HK_Q4>(threadIdx.x, img, S);
-                if (threadIdx.x < nch) bad |= image_chunk<HK_Q4>(threadIdx.x, v[j], img, sx, 0u, 0u);
-                for (uint32_t ch = threadIdx.x + blockDim.x; ch < nch; ch += blockDim.x) {
-                    float4 c[2];
-                    load_chunk(ws.act + (size_t)pair[j] * d.Imax, 8u * ch, o.cols, c);
-                    bad |= image_chunk<HK_Q4>(ch, c, img, sx, 0u, 0u);
-                }
-            }
-            if (bad) atomicOr(ws.status, HK_DEVERR_NONFINITE);
-        } else {
-            if (vw[0]) tiles_fetch_first<TPW, D>(bd, bs, S, f);
-            __syncthreads();
-            stage_images<TB, 2>(lds, ws.aimg, ws.aimg_stride, pair, nm, img_bytes);
-        }
+        if (vw[0]) tiles_fetch_first<TPW, D>(bd, bs, S, f);
+        __syncthreads();
+        stage_images<TB, 2>(lds, ws.aimg, ws.aimg_stride, pair, nm, img_bytes);
         __syncthreads();
         if (!vw[0]) continue;
         float acc[TB][TPW] = {};
@@ -735,7 +707,7 @@ moe_batch_down_kernel(MoeBatchDims d, MoeLayerDev L, MoeBatchWs ws) {
 #pragma unroll
         for (int j = 0; j < TB; ++j) {
             if ((uint32_t)j >= nm) break;
-            const int E = OWN ? 0 : ws.aimg_e[pair[j]];
+            const int E = ws.aimg_e[pair[j]];
             const bool routed = pair[j] < np;
             const float w = routed ? ws.w[pair[j]] : 1.0f;
             // a routed pair's output goes to its token's row of its rank in expert order
@@ -794,12 +766,6 @@ static void by_tokens(uint32_t tb, F f) {
     else if (tb >= 2) f(std::integral_constant<int, 2>{});
     else f(std::integral_constant<int, 1>{});
 }
-
-// Down items up to which the down kernel builds its activation images itself:
-// hidden 4096 x 1024, 2 tokens (416 items) 49.2 -> 47.2 us a step, 7168 x 2048,
-// 1 token (504) 69.7 -> 66.7, 2176 x 256, 1 token (51) 33.9 -> 31.1; 4096 x 1024,
-// 8 tokens (1,600) 88.2 against 90.6.
-constexpr uint32_t OWN_IMAGE_ITEMS = 512;
 
 hipError_t launch_moe_batch(const MoeBatchDims& d, const MoeLayerDev& L, const float* bias, const uint16_t* x_bf16,
                             float* y, const MoeBatchWs& ws, int32_t* ids_out, float* w_out, hipStream_t s) {
@@ -860,15 +826,12 @@ hipError_t launch_moe_batch(const MoeBatchDims& d, const MoeLayerDev& L, const f
 #ifndef HK_BATCH_AIMG_COLS
 #define HK_BATCH_AIMG_COLS 2048  // activation image columns per block (512: +0.4 us; build-time override)
 #endif
-    const bool own = dn_items <= OWN_IMAGE_ITEMS;
-    if (!own)
-        hipLaunchKernelGGL(moe_batch_act_image_kernel, dim3(pairs, (d.Imax + HK_BATCH_AIMG_COLS - 1) / HK_BATCH_AIMG_COLS),
-                           dim3(256), (size_t)q4_stage_floats(d.Imax) * sizeof(float), s, d, ws);
+    hipLaunchKernelGGL(moe_batch_act_image_kernel, dim3(pairs, (d.Imax + HK_BATCH_AIMG_COLS - 1) / HK_BATCH_AIMG_COLS),
+                       dim3(256), (size_t)q4_stage_floats(d.Imax) * sizeof(float), s, d, ws);
     by_tokens(tbd, [&](auto tb) {
         constexpr int TB = decltype(tb)::value;
-        const dim3 grid(dn_items), block(64 * DN_TPI / DN_TPW);
-        if (own) hipLaunchKernelGGL((moe_batch_down_kernel<TB, DN_D, DN_TPW, DN_TPI, true>), grid, block, ldn, s, d, L, ws);
-        else hipLaunchKernelGGL((moe_batch_down_kernel<TB, DN_D, DN_TPW, DN_TPI, false>), grid, block, ldn, s, d, L, ws);
+        hipLaunchKernelGGL((moe_batch_down_kernel<TB, DN_D, DN_TPW, DN_TPI>), dim3(dn_items), dim3(64 * DN_TPI / DN_TPW), ldn,
+                           s, d, L, ws);
     });
     hipLaunchKernelGGL(moe_batch_combine_kernel, dim3(d.T, (d.H + 255u) / 256u), dim3(256), 0, s, d, ws, y);
     return hipGetLastError();

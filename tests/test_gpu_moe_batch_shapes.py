@@ -1,5 +1,5 @@
 """The batched block's launch shapes: gate/up with one or two workgroups a CU,
-down with its own or staged activation images, routed and shared intermediates
+routed and shared intermediates
 of different sizes.  A token's output must be the same bits in every batch it
 runs in, and within tolerance of the oracle."""
 from __future__ import annotations
@@ -52,3 +52,22 @@ def test_batch_shapes(ctx, oracle, H, I, SI, E, K, T):
     if U.noaux_margin_ok(oracle.gemv_f32(router, x), U.router_bias(oracle, U.SEED, shape, 0), 1, 1, K):
         assert ids[0].tolist() == rids.tolist()
         assert oracle.relative_l2(y[0], out) < 2e-5
+
+
+def test_batch_shapes_tiny_activations(ctx):
+    """Activations near 2^-112 keep their precision in every batch: the images
+    carry an exponent each, so a token's bits do not depend on the batch."""
+    from hawking_amd.moe import MoeModel, MoeShape
+    print("[gpu-case] batch tiny activations", flush=True)
+    H, T = 1024, 40
+    shape = MoeShape(n_layers=1, hidden=H, inter=768, shared_inter=128, n_experts=32, top_k=8, expert_kind=U.HK_Q4,
+                     expert_group=32, shared_gate=False, router=1, routed_scaling_factor=2.5)
+    m = MoeModel(ctx, shape)
+    m.fill_synthetic(U.SEED)
+    x = np.random.default_rng(7).standard_normal((T, H)).astype(np.float32) * np.float32(2.0 ** -56)
+    xb = U.to_bf16_bits(x).reshape(T, H)
+    y, ids, _ = m.routed_moe(0, xb)
+    assert ctx.device_status() == 0 and np.abs(y).max() > 0.0
+    for t in (0, T - 1):
+        y1, ids1, _ = m.routed_moe(0, xb[t:t + 1])
+        assert np.array_equal(ids1[0], ids[t]) and np.array_equal(y1[0], y[t]), f"token {t} depends on the batch"
