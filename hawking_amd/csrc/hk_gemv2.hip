@@ -863,8 +863,8 @@ static hipError_t launch_kind(const OrganView* organs, uint32_t n, const OrganVi
 // part of the x image.  A single organ's view comes with the kernel
 // arguments (one round trip fewer than a descriptor load).
 struct SplitArgs {
-    OrganView one;            // n = 1: the organ
-    const OrganView* organs;  // else the set's table
+    OrganView one;            // organs null: the one organ
+    const OrganView* organs;  // else the table of the n organs
     ResView res_one;          // RES, the same way
     const ResView* res;
     const float* x;
@@ -1217,12 +1217,15 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw;
     const size_t lds = SplitLds<KIND, ORD, RES>(sh.steps, sh.cols, tpw, ks).total;
     if (lds > SPLIT_LDS_LIMIT) return hipSuccess;
+    if (RES && (!organs || !res) && !(n == 1 && res_one)) return hipErrorInvalidValue;
     *done = true;
     SplitArgs a{};
     a.ks_log = (uint32_t)__builtin_ctz(ks);
     a.ts_log = (uint32_t)__builtin_ctz(waves / ks);
     a.one = sh;
-    a.organs = n > 1 ? organs : nullptr;
+    // one organ's view comes with the arguments where the host has its
+    // residual's too (a set of one has that only in its device table)
+    a.organs = n > 1 || (RES && !res_one) ? organs : nullptr;
     if (res_one) a.res_one = *res_one;
     a.res = res;
     a.x = x;

@@ -305,8 +305,8 @@ constexpr size_t GEMV_LDS_LIMIT = 64 * 1024;
 struct ResView;
 // The binary GEMV of HGRAVR02 organs with the residual added in the same
 // launch (the bits of launch_gemv_tiled then launch_rice_apply); res_one: a
-// host copy of the residual's view for n = 1 (else null); pieces256 /
-// pieces512: rice_part_pieces8 of the organs for 256- and 512-row parts.
+// host copy of the residual's view where n = 1 and the caller has one, else
+// null (res_dev is read); pieces256 / pieces512: rice_part_pieces8 of the organs for 256- and 512-row parts.
 // *fused = false (nothing launched) when the launch shape has no fused form.
 hipError_t launch_gemv_rice(const OrganView* organs_dev, const ResView* res_dev, const ResView* res_one, uint32_t n,
                             const OrganView& sh, uint32_t pieces256, uint32_t pieces512, const float* x,

@@ -98,3 +98,23 @@ def test_split_sums_are_the_streamed_sums(ctx, oracle, kind, rows, cols):
     got = y.download()
     for i in (0, 5, n // 2 + 3, n - 1):
         assert np.array_equal(got[i], base[i % 8].matvec(xs[i])), i
+
+
+ONE = [(k, 300, 1024) for k in KIND] + [("rice", 8, 128), ("rice", 65536, 128), ("bin", 40, 512)]
+
+
+@pytest.mark.parametrize("kind,rows,cols", ONE, ids=[f"{k}-{r}x{c}" for k, r, c in ONE])
+def test_set_of_one_organ(ctx, oracle, kind, rows, cols):
+    """A set of one organ (its views only in the set's device tables) is the
+    organ's own call to the bit."""
+    from hawking_amd.organs import OrganSet
+    print("[gpu-case] split gemv, set of one", kind, rows, cols, flush=True)
+    sys.stdout.flush()
+    o = _organ(ctx, oracle, kind, rows, cols, 0x3000 + ONE.index((kind, rows, cols)))
+    x = np.random.default_rng(rows).standard_normal(cols).astype(np.float32)
+    y = ctx.to_device(np.full((1, rows + 4), 7.0, np.float32))
+    OrganSet(ctx, [o]).gemv(ctx.to_device(x), cols, y, (rows + 4) // 4 * 4)
+    got = y.download()[0]
+    assert np.array_equal(got[:rows], o.matvec(x)) and np.all(got[rows:] == 7.0)
+    edge = min(48, rows)
+    _check_rows(o, kind, x, got, [(0, edge), (rows - edge, edge)])
