@@ -7,6 +7,8 @@
 // (16 rows each) of its slice of the organ; one LDS operand fetch feeds the R
 // tiles' MFMAs and the next step's weight loads are in flight while the
 // current step computes.
+#include <type_traits>
+
 #include "hk_mfma.h"
 #include "hk_rice.h"
 
@@ -67,7 +69,7 @@ __device__ __forceinline__ void flush_group(float* acc, const uint32_t* T, int n
     }
 }
 
-constexpr size_t SPLIT_LDS_LIMIT = 96 * 1024;  // of the small launches (one workgroup per CU)
+constexpr size_t LOWRANK_LDS_LIMIT = 96 * 1024;  // of few pairs' launches (one workgroup per CU)
 
 // Mixed step headers staged per workgroup: tiles x steps <= 32 x 24.
 constexpr uint32_t GEMV_MAX_MIXED_TILES_PER_WG = 32;
@@ -779,7 +781,7 @@ hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint3
         a.parts = (l.n_tiles + a.tpw - 1u) / a.tpw;
         a.round = std::min(std::min(LOWRANK_ROUND, r.n_tiles), 128u / r.steps);
         const size_t sl = LowrankSplitLds(l, r, a.round).total;
-        if (a.round && sl <= SPLIT_LDS_LIMIT) {
+        if (a.round && sl <= LOWRANK_LDS_LIMIT) {
             a.left = l;
             a.right = r;
             a.lefts = n > 1 ? lefts : nullptr;
@@ -873,39 +875,53 @@ struct SplitArgs {
     uint32_t n, parts;        // organs, workgroups per organ
     uint32_t tpw;             // tiles per workgroup, a multiple of TS
     uint32_t ks_log, ts_log;  // log2 KS, log2 TS
+    uint32_t bufs;            // KS > 1: buffers of a chunk's terms (one: a single chunk)
     HeadArgs ha;              // HEAD: the terminal head's prologue and epilogue
     uint32_t* status;
 };
 
+constexpr size_t SPLIT_LDS_LIMIT = 128 * 1024;
+
 // LDS: the x image, then (RES) a copy of x and the residual's products, then
-// the terms of every (tile, step) {scale, v} (ORD with KS > 1) or one partial
-// row sum per (K slice, row), then (RES) the rows' base sums.
-template <int KIND, bool ORD, bool RES>
+// (KS > 1) the {scale, v} terms of a chunk of steps of every tile of a round,
+// then (RES) the rows' base sums.
+template <int KIND, bool RES>
 struct SplitLds {
+    static constexpr uint32_t TERMS = KIND == HK_MIXED ? 2u : 1u;  // a step's
+    uint32_t chunk;  // items of a wave between barriers
     size_t xs, vals, terms, ysh, total;
-    __host__ __device__ SplitLds(uint32_t S, uint32_t cols, uint32_t tpw, uint32_t ks) {
-        constexpr size_t TERM = KIND == HK_MIXED ? 16 : 8;
+    __host__ __device__ SplitLds(uint32_t S, uint32_t cols, uint32_t tpw, uint32_t waves, uint32_t per, uint32_t bufs)
+        : chunk(per < 4u ? per : 4u) {
         xs = (x_lds_bytes<KIND>(S) + 15u) & ~(size_t)15;
         vals = xs + (RES ? (size_t)cols * 4u : 0);
         terms = vals + (RES ? (size_t)RICE_BATCH * 4u : 0);
-        ysh = terms + (ORD && ks > 1 ? (size_t)tpw * S * 64u * TERM : (size_t)ks * tpw * 64u);
+        ysh = terms + (size_t)bufs * waves * chunk * TERMS * 512u;  // (bufs 0: KS = 1)
         total = ysh + (RES ? (size_t)tpw * 64u : 0);
     }
 };
 
-// ORD: a row's terms are added in step order whatever KS is: the waves leave
-// each lane's {scale, v} in LDS and one wave per tile runs the same chain of
-// fused multiply-adds that one wave walking the tile would, so the sums are
-// the streamed launches' to the bit.  Otherwise (Q4, Q8: 16 to 128 steps) each
-// wave sums its own slice and the slices are added in order.
+// A row's terms are added in step order whatever KS is, so an organ's sums are
+// the same bits alone, in a set of any size and as an lm_head.  KS = 1: a wave
+// walks its tiles (t0 + its index, + TS, ...).  SPLIT (KS > 1): the workgroup
+// takes TS tiles a round, wave k of a tile its steps k, k + KS, ...; the waves
+// leave each lane's {scale, v} in LDS and, every four items, one wave per tile
+// (another each round) runs the same chain of fused multiply-adds that one
+// wave walking the tile would, while the others are in the next items.  Every
+// wave runs the same number of items, so all meet at each barrier; items past
+// the tile's steps re-read a valid one and leave {-0, 0}, which changes no
+// sum.  (The chain is in the code once: inlined after every item of the
+// unrolled loop it cost up to 1 us of instruction fetches, 20 q8 512 x 2048 5.6
+// against 5.1.)
 // RES: the HGRAVR02 residual added to the base sums in the same launch (256
-// threads; records loaded before the image build).
+// threads; one round; records loaded before the image build).
 // HEAD: x is the hidden state; the prologue forms RMSNorm(1+w) of it and the
 // epilogue folds the rows' greedy keys (HeadArgs; cols <= 8192, 512 threads).
 // NT: the weight loads carry the non-temporal hint.
-template <int KIND, int D, bool ORD, bool RES, bool HEAD, bool NT = false>
+template <int KIND, bool SPLIT, bool RES, bool HEAD, bool NT = false>
 __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs a) {
     static_assert(!(RES && HEAD), "an lm_head has no fused residual");
+    constexpr uint32_t D = KIND == HK_MIXED ? 2 : 4;  // steps in flight per wave
+    constexpr uint32_t TERMS = SplitLds<KIND, RES>::TERMS;
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ float red[HEAD ? 16 : 1];
     __shared__ uint64_t kred[HEAD ? 16 : 1];
@@ -923,10 +939,14 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nthr = blockDim.x;
     const uint32_t S = o.steps, KS = 1u << a.ks_log, TS = 1u << a.ts_log;
     const uint32_t ksl = wave & (KS - 1u), tsl = wave >> a.ks_log;
-    const uint32_t per = (S + KS - 1u) >> a.ks_log, s0 = min(ksl * per, S), ns = min(per, S - s0);
-    const uint32_t t0 = part * a.tpw, t1 = min(t0 + a.tpw, o.n_tiles), tf = t0 + tsl;
-    const uint32_t n = tf < t1 ? ((t1 - tf + TS - 1u) >> a.ts_log) * ns : 0u;  // this wave's (tile, step) items
-    const SplitLds<KIND, ORD, RES> M(S, o.cols, a.tpw, KS);
+    const uint32_t t0 = part * a.tpw, t1 = min(t0 + a.tpw, o.n_tiles);
+    // SPLIT: item j of a wave is step ksl + KS j of its tile, per items a
+    // tile, D of them in flight
+    const uint32_t per = SPLIT ? (S + KS - 1u) >> a.ks_log : S;
+    // (KS = 1: a wave may have no tile)
+    const uint32_t rounds = SPLIT || t0 + tsl < t1 ? (t1 - t0 - (SPLIT ? 0u : tsl) + TS - 1u) >> a.ts_log : 0u;
+    const uint32_t n = rounds * per;
+    const SplitLds<KIND, RES> M(S, o.cols, a.tpw, nthr >> 6, per, a.bufs);
 
     constexpr int NC = 2;  // (HEAD: 512 threads x 2 chunks = 8192 columns, all in registers)
     XChunks<NC> xc;
@@ -936,31 +956,33 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     RiceTile rt;
     const uint32_t r0 = t0 * 16u, r1 = min(t1 * 16u, o.rows);
     if constexpr (RES) rice_ranges(rv, r0, r1, rt);
-    // the first D items, unconditionally (a wave with fewer re-reads its last)
-    uint32_t fT = n ? tf : t0, fs = n ? s0 : 0u, fi = 0;
+    // the first D items, unconditionally (past its last a wave re-reads a valid
+    // one)
+    uint32_t fT = t0 + tsl, fj = 0, fi = 0;
     auto step_on = [&]() {
-        if (++fi < n) {
-            ++fs;
-            if (fs == s0 + ns) {
-                fs = s0;
-                fT += TS;
-            }
+        if constexpr (SPLIT) {
+            ++fj;
+        } else if (++fi < n && ++fj == per) {
+            fj = 0;
+            fT += TS;
         }
     };
+    auto f_tile = [&]() { return min(fT, t1 - 1u); };
+    auto f_step = [&]() { return SPLIT ? min(ksl + (fj << a.ks_log), S - 1u) : fj; };
     Frag<KIND, 1> f[D];
     if constexpr (KIND == HK_MIXED) {
         uint4 h[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            h[d] = ldg(o.hdr + (fT * S + fs));
+        for (uint32_t d = 0; d < D; ++d) {
+            h[d] = ldg(o.hdr + (f_tile() * S + f_step()));
             step_on();
         }
 #pragma unroll
-        for (int d = 0; d < D; ++d) fetch_mixed<1>(o, h[d], lane, f[d], 0);
+        for (uint32_t d = 0; d < D; ++d) fetch_mixed<1>(o, h[d], lane, f[d], 0);
     } else {
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            fetch_one<KIND, 1, NT>(o, fT, fs, lane, f[d], 0);
+        for (uint32_t d = 0; d < D; ++d) {
+            fetch_one<KIND, 1, NT>(o, f_tile(), f_step(), lane, f[d], 0);
             step_on();
         }
     }
@@ -1001,78 +1023,105 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     }
 
     const ImageA A{lds, a_lane_offset(lane)};
-    float* terms = reinterpret_cast<float*>(lds + M.terms);
-    const bool split = ORD && KS > 1u;
-    float acc = 0.0f;
-    uint32_t cT = tf, cs = s0;
-    auto consume = [&](const Frag<KIND, 1>& fr) {
-        if (split) {
-            constexpr uint32_t TERMS = KIND == HK_MIXED ? 2u : 1u;
-            float2* o2 = reinterpret_cast<float2*>(terms) + ((cT - t0) * S + cs) * 64u * TERMS + (uint32_t)lane * TERMS;
-            uint32_t k = 0;
-            compute_terms<KIND, 1>(fr, cs, A, sx, q, [&](int, float s, float v) { o2[k++] = make_float2(s, v); });
-        } else {
-            compute_step<KIND, 1>(fr, cs, A, sx, q, &acc);
-            if (cs + 1u == s0 + ns) {
-                const float v = tile_row_sum(acc);
-                if (lane < 16) terms[(ksl * a.tpw + cT - t0) * 16u + (uint32_t)lane] = v;
-                acc = 0.0f;
-            }
-        }
-        ++cs;
-        if (cs == s0 + ns) {
-            cs = s0;
-            cT += TS;
-        }
-    };
-    uint32_t it = 0;
-    for (; it + D < n; it += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            consume(f[d]);
-            fetch_one<KIND, 1, NT>(o, fT, fs, lane, f[d], 0);
-            step_on();
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-        if (it + (uint32_t)d < n) consume(f[d]);
-    __syncthreads();
-
+    float2* terms = reinterpret_cast<float2*>(lds + M.terms) + (uint32_t)lane * TERMS;  // + 64 TERMS a step
     float* ysh = reinterpret_cast<float*>(lds + M.ysh);
     uint64_t best = 0;
-    auto put = [&](uint32_t i, float v) {  // row i of the workgroup
+    auto put_tile = [&](uint32_t T, float v) {  // v: this lane's part of the tile's row sums
+        v = tile_row_sum(v);
+        const uint32_t row = T * 16u + (uint32_t)lane;
+        if (lane >= 16) return;
         if constexpr (RES) {
-            ysh[i] = v;
-        } else if (r0 + i < o.rows) {
-            y[r0 + i] = v;
+            ysh[row - r0] = v;
+        } else if (row < o.rows) {
+            y[row] = v;
             if constexpr (HEAD)
-                if (r0 + i < a.ha.n_valid) best = max(best, greedy_key(v, r0 + i));
+                if (row < a.ha.n_valid) best = max(best, greedy_key(v, row));
         }
     };
-    if (split) {
-        constexpr uint32_t TERMS = KIND == HK_MIXED ? 2u : 1u;
-        for (uint32_t T = wave; T < t1 - t0; T += nthr >> 6) {
-            const float2* t2 = reinterpret_cast<const float2*>(terms) + T * S * 64u * TERMS + (uint32_t)lane * TERMS;
-            float v = 0.0f;
-#pragma unroll 4
-            for (uint32_t s = 0; s < S; ++s)
-#pragma unroll
-                for (uint32_t h = 0; h < TERMS; ++h) {
-                    const float2 e = t2[s * 64u * TERMS + h];
-                    v = __builtin_fmaf(e.x, e.y, v);
+    float acc = 0.0f;  // SPLIT: of the tile that this wave sums
+    if constexpr (SPLIT) {
+        uint32_t buf = 0;
+        for (uint32_t round = 0; round < rounds; ++round)
+            for (uint32_t j0 = 0; j0 < per; j0 += D) {
+                // chunks of 4 items: this group's first slot
+                const uint32_t c0 = j0 & 3u;
+                const bool last = j0 + D >= per;  // of the tile
+                if (last) {
+                    fj = 0;
+                    fT += TS;
                 }
-            v = tile_row_sum(v);
-            if (lane < 16) put(T * 16u + (uint32_t)lane, v);
-        }
+                auto leave = [&](uint32_t d) {
+                    if (j0 + d >= per) return;
+                    const uint32_t cs = ksl + ((j0 + d) << a.ks_log);
+                    const bool on = cs < S;
+                    float2* o2 = terms + (((((buf << a.ts_log) + tsl) * M.chunk + c0 + d) << a.ks_log) + ksl) * 64u * TERMS;
+                    compute_terms<KIND, 1>(f[d], min(cs, S - 1u), A, sx, q, [&](int, float s, float v) {
+                        *o2++ = make_float2(on ? s : -0.0f, on ? v : 0.0f);
+                    });
+                };
+                // (two bodies: a load under a condition would have every later
+                // item wait for all loads)
+                if (!last || round + 1u < rounds) {
+#pragma unroll
+                    for (uint32_t d = 0; d < D; ++d) {
+                        leave(d);
+                        fetch_one<KIND, 1, NT>(o, f_tile(), f_step(), lane, f[d], 0);
+                        step_on();
+                    }
+                } else {
+#pragma unroll
+                    for (uint32_t d = 0; d < D; ++d) leave(d);
+                }
+                if (!last && c0 + D < 4u) continue;
+                __syncthreads();
+                // the chunk's terms of the round's tiles, one tile per wave
+                const uint32_t k = (wave - (round << a.ts_log)) & ((nthr >> 6) - 1u), T = t0 + (round << a.ts_log) + k;
+                if (k < TS && T < t1) {
+                    const float2* t = terms + (((buf << a.ts_log) + k) * M.chunk << a.ks_log) * 64u * TERMS;
+                    const uint32_t m = (min(c0 + D, per - (j0 - c0)) << a.ks_log) * TERMS;  // a multiple of 2
+                    auto add = [&](auto count) {
+                        constexpr uint32_t N = decltype(count)::value;
+                        float2 e[N];
+#pragma unroll
+                        for (uint32_t u = 0; u < N; ++u) e[u] = t[u / TERMS * 64u * TERMS + u % TERMS];
+#pragma unroll
+                        for (uint32_t u = 0; u < N; ++u) acc = __builtin_fmaf(e[u].x, e[u].y, acc);
+                        t += N * 64u;
+                    };
+                    for (uint32_t i = m >> 4; i; --i) add(std::integral_constant<uint32_t, 16>{});
+                    if (m & 8u) add(std::integral_constant<uint32_t, 8>{});
+                    if (m & 4u) add(std::integral_constant<uint32_t, 4>{});
+                    if (m & 2u) add(std::integral_constant<uint32_t, 2>{});
+                    if (last) {
+                        put_tile(T, acc);
+                        acc = 0.0f;
+                    }
+                }
+                buf ^= a.bufs - 1u;
+            }
     } else {
-        for (uint32_t i = threadIdx.x; i < (t1 - t0) * 16u; i += nthr) {
-            float v = terms[i];
-            // (slices past the last step hold no sums)
-            for (uint32_t k = 1; k * per < S && k < KS; ++k) v += terms[k * a.tpw * 16u + i];
-            put(i, v);
+        uint32_t cT = t0 + tsl, cj = 0, it = 0;
+        auto consume = [&](const Frag<KIND, 1>& fr) {
+            compute_step<KIND, 1>(fr, cj, A, sx, q, &acc);
+            if (++cj < per) return;
+            put_tile(cT, acc);
+            acc = 0.0f;
+            cj = 0;
+            cT += TS;
+        };
+        for (; it + D < n; it += D) {
+#pragma unroll
+            for (uint32_t d = 0; d < D; ++d) {
+                consume(f[d]);
+                fetch_one<KIND, 1, NT>(o, f_tile(), f_step(), lane, f[d], 0);
+                step_on();
+            }
         }
+#pragma unroll
+        for (uint32_t d = 0; d < D; ++d)
+            if (it + d < n) consume(f[d]);
     }
+
     if constexpr (RES) {
         __syncthreads();
         float racc[2];
@@ -1143,64 +1192,67 @@ static uint32_t pow2_ceil(uint32_t v) {
     return p;
 }
 
-// Where the split pays and its shape (us per launch in a graph of one launch,
-// split against the walk of gemv_tiled_kernel; organs of 512 x 2048 unless
-// stated):
-//   * one step (<= 512 binary columns): nothing to split (2.92 against 2.89);
-//   * up to 2,048 row tiles the workgroups are what is scarce: about one per
+// Where the split pays and its shape (us per launch, 20 launches in a graph;
+// against the walk of gemv_tiled_kernel; organs of 512 x 2048 unless stated):
+//   * one step (<= 512 binary columns): nothing to split (2.95 against 3.1-3.35);
+//   * up to 1,024 row tiles the workgroups are what is scarce: about one per
 //     CU, so tpw = tiles / 256 rounded up to a power of two, and as many waves
 //     as the steps and the image (one chunk of 8 columns a thread) employ.
-//     One Q4 2048 x 7168: 15.2 -> 5.0, q8 4096 x 2048: 7.6 -> 3.5, binary:
-//     3.74 -> 3.11, mixed: 4.4 -> 3.2; 20 mixed organs (640 tiles): 5.3 -> 3.9;
-//     40 Q4 organs: 7.3 -> 4.8;
-//   * up to 4,096 tiles Q4 and q8 (long rows) still gain from four slices (80
-//     Q4 organs: 9.7 -> 9.4, with 7168 columns 30.8 -> 24.7), the short kinds
-//     from one wave per tile without slices (mixed 6.05 -> 5.63, binary 5.07 ->
-//     4.88);
-//   * beyond, q8 (160 organs: 29.1 -> 26.0; 320: 60.2 -> 54.4) and mixed
-//     (8.9 -> 8.05) up to the streamed shapes; the others' walk is faster
-//     (binary 320 organs: 9.7 against 10.8; Q4 with 7168 columns 99 against 107).
+//     One Q4 2048 x 7168: 14.2 -> 5.3, q8 4096 x 2048: 7.6 -> 3.7, q8 2048 x
+//     7168: 21.8 -> 5.9, binary 4096 x 2048: 4.1 -> 3.35; 20 mixed organs (640
+//     tiles): 5.35 -> 4.1; 20 Q4 organs: 6.8 -> 4.4.  (Wide rows with 8 waves
+//     instead of 16: 0.3 us more for Q4 2048 x 7168, 0.7 for q8.)
+//   * up to 2,048 tiles one wave per tile, 8 tiles side by side (34 Q4 organs:
+//     6.95 -> 5.1, binary 4.4 -> 3.9, mixed 5.2 -> 4.6; 40 Q4 organs with 7168
+//     columns: 25.4 -> 15.1; steps split over two waves: 6.1 and 17);
+//   * up to 4,096 tiles four waves a tile where the rows have more than 16
+//     steps (80 Q4 organs with 7168 columns: 30.5 -> 26.3; q8 with 4096: 31.2
+//     -> 27.3), the short kinds one wave per tile (mixed 6.05 -> 5.63, binary
+//     5.07 -> 4.88); Q4 of 16 steps walks (80 organs: 9.4 against 9.8);
+//   * beyond, q8 (200 organs: 42.7 -> 36.6) and mixed (8.9 -> 8.05) up to the
+//     streamed shapes; the others' walk is faster (binary 320 organs: 9.7
+//     against 10.8; 200 Q4 organs: 20.1 against 19.9, with 7168 columns equal).
 // HEAD: every workgroup ends in one atomic max on the same word, which the
 // memory side takes at about 12 ns each (a binary 151,936 x 2048 lm_head over
 // 1,900 workgroups: 30 us for 44 MB), so one or two balanced workgroups per
-// CU, 8 waves each: binary 16.8 us (one wave per tile, one workgroup per CU),
-// Q4 40.0 -> 30.4, q8 56.3 -> 55 (four slices, two workgroups per CU above
-// 4,096 tiles); q8 65,000 rows 29.8 -> 25.5, 11,409 rows 13.0 -> 10.8; a q8
-// lm_head larger than the Infinity Cache loads non-temporally with one
-// workgroup per CU (151,936 x 2048: 53.4 -> 51.4, 128,256 x 4096: 96.2 -> 84;
-// below, the hint and the fewer loads in flight cost: 65,000 rows 25.9 -> 34.8;
-// Q4 of these sizes fits and gains nothing from it); tile
-// counts that leave a nearly empty last round cost up to 30 % (q8 151,936 over
-// 32 tiles: 69.7).
+// CU, 8 waves each.  One wave per tile for binary (16.5 us) and for short rows
+// or few tiles (q8 32,000 x 1024 10.9 against 13.3 with four waves a tile; Q4
+// 32,000 x 2048 12.3 against 13.7), four else (q8 151,936 x 2048 49.9 against
+// 52.2, 65,000 rows 26.5 against 29.2; Q4 151,936 x 4096 62.7).  A q8 lm_head
+// larger than the Infinity Cache loads non-temporally with one workgroup per
+// CU (128,256 x 4096: 96.2 -> 84; below, the hint and the fewer loads in flight
+// cost: 65,000 rows 25.9 -> 34.8; Q4 of these sizes fits and gains nothing from
+// it); tile counts that leave a nearly empty last round cost up to 30 %.
 // RES (256 threads, at most 4 tiles a workgroup: a row's records are one
-// thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8 ->
-// 6.7, 512 x 7168: 35.4 -> 8.9; above 4,096 tiles the two launches are faster
-// (160 organs: 11.0 against 11.8).
+// thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8
+// -> 6.6, 512 x 7168: 35.4 -> 8.7; above 4,096 tiles the two launches are
+// faster (160 organs: 11.0 against 11.8).
 static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uint32_t S, uint32_t cols) {
     const uint32_t s2 = pow2_ceil(S);
     if (head) {
-        const uint32_t ks = kind == HK_BIN ? 1u : std::min(4u, s2), ts = 8u / ks;
+        const bool walk = kind == HK_BIN || S <= 8 || (S <= 16 && tiles <= 2048) || (S <= 32 && tiles > 512 && tiles <= 1024);
+        const uint32_t ks = walk ? 1u : 4u, ts = 8u / ks;
         const bool past_mall = kind == HK_Q8 && tiles * 16u * cols > MALL_BYTES;
         const uint32_t wgs = kind == HK_BIN || tiles <= 4096 || past_mall ? 256u : 512u;
         const uint32_t even = (uint32_t)((tiles + wgs - 1u) / wgs);
         return {8, ks, std::min((even + ts - 1u) / ts * ts, 64u)};
     }
-    if (tiles >= 16384) return {0, 0, 0};
-    uint32_t tpw = std::min(pow2_ceil((uint32_t)((tiles + 255) / 256)), 8u);
+    const uint32_t tpw = std::min(pow2_ceil((uint32_t)((tiles + 255) / 256)), 4u);
     if (res) {
         if (tiles > 4096) return {0, 0, 0};
-        tpw = std::min(tpw, 4u);
         const uint32_t ks = std::min(std::max(4u / tpw, 1u), s2);
         return {4, ks, std::max(tpw, 4u / ks)};
     }
-    if (S == 1) return {0, 0, 0};
+    if (S == 1 || tiles >= 16384) return {0, 0, 0};
     const bool wide = kind == HK_Q4 || kind == HK_Q8;
-    if (tiles <= 2048) {
-        const uint32_t w = cols > 4096 ? 16u : S >= 16 ? (tpw >= 4 ? 16u : 8u) : tpw == 1 ? 4u : 8u;
-        const uint32_t ks = std::min(std::max(w / tpw, 1u), s2);
+    if (tiles <= 1024) {
+        const bool w16 = cols > 4096 || (S >= 16 && tpw == 4) || (wide && S >= (tpw == 1 ? 48u : 32u));
+        const uint32_t w = w16 ? 16u : S < 16 && tpw == 1 ? 4u : 8u;
+        const uint32_t ks = std::min(w / tpw, s2);
         return {w, ks, std::max(tpw, w / ks)};
     }
-    if (wide && S >= 16 && (tiles <= 4096 || kind == HK_Q8)) return {8, kind == HK_Q8 ? 8u : 4u, 2};
+    if (tiles <= 2048) return {8, 1, 8};
+    if (wide && S >= 16 && (tiles <= 4096 ? S > 16 : kind == HK_Q8)) return {8, 4, 2};
     if (!wide && (tiles <= 4096 || kind == HK_MIXED)) return {4, 1, 4};
     return {0, 0, 0};
 }
@@ -1209,19 +1261,19 @@ template <int KIND, bool RES, bool HEAD = false>
 static hipError_t launch_split(const OrganView* organs, const ResView* res, const ResView* res_one, uint32_t n,
                                const OrganView& sh, const float* x, size_t xs, float* y, size_t ys, hipStream_t s,
                                bool* done, const HeadArgs& ha = {}, uint32_t* status = nullptr) {
-    constexpr bool ORD = KIND != HK_Q4 && KIND != HK_Q8;
-    constexpr int D = KIND == HK_MIXED ? 2 : 4;
     *done = false;
-    SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
+    const SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
     if (!c.waves) return hipSuccess;
-    const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw;
-    const size_t lds = SplitLds<KIND, ORD, RES>(sh.steps, sh.cols, tpw, ks).total;
+    const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw, ts = waves / ks, per = (sh.steps + ks - 1u) / ks;
+    const uint32_t bufs = ks == 1u ? 0u : tpw == ts && per <= 4u ? 1u : 2u;
+    const size_t lds = SplitLds<KIND, RES>(sh.steps, sh.cols, tpw, waves, per, bufs).total;
     if (lds > SPLIT_LDS_LIMIT) return hipSuccess;
     if (RES && (!organs || !res) && !(n == 1 && res_one)) return hipErrorInvalidValue;
     *done = true;
     SplitArgs a{};
     a.ks_log = (uint32_t)__builtin_ctz(ks);
-    a.ts_log = (uint32_t)__builtin_ctz(waves / ks);
+    a.ts_log = (uint32_t)__builtin_ctz(ts);
+    a.bufs = bufs;
     a.one = sh;
     // one organ's view comes with the arguments where the host has its
     // residual's too (a set of one has that only in its device table)
@@ -1237,11 +1289,12 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     a.tpw = tpw;
     a.ha = ha;
     a.status = status;
-    if (HEAD && KIND == HK_Q8 && (uint64_t)sh.rows * sh.cols > MALL_BYTES)
-        hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES, HEAD, HEAD && KIND == HK_Q8>), dim3(a.parts * n),
-                           dim3(64u * waves), lds, s, a);
-    else
-        hipLaunchKernelGGL((gemv_split_kernel<KIND, D, ORD, RES, HEAD>), dim3(a.parts * n), dim3(64u * waves), lds, s, a);
+    const bool nt = HEAD && KIND == HK_Q8 && (uint64_t)sh.rows * sh.cols > MALL_BYTES;
+    auto* k = ks > 1 ? nt ? gemv_split_kernel<KIND, true, RES, HEAD, HEAD && KIND == HK_Q8>
+                          : gemv_split_kernel<KIND, true, RES, HEAD>
+              : nt   ? gemv_split_kernel<KIND, false, RES, HEAD, HEAD && KIND == HK_Q8>
+                     : gemv_split_kernel<KIND, false, RES, HEAD>;
+    hipLaunchKernelGGL(k, dim3(a.parts * n), dim3(64u * waves), lds, s, a);
     return hipGetLastError();
 }
 

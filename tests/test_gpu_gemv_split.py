@@ -65,27 +65,34 @@ def test_small_launches_within_bound(ctx, oracle, kind, rows, cols):
     assert np.all(got[:, rows:] == 7.0)  # nothing past the organ's rows
     for i in range(n):
         _check_rows(orgs[i], kind, xs[i], got[i], [(0, rows)])
-        assert np.array_equal(got[i, :rows], orgs[i].matvec(xs[i])) or kind in ("q4", "q8")
+        assert np.array_equal(got[i, :rows], orgs[i].matvec(xs[i]))
 
 
-# ragged organs whose row tiles sit on both sides of each change of shape
-TILES = [(k, t) for k in ("q4", "q8", "bin", "mixed", "rice") for t in (256, 257, 513, 1025, 2049, 4097)]
+# ragged organs whose row tiles sit on both sides of each change of shape (the
+# long rows: the shapes of Q4 and q8 organs of more than 16 steps)
+TILES = [(k, t, 1024) for k in ("q4", "q8", "bin", "mixed", "rice") for t in (256, 257, 513, 1025, 2049, 4097)]
+TILES += [("q4", t, 2176) for t in (1024, 1025, 2048, 2049, 4096, 4097)]
+TILES += [(k, t, c) for k, c in (("q8", 1088), ("mixed", 1024)) for t in (4096, 16383, 16384)]
 
 
-@pytest.mark.parametrize("kind,tiles", TILES, ids=[f"{k}-{t}" for k, t in TILES])
-def test_tile_count_edges(ctx, oracle, kind, tiles):
-    rows, cols = 16 * tiles - 3, 1024
-    print("[gpu-case] split gemv tiles", kind, tiles, flush=True)
+@pytest.mark.parametrize("kind,tiles,cols", TILES, ids=[f"{k}-{t}x{c}" for k, t, c in TILES])
+def test_tile_count_edges(ctx, oracle, kind, tiles, cols):
+    rows = 16 * tiles - 3
+    print("[gpu-case] split gemv tiles", kind, tiles, cols, flush=True)
     sys.stdout.flush()
-    o = _organ(ctx, oracle, kind, rows, cols, 0x1000 + TILES.index((kind, tiles)))
+    o = _organ(ctx, oracle, kind, rows, cols, 0x1000 + TILES.index((kind, tiles, cols)))
     x = np.random.default_rng(tiles).standard_normal(cols).astype(np.float32)
     _check_rows(o, kind, x, o.matvec(x), [(0, 48), (rows // 2, 64), (rows - 48, 48)])
 
 
-@pytest.mark.parametrize("kind,rows,cols", [("bin", 64, 1536), ("mixed", 64, 1152), ("u3", 64, 800)])
+STREAMED = [("bin", 64, 1536), ("mixed", 64, 1152), ("u3", 64, 800), ("q4", 64, 2048), ("q4", 64, 5248), ("q8", 64, 1088),
+            ("q8", 64, 4160)]
+
+
+@pytest.mark.parametrize("kind,rows,cols", STREAMED, ids=[f"{k}-{r}x{c}" for k, r, c in STREAMED])
 def test_split_sums_are_the_streamed_sums(ctx, oracle, kind, rows, cols):
-    """Kinds whose terms keep their step order: an organ alone and in a set of
-    the streamed launch shapes (16,384 row tiles) gives the same bits."""
+    """An organ alone and in a set of the streamed launch shapes (16,384 row
+    tiles) gives the same bits: its terms keep their step order."""
     from hawking_amd.organs import OrganSet
     n = 16384 // (rows // 16)
     print("[gpu-case] split = streamed", kind, rows, cols, flush=True)
@@ -98,6 +105,29 @@ def test_split_sums_are_the_streamed_sums(ctx, oracle, kind, rows, cols):
     got = y.download()
     for i in (0, 5, n // 2 + 3, n - 1):
         assert np.array_equal(got[i], base[i % 8].matvec(xs[i])), i
+
+
+SETS = [(k, c) for k in KIND for c in (1024, 4224)]
+
+
+@pytest.mark.parametrize("kind,cols", SETS, ids=[f"{k}-{c}" for k, c in SETS])
+def test_bits_do_not_depend_on_the_set(ctx, oracle, kind, cols):
+    """An organ's result is the same bits in sets on both sides of every change
+    of the launch shape (32 row tiles an organ: 160 to 6,400 tiles)."""
+    from hawking_amd.organs import OrganSet
+    print("[gpu-case] split gemv, sets", kind, cols, flush=True)
+    sys.stdout.flush()
+    base = [_organ(ctx, oracle, kind, 509, cols, 0x4000 + i) for i in range(3)]
+    xs = np.random.default_rng(cols).standard_normal((200, cols)).astype(np.float32)
+    x = ctx.to_device(xs)
+    alone = {i: base[i % 3].matvec(xs[i]) for i in (0, 1, 4, 9, 19, 32, 63, 99, 199)}
+    for n in (2, 5, 10, 20, 33, 64, 100, 200):
+        y = ctx.to_device(np.full((n, 512), 7.0, np.float32))
+        OrganSet(ctx, [base[i % 3] for i in range(n)]).gemv(x, cols, y, 512)
+        got = y.download()
+        assert np.all(got[:, 509:] == 7.0)
+        for i in alone:
+            assert i >= n or np.array_equal(got[i, :509], alone[i]), (n, i)
 
 
 ONE = [(k, 300, 1024) for k in KIND] + [("rice", 8, 128), ("rice", 65536, 128), ("bin", 40, 512)]

@@ -45,6 +45,8 @@ def test_head_kinds(ctx, oracle, kind, vocab, hidden, cut):
         tok = head.greedy(h)
         logits, xn = head.logits.download(), head.xn.download()
         assert tok == oracle.argmax_greedy(logits, vocab - cut)
+    # the logits are the lm_head's own GEMV of xn, to the bit
+    assert np.array_equal(logits, lm.matvec(xn))
     # each xn to a few roundings, the logits to the engine's bound on it
     assert np.all(np.abs(xn - oracle.rmsnorm_1p(h, nw, 1e-6)) <= 2e-6 * np.abs(xn) + 1e-30)
     w, x64 = lm.decode(0, min(vocab, 300)).astype(np.float64), xn.astype(np.float64)
