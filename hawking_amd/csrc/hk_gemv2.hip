@@ -773,8 +773,14 @@ hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint3
     // 6.2 -> 4.8, 256 pairs 6.6 -> 5.6, 512 pairs 7.5 against 7.8; r384 4096 x
     // 2048, 1 pair 53 -> 15.
     const uint32_t few = l.n_tiles >= 64u ? 512u : 256u;
-    const uint32_t parts = n > few ? 0u
-                                   : std::min(std::max(256u / n, 1u), (l.n_tiles + LOWRANK_WAVES - 1u) / LOWRANK_WAVES);
+    // (overlapping buffers: one workgroup a pair, which has read what it
+    // overwrites)
+    const bool shared = vectors_overlap(x, x_stride, r.cols, y, y_stride, l.rows, n) ||
+                        vectors_overlap(x, x_stride, r.cols, mid, mid_stride, r.rows, n) ||
+                        vectors_overlap(mid, mid_stride, r.rows, y, y_stride, l.rows, n);
+    const uint32_t parts = n > few || shared
+                               ? 0u
+                               : std::min(std::max(256u / n, 1u), (l.n_tiles + LOWRANK_WAVES - 1u) / LOWRANK_WAVES);
     if (parts) {
         LowrankArgs a{};
         a.tpw = (l.n_tiles + parts - 1u) / parts;
@@ -1263,7 +1269,7 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
                                bool* done, const HeadArgs& ha = {}, uint32_t* status = nullptr) {
     *done = false;
     const SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
-    if (!c.waves) return hipSuccess;
+    if (!c.waves || (!HEAD && vectors_overlap(x, xs, sh.cols, y, ys, sh.rows, n))) return hipSuccess;
     const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw, ts = waves / ks, per = (sh.steps + ks - 1u) / ks;
     const uint32_t bufs = ks == 1u ? 0u : tpw == ts && per <= 4u ? 1u : 2u;
     const size_t lds = SplitLds<KIND, RES>(sh.steps, sh.cols, tpw, waves, per, bufs).total;
@@ -1313,7 +1319,8 @@ static hipError_t launch_r(const OrganView* organs, uint32_t n, const OrganView&
         } else if constexpr (KIND == HK_U3) {
             // narrow factors: up to 128 tiles share an image, as long as 1,024
             // workgroups remain
-            const uint32_t share = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tiles / 1024u, 16u), 128u) & ~7u;
+            const bool one = vectors_overlap(x, xs, sh.cols, y, ys, sh.rows, n);  // (one workgroup an organ)
+            const uint32_t share = one ? 128u : (uint32_t)std::min<uint64_t>(std::max<uint64_t>(tiles / 1024u, 16u), 128u) & ~7u;
             return launch_kind<KIND, 2, 3>(organs, n, sh, x, xs, y, ys, gemv_max_tiles(KIND, sh.steps) == 128u ? share : 16, s);
         } else if constexpr (KIND == HK_Q4 || KIND == HK_Q8) {
             return launch_kind<KIND, HK_Q_R, HK_Q_D>(organs, n, sh, x, xs, y, ys, HK_Q_TPW, s);

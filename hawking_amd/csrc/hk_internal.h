@@ -303,6 +303,17 @@ int check_hip(hk_ctx* ctx, hipError_t e, const char* what);
 size_t gemv_lds_bytes(int kind, uint32_t cols);
 constexpr size_t GEMV_LDS_LIMIT = 64 * 1024;
 struct ResView;
+// Whether vectors a_i (na floats at a + i a_stride) and b_i of the same i < n
+// share memory.  A launch that gives one organ several workgroups reads x in
+// some after others have written y, so such calls keep one workgroup an organ
+// where they had it.
+inline bool vectors_overlap(const float* a, size_t a_stride, uint32_t na, const float* b, size_t b_stride, uint32_t nb,
+                            uint32_t n) {
+    if (!a || !b || a + (n - 1u) * a_stride + na <= b || b + (n - 1u) * b_stride + nb <= a) return false;
+    for (uint32_t i = 0; i < (a_stride == b_stride ? 1u : n); ++i)
+        if (a + i * a_stride < b + i * b_stride + nb && b + i * b_stride < a + i * a_stride + na) return true;
+    return false;
+}
 // The binary GEMV of HGRAVR02 organs with the residual added in the same
 // launch (the bits of launch_gemv_tiled then launch_rice_apply); res_one: a
 // host copy of the residual's view where n = 1 and the caller has one, else

@@ -187,7 +187,10 @@ int hk_organ_info(const hk_organ* organ, int32_t* kind, int32_t* group, uint32_t
  * Replaces BackendGemv::gemv (backend/mod.rs:270-291) for the packed kinds and
  * the Q4/binary matvec kernels (shaders/qwen_uniform_q4.metal:183-272,
  * shaders/q80_mixed_decode.metal:701-741).  Numerics: within 2e-5 relative L2
- * of Qwen80Q4PackedTensor::matvec / binary_group_matvec_f32. */
+ * of Qwen80Q4PackedTensor::matvec / binary_group_matvec_f32; an organ's result
+ * is the same bits alone, in a set of any size and as an lm_head.  x and y
+ * must not overlap (here and in the set forms): workgroups read x while others
+ * write y. */
 int hk_gemv(hk_ctx* ctx, const hk_organ* organ, const float* x, float* y, hk_stream stream);
 
 /* SYNCHRONOUS helper: n organs of one kind and shape in ONE launch,
@@ -212,7 +215,9 @@ int hk_gemv_set(hk_ctx* ctx, const hk_organ_set* set, const float* x, size_t x_s
 /* HGRAVS01 low-rank organ: mid[rank] = right x, then y[rows] = left mid (mid
  * is a caller buffer of rank floats, 16-byte aligned, and receives R x).  The
  * factors are HK_U3 organs (left rows x rank, right rank x cols); one launch
- * when cols <= 8192 and rank <= 2048, else two ordered on `stream`.
+ * when cols <= 8192 and rank <= 2048, else two ordered on `stream`.  In one
+ * launch y and mid may overlap x, and mid may lie in y (which then holds the
+ * result): such calls run one workgroup a pair.
  * Replaces hgravs01_two_stage_matvec_f32 (q80_mixed_decode.rs:614-629). */
 int hk_gemv_lowrank(hk_ctx* ctx, const hk_organ* left, const hk_organ* right, const float* x,
                     float* mid, float* y, hk_stream stream);
@@ -223,7 +228,8 @@ int hk_gemv_lowrank(hk_ctx* ctx, const hk_organ* left, const hk_organ* right, co
  * mid.  mid (device, mid_i = mid + i*mid_stride, 16-byte aligned) may be
  * NULL when the pair is fused; when given it receives R_i x_i; the two-launch
  * shapes (right cols > 8192 or rank > 2048) require it (HK_E_INVALID_ARG).
- * Strides as hk_gemv_batch.  The set form of hgravs01_two_stage_matvec_f32
+ * Strides as hk_gemv_batch; a pair's own vectors may overlap as in
+ * hk_gemv_lowrank, those of two pairs must not.  The set form of hgravs01_two_stage_matvec_f32
  * (q80_mixed_decode.rs:614-629) over a routed wave's down projections. */
 int hk_gemv_lowrank_set(hk_ctx* ctx, const hk_organ_set* left, const hk_organ_set* right, const float* x,
                         size_t x_stride, float* mid, size_t mid_stride, float* y, size_t y_stride,

@@ -51,3 +51,48 @@ def test_few_pairs_match_two_launches(ctx, oracle, rows, rank, cols, n):
         w = lefts[i % m].decode().astype(np.float64) @ (rights[i % m].decode().astype(np.float64) @
                                                         xs[i].astype(np.float64))
         assert oracle.relative_l2(a[i, :rows], w) < 2e-5
+
+
+OVERLAPS = [(2048, 160, 768, 1), (300, 64, 1024, 3), (64, 2016, 160, 2)]
+
+
+@pytest.mark.parametrize("rows,rank,cols,n", OVERLAPS)
+def test_few_pairs_in_place(ctx, oracle, rows, rank, cols, n):
+    """A pair's y or mid over its x, and mid inside y: the bits of separate
+    buffers (a pair in one workgroup has read what it overwrites)."""
+    from hawking_amd.organs import HgravS01LowRank, OrganSet, SyntheticOrgan, gemv_lowrank_set
+    print("[gpu-case] lowrank in place", rows, rank, cols, n, flush=True)
+    sys.stdout.flush()
+    key = lambda k: oracle.stream_key(U.SEED, (0x10F << 40) + rows * 16 + k)
+    lefts = [SyntheticOrgan(ctx, 5, rows, rank, key(2 * i), 0, group=64, sigma=0.05) for i in range(n)]
+    rights = [SyntheticOrgan(ctx, 5, rank, cols, key(2 * i + 1), 0, group=64) for i in range(n)]
+    ls, rs = OrganSet(ctx, lefts), OrganSet(ctx, rights)
+    xs = np.random.default_rng(rows).standard_normal((n, cols)).astype(np.float32)
+    y, st = ctx.empty((n, rows)), 4096
+
+    def call(x, x_stride, mid, mid_stride, out, out_stride):
+        ctx.call("hk_gemv_lowrank_set", ls.h, rs.h, x, x_stride, mid, mid_stride, out, out_stride, ctx.stream)
+
+    gemv_lowrank_set(ctx, ls, rs, ctx.to_device(xs), cols, y, rows)
+    want = y.download()
+    rec = np.zeros((n, st), np.float32)
+    rec[:, :cols] = xs
+    for at in (0, 4, cols // 8 * 4):  # y, then mid, from x's start and from inside it
+        b = ctx.to_device(rec)
+        call(b.ptr, st, None, 0, b.offset(at), st)
+        assert np.array_equal(b.download()[:, at:at + rows], want), ("y over x", at)
+        b = ctx.to_device(rec)
+        call(b.ptr, st, b.offset(at), st, y.ptr, rows)
+        assert np.array_equal(y.download(), want), ("mid over x", at)
+    if rank <= rows:
+        x = ctx.to_device(xs)
+        call(x.ptr, cols, y.ptr, rows, y.ptr, rows)
+        assert np.array_equal(y.download(), want), "mid in y"
+    # x and y side by side in a record do not overlap
+    b = ctx.to_device(rec)
+    call(b.ptr, st, None, 0, b.offset(cols), st)
+    assert np.array_equal(b.download()[:, cols:cols + rows], want)
+    if rows <= cols:
+        x = ctx.to_device(xs[0])
+        HgravS01LowRank(lefts[0], rights[0]).matvec_device(x, x)
+        assert np.array_equal(x.download()[:rows], want[0])
