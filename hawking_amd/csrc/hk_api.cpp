@@ -1248,8 +1248,13 @@ extern "C" int hk_synth_normal(hk_ctx* ctx, uint64_t key, uint64_t first, size_t
 static int head_greedy(hk_ctx* ctx, const float* hidden, const float* norm_w, float eps, const hk_organ* lm_head,
                        uint32_t n_valid, float* xn, float* logits, uint64_t* pick, int32_t* token, hipStream_t st) {
     // (a residual is not part of the fused GEMV, and kinds other than q8 keep
-    // hk_gemv's alignment rule for the logits)
-    if (head_gemv_fusable(lm_head->view) && !lm_head->res_dev && aligned16(norm_w) && aligned16(xn) &&
+    // hk_gemv's alignment rule for the logits; the fused GEMV's workgroups read
+    // hidden and the norm weight while others write xn and the logits)
+    const uint32_t rows = lm_head->view.rows, cols = lm_head->view.cols;
+    const bool shared = vectors_overlap(hidden, 0, cols, xn, 0, cols, 1) || vectors_overlap(norm_w, 0, cols, xn, 0, cols, 1) ||
+                        vectors_overlap(hidden, 0, cols, logits, 0, rows, 1) ||
+                        vectors_overlap(norm_w, 0, cols, logits, 0, rows, 1);
+    if (head_gemv_fusable(lm_head->view) && !lm_head->res_dev && !shared && aligned16(norm_w) && aligned16(xn) &&
         (lm_head->view.kind == HK_Q8 || aligned16(logits)))
         return check_hip(ctx,
                          launch_head_fused(lm_head->view, hidden, norm_w, eps, xn, logits, n_valid, pick, token, ctx->dev_status, st),

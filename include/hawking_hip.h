@@ -386,7 +386,9 @@ int hk_catalog_load(hk_ctx* ctx, hk_catalog* catalog, const char* name, int veri
  * logits [lm_head rows] are caller workspaces (16-byte aligned), pick a
  * 16-byte caller workspace (8-byte aligned) the greedy key reduces into,
  * which must hold zeros before its first use and which every call leaves
- * zeroed, token one int32.  A non-finite xn or a best logit that is not
+ * zeroed, token one int32.  xn may be hidden itself and logits may overlap
+ * hidden or norm_w (such calls form xn in a launch of its own); xn and logits
+ * must not overlap each other.  A non-finite xn or a best logit that is not
  * finite writes token -1 and latches HK_E_NONFINITE in the device status
  * (hk_check_device_status), where the reference returns an error.
  * Stream-ordered, no host round trip; the lm_head organ is only read, so

@@ -71,3 +71,31 @@ def test_head_kinds_flag_nonfinite(ctx, oracle, kind):
             head.greedy(bad)
         assert int(head.token.download()[0]) == -1
     assert head.greedy(h) == oracle.argmax_greedy(head.logits.download())
+
+
+@pytest.mark.parametrize("kind", sorted(KIND))
+def test_head_in_place(ctx, oracle, kind):
+    """xn over hidden and the logits over hidden: hidden has been read when
+    either is written."""
+    from hawking_amd.head import TerminalHead
+    print("[gpu-case] head in place", kind, flush=True)
+    sys.stdout.flush()
+    lm = _organ(ctx, oracle, kind, 70000, 2048)
+    rng = np.random.default_rng(11)
+    h, nw = rng.standard_normal(2048).astype(np.float32), (rng.standard_normal(2048) * 0.02).astype(np.float32)
+    head = TerminalHead(ctx, nw, lm)
+    want = head.greedy(h)
+    want_xn = head.xn.download()
+    for case in ("xn", "logits"):
+        head = TerminalHead(ctx, nw, lm)
+        if case == "xn":
+            head.xn.upload(h)
+            head.greedy_device(head.xn)
+        else:
+            head.logits.upload(np.concatenate([h, np.zeros(70000 - 2048, np.float32)]))
+            head.greedy_device(head.logits)
+        assert ctx.device_status() == 0
+        xn, logits = head.xn.download(), head.logits.download()
+        assert np.all(np.abs(xn - want_xn) <= 2e-6 * np.abs(want_xn)), case
+        assert np.array_equal(logits, lm.matvec(xn)), case
+        assert int(head.token.download()[0]) == oracle.argmax_greedy(logits) == want, case
