@@ -1254,7 +1254,7 @@ static int head_greedy(hk_ctx* ctx, const float* hidden, const float* norm_w, fl
     const bool shared = vectors_overlap(hidden, 0, cols, xn, 0, cols, 1) || vectors_overlap(norm_w, 0, cols, xn, 0, cols, 1) ||
                         vectors_overlap(hidden, 0, cols, logits, 0, rows, 1) ||
                         vectors_overlap(norm_w, 0, cols, logits, 0, rows, 1);
-    if (head_gemv_fusable(lm_head->view) && !lm_head->res_dev && !shared && aligned16(norm_w) && aligned16(xn) &&
+    if (head_gemv_fusable(lm_head->view) && !lm_head->res_dev && !shared && aligned16(xn) &&
         (lm_head->view.kind == HK_Q8 || aligned16(logits)))
         return check_hip(ctx,
                          launch_head_fused(lm_head->view, hidden, norm_w, eps, xn, logits, n_valid, pick, token, ctx->dev_status, st),

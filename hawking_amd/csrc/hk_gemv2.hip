@@ -97,6 +97,7 @@ __host__ __device__ constexpr size_t gemv_hdr_offset(uint32_t steps) {
 // sets the low word of key[1].
 struct HeadArgs {
     const float* norm_w;
+    bool norm_w4;  // 16-byte aligned
     float eps;
     float* xn;
     uint32_t n_valid;
@@ -134,6 +135,20 @@ __device__ __forceinline__ float block_sum_f(float v, float* red) {
     for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) t += red[w];
     __syncthreads();
     return t;
+}
+
+// load_x of a norm weight that is only 4-byte aligned (it has no alignment
+// rule; the same kernel takes it, so xn and the logits are the same bits).
+template <int NC>
+__device__ __forceinline__ void load_norm_w(const float* w, uint32_t cols, XChunks<NC>& gw) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const uint32_t c0 = 8u * (threadIdx.x + blockDim.x * (uint32_t)j);
+        const float* p = w + min(c0, cols - 8u);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            gw.v[j][k] = make_float4(p[4 * k], p[4 * k + 1], p[4 * k + 2], p[4 * k + 3]);
+    }
 }
 
 // xn = h * (1 / sqrt(mean(h^2) + eps)) * (1 + w) on this thread's register
@@ -958,7 +973,10 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     XChunks<NC> xc;
     load_x<NC>(BlockTeam{}, x, o.cols, xc);
     XChunks<HEAD ? NC : 1> gw;
-    if constexpr (HEAD) load_x<NC>(BlockTeam{}, a.ha.norm_w, o.cols, gw);
+    if constexpr (HEAD) {
+        if (a.ha.norm_w4) load_x<NC>(BlockTeam{}, a.ha.norm_w, o.cols, gw);
+        else load_norm_w<NC>(a.ha.norm_w, o.cols, gw);
+    }
     RiceTile rt;
     const uint32_t r0 = t0 * 16u, r1 = min(t1 * 16u, o.rows);
     if constexpr (RES) rice_ranges(rv, r0, r1, rt);
@@ -1369,7 +1387,7 @@ hipError_t launch_head_fused(const OrganView& sh, const float* h, const float* n
                              float eps, float* xn, float* logits, uint32_t n_valid, uint64_t* key, int32_t* token,
                              uint32_t* status, hipStream_t s) {
     if (!head_gemv_fusable(sh)) return hipErrorInvalidValue;
-    const HeadArgs ha{norm_w, eps, xn, n_valid, key};
+    const HeadArgs ha{norm_w, (reinterpret_cast<uintptr_t>(norm_w) & 15u) == 0, eps, xn, n_valid, key};
     const hipError_t e = sh.kind == HK_Q8   ? launch_head_gemv<HK_Q8>(sh, h, logits, ha, status, s)
                          : sh.kind == HK_Q4 ? launch_head_gemv<HK_Q4>(sh, h, logits, ha, status, s)
                                             : launch_head_gemv<HK_BIN>(sh, h, logits, ha, status, s);

@@ -414,7 +414,7 @@ hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint3
 // The fused form for a q8, Q4 or binary lm_head (without a residual) of at
 // most 8192 columns: the GEMV forms the
 // norm itself and reduces the greedy key (key: 16 zeroed bytes, left zeroed),
-// then one pick; h, norm_w and xn 16-byte aligned.
+// then one pick; h and xn 16-byte aligned.
 bool head_gemv_fusable(const OrganView& sh);
 hipError_t launch_head_fused(const OrganView& sh, const float* h, const float* norm_w,
                              float eps, float* xn, float* logits, uint32_t n_valid, uint64_t* key, int32_t* token,

@@ -99,3 +99,23 @@ def test_head_in_place(ctx, oracle, kind):
         assert np.all(np.abs(xn - want_xn) <= 2e-6 * np.abs(want_xn)), case
         assert np.array_equal(logits, lm.matvec(xn)), case
         assert int(head.token.download()[0]) == oracle.argmax_greedy(logits) == want, case
+
+
+@pytest.mark.parametrize("kind,hidden", [(k, h) for k in sorted(KIND) for h in (640, 8192)])
+def test_head_norm_weight_alignment(ctx, oracle, kind, hidden):
+    """The norm weight at any 4-byte address gives the same bits."""
+    from hawking_amd.head import TerminalHead
+    print("[gpu-case] head norm weight alignment", kind, hidden, flush=True)
+    sys.stdout.flush()
+    rng = np.random.default_rng(hidden)
+    h, nw = rng.standard_normal(hidden).astype(np.float32), (rng.standard_normal(hidden) * 0.02).astype(np.float32)
+    head = TerminalHead(ctx, nw, _organ(ctx, oracle, kind, 300, hidden))
+    want = head.greedy(h)
+    xn, logits = head.xn.download(), head.logits.download()
+    hd = ctx.to_device(h)
+    for shift in (1, 2, 3):
+        w = ctx.to_device(np.concatenate([np.full(shift, 9.0, np.float32), nw, np.full(4, 9.0, np.float32)]))
+        ctx.call("hk_terminal_greedy", hd.ptr, w.offset(shift), head.eps, head.lm_head.h, 300, head.xn.ptr,
+                 head.logits.ptr, head.pick.ptr, head.token.ptr, ctx.stream)
+        assert ctx.device_status() == 0 and int(head.token.download()[0]) == want, shift
+        assert np.array_equal(head.xn.download(), xn) and np.array_equal(head.logits.download(), logits), shift
