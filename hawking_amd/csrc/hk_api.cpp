@@ -616,7 +616,7 @@ extern "C" int hk_gemv_lowrank(hk_ctx* ctx, const hk_organ* left, const hk_organ
         return check_hip(ctx,
                          launch_lowrank(static_cast<const OrganView*>(left->view_dev),
                                         static_cast<const OrganView*>(right->view_dev), 1, left->view, right->view, x, 0,
-                                        mid, 0, y, 0, nullptr, static_cast<hipStream_t>(stream)),
+                                        mid, 0, y, 0, static_cast<hipStream_t>(stream)),
                          "low-rank launch");
     // stream order carries mid from the first launch to the second
     rc = hk_gemv(ctx, right, x, mid, stream);
@@ -748,7 +748,7 @@ extern "C" int hk_gemv_lowrank_set(hk_ctx* ctx, const hk_organ_set* left, const 
     if (fused)
         return check_hip(ctx,
                          launch_lowrank(left->dev, right->dev, left->n, left->first, right->first, x, x_stride, mid,
-                                        mid_stride, y, y_stride, nullptr, st),
+                                        mid_stride, y, y_stride, st),
                          "low-rank set launch");
     // other shapes: two launches ordered on the stream through the caller's mid
     rc = hk_gemv_set(ctx, right, x, x_stride, mid, mid_stride, stream);

@@ -526,7 +526,7 @@ template <int NC>
 __global__ void __launch_bounds__(256, HK_LR_MINW)
 lowrank_kernel(const OrganView* __restrict__ lefts, const OrganView* __restrict__ rights, uint32_t n,
                const float* __restrict__ xall, size_t x_stride, float* __restrict__ mid_all, size_t mid_stride,
-               float* __restrict__ yall, size_t y_stride, uint32_t* status) {
+               float* __restrict__ yall, size_t y_stride) {
     extern __shared__ __align__(16) uint8_t lds[];
     uint32_t oi, part;
     organ_part(blockIdx.x, 1, n, &oi, &part);
@@ -546,7 +546,6 @@ lowrank_kernel(const OrganView* __restrict__ lefts, const OrganView* __restrict_
     TileWalk<HK_U3, HK_LR_LR, HK_LR_LD> wl;
     // both x images with E = 0, scattered from each thread's chunks (the
     // two launches' images to the bit: the GEMV builds them the same way)
-    bool bad = false;
     {
         uint8_t* img = lds + M.img_r;
         float* sx = reinterpret_cast<float*>(img + (size_t)rv.steps * Kcfg<HK_U3>::P * A_TILE_STRIDE);
@@ -555,12 +554,12 @@ lowrank_kernel(const OrganView* __restrict__ lefts, const OrganView* __restrict_
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
             const uint32_t ch = threadIdx.x + 256u * (uint32_t)j;
-            if (ch < nch) bad |= image_chunk<HK_U3>(ch, xc.v[j], img, sx, 0u, 0u);
+            if (ch < nch) (void)image_chunk<HK_U3>(ch, xc.v[j], img, sx, 0u, 0u);
         }
         for (uint32_t ch = threadIdx.x + 256u * NC; ch < nch; ch += 256u) {
             float4 v[2];
             load_chunk(x, 8u * ch, rv.cols, v);
-            bad |= image_chunk<HK_U3>(ch, v, img, sx, 0u, 0u);
+            (void)image_chunk<HK_U3>(ch, v, img, sx, 0u, 0u);
         }
         __syncthreads();
     }
@@ -577,14 +576,13 @@ lowrank_kernel(const OrganView* __restrict__ lefts, const OrganView* __restrict_
         for (uint32_t ch = threadIdx.x; ch < nch; ch += 256u) {
             float4 v[2];
             load_chunk(mid, 8u * ch, rv.rows, v);
-            bad |= image_chunk<HK_U3>(ch, v, img, sx, 0u, 0u);
+            (void)image_chunk<HK_U3>(ch, v, img, sx, 0u, 0u);
         }
         __syncthreads();
     }
     wl.run(lv, 0, lds + M.img_l, lane, ysh);
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < lv.rows; i += blockDim.x) y[i] = ysh[i];
-    if (bad && status) atomicOr(status, 1u);
 }
 
 // The same pairs when there are too few of them for one workgroup each to
@@ -779,7 +777,7 @@ bool lowrank_fusable(const OrganView& l, const OrganView& r) {
 
 hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint32_t n, const OrganView& l,
                           const OrganView& r, const float* x, size_t x_stride, float* mid, size_t mid_stride, float* y,
-                          size_t y_stride, uint32_t* status, hipStream_t s) {
+                          size_t y_stride, hipStream_t s) {
     if (!lowrank_fusable(l, r)) return hipErrorInvalidValue;
     // One workgroup per CU over all pairs, at least 16 left tiles each (us in a
     // graph of one launch, against one 4-wave workgroup per pair): r160 2048 x
@@ -821,10 +819,10 @@ hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint3
     const size_t lds = lowrank_lds(l, r).total;
     if (x_image_cols<HK_U3>(r.steps) <= 2048u)
         hipLaunchKernelGGL(lowrank_kernel<1>, dim3(n), dim3(256), lds, s, lefts, rights, n, x, x_stride, mid,
-                           mid_stride, y, y_stride, status);
+                           mid_stride, y, y_stride);
     else
         hipLaunchKernelGGL(lowrank_kernel<4>, dim3(n), dim3(256), lds, s, lefts, rights, n, x, x_stride, mid,
-                           mid_stride, y, y_stride, status);
+                           mid_stride, y, y_stride);
     return hipGetLastError();
 }
 

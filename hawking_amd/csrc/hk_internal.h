@@ -410,7 +410,7 @@ hipError_t launch_head_argmax(const float* logits, uint32_t n_valid, uint64_t* k
 bool lowrank_fusable(const OrganView& l, const OrganView& r);
 hipError_t launch_lowrank(const OrganView* lefts, const OrganView* rights, uint32_t n, const OrganView& l,
                           const OrganView& r, const float* x, size_t x_stride, float* mid, size_t mid_stride, float* y,
-                          size_t y_stride, uint32_t* status, hipStream_t s);
+                          size_t y_stride, hipStream_t s);
 // The fused form for a q8, Q4 or binary lm_head (without a residual) of at
 // most 8192 columns: the GEMV forms the
 // norm itself and reduces the greedy key (key: 16 zeroed bytes, left zeroed),
