@@ -1,11 +1,13 @@
-"""GEMV over organ sets in every launch shape the dispatcher picks, and x
+"""GEMV over organ sets in the launch shapes the dispatcher picks, and x
 images of several quantization rounds, against the oracle (through the C ABI).
 
 The dispatcher sizes the launch by the set's total row tiles: >= 16384 tiles
 (the streamed shapes of the benchmark, as tiles per wave group / steps in
-flight / tiles per workgroup: binary 4 / 3 / 16 with >= 4 steps, else
-2 / 3 / 32; Q4 2 / 3 / 16; mixed 1 / 3 / 16), >= 4096 (2 / 2 / 8) and below
-(1 / 2 / 4 or 1).  The x image is built 2048 columns per
+flight / tiles per workgroup: binary 2 / 5 / 16 with >= 4 steps, else
+2 / 5 / 32; Q4 and q8 2 / 3 / 32; mixed 1 / 3 / 16) and below, where the row
+tiles' steps are split over a workgroup's waves or walked (2 / 2 / 8 from 4096
+tiles on); the edges of the split shapes' rule are in test_gpu_gemv_split.py.
+The x image is built 2048 columns per
 round; organs wider than 2048 columns take several rounds, and beyond 8192
 columns the later rounds re-read x.  Organs are generated on the device; the
 oracle regenerates the ones it checks (first, middle, last) bit-identically.

@@ -1,7 +1,8 @@
 """Few HGRAVS01 pairs (several workgroups per pair): the same bits as the
 right factor's and then the left factor's GEMV through a mid buffer, at
-ragged rows, ranks of one to many rounds of right tiles, and pair counts on
-both sides of the rule."""
+ragged rows, ranks of one to many rounds of right tiles, inputs on both sides
+of the widest that fit its LDS (3,072 and 4,096 columns at rank 288), and pair
+counts on both sides of the rule."""
 from __future__ import annotations
 
 import sys
@@ -12,7 +13,8 @@ import pytest
 from tests import hk_testutil as U
 
 pytestmark = pytest.mark.gpu
-SHAPES = [(1, 32, 32, 1), (17, 32, 1024, 1), (2048, 160, 768, 1), (1000, 384, 2048, 2), (300, 288, 4096, 3),
+SHAPES = [(1, 32, 32, 1), (17, 32, 1024, 1), (2048, 160, 768, 1), (1000, 384, 2048, 2), (300, 288, 3072, 3),
+          (300, 288, 4096, 3),
           (4100, 64, 96, 2), (64, 2016, 160, 2), (40, 96, 256, 256), (40, 96, 256, 257), (1040, 32, 64, 512),
           (1040, 32, 64, 513)]
 

@@ -64,3 +64,40 @@ def test_packers_bit_exact_at_group_edges(ctx, oracle, groups, shift):
         s, c = run("hk_pack_u3", w[:count].copy(), g3, g3 * 24, C.c_size_t(count))
         rs, rc = oracle.uniform_pack(w[:count], 1, count, 3, 64)
         assert np.array_equal(s, rs) and np.array_equal(c, rc), ("hk_pack_u3", count)
+
+
+PACKERS = [("hk_pack_q4", 32, 16), ("hk_pack_bin", 128, 16), ("hk_pack_q8", 64, 64), ("hk_pack_q2", 64, 16),
+           ("hk_pack_u3", 64, 24)]
+
+
+@pytest.mark.parametrize("fn,group,per", PACKERS)
+def test_packers_flag_nonfinite_and_clear(ctx, oracle, fn, group, per):
+    """A NaN or infinity anywhere (first, last and inside), and a scale past
+    f16 where the format refuses one, is HK_E_NONFINITE; the next call on the
+    same context is clean and packs the same bytes."""
+    from hawking_amd._lib import HK_E_NONFINITE, HawkingError
+    print("[gpu-case] packers non-finite", fn, flush=True)
+    sys.stdout.flush()
+    rows, cols = 33, 384
+    n = rows * cols
+    shape = {"hk_pack_q4": (rows, cols, group), "hk_pack_q2": (C.c_size_t(n),),
+             "hk_pack_u3": (C.c_size_t(n),)}.get(fn, (rows, cols))
+    w = (np.random.default_rng(5).standard_normal(n) * 0.02).astype(np.float32)
+    s, c = ctx.empty(n // group, np.uint16), ctx.empty(n // group * per, np.uint8)
+
+    def pack(v):
+        ctx.call(fn, ctx.to_device(v).ptr, *shape, s.ptr, c.ptr, ctx.stream)
+        return s.download(), c.download()
+
+    want = pack(w)
+    bad = [(i, v) for i in (0, 777, n - 1) for v in (np.nan, np.inf, -np.inf)]
+    if fn not in ("hk_pack_bin", "hk_pack_q2"):  # (those two store an infinite scale)
+        bad.append((n // 2, np.float32(3e38)))
+    for i, v in bad:
+        b = w.copy()
+        b[i] = v
+        with pytest.raises(HawkingError) as e:
+            pack(b)
+        assert e.value.code == HK_E_NONFINITE, (i, v)
+        got = pack(w)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), (i, v)
