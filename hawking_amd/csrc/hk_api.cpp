@@ -1225,8 +1225,9 @@ extern "C" int hk_pack_mixed(hk_ctx* ctx, const float* w, uint32_t rows, uint32_
     rc = check_hip(ctx, hipMemcpyAsync(tmp, &j, sizeof(j), hipMemcpyHostToDevice, st), "mixed job upload");
     if (!rc) rc = check_hip(ctx, launch_mixed_pack_buffer(static_cast<SynthJob*>(tmp), groups, bad, st), "pack launch");
     if (!rc) rc = check_hip(ctx, hipMemcpyAsync(&bad_host, bad, 4, hipMemcpyDeviceToHost, st), "pack status read");
-    (void)hipStreamSynchronize(st);
+    const int drained = check_hip(ctx, hipStreamSynchronize(st), "hipStreamSynchronize (pack)");
     (void)hipFree(tmp);
+    if (!rc) rc = drained;
     return rc ? rc : pack_verdict(ctx, bad_host);
 }
 
