@@ -56,16 +56,55 @@ struct ItemStride {
     }
 };
 
+// How a lane's terms of a row are summed, in every launch shape alike: in step
+// order, and for Q4 and q8 (16 to 128 steps a row) in blocks of four steps,
+// the blocks' sums added up four at a time and those in order.  The shorter
+// chains round less (relative error against 64 bits at 2048 x 7168, one chain
+// -> blocks: Q4 2.1e-7 -> 1.75e-7, q8 2.3e-7 -> 1.5e-7; the same at 4 steps a
+// row), and a wave of a split row adds a whole block by itself.
+template <int KIND>
+constexpr bool BLOCK_SUMS = KIND == HK_Q4 || KIND == HK_Q8;
+struct BlockSum {
+    float mid = 0.0f, tot = 0.0f;  // of blocks in the open group of four; of the groups
+    __device__ __forceinline__ void add(uint32_t b, float v) {  // block b's sum
+        mid += v;
+        if ((b & 3u) == 3u) {
+            tot += mid;
+            mid = 0.0f;
+        }
+    }
+};
+// After step t: acc[r] into its block sums where t ends a block.
+template <int KIND, int R>
+__device__ __forceinline__ void end_step(uint32_t t, float* acc, BlockSum* bs) {
+    if constexpr (BLOCK_SUMS<KIND>) {
+        if ((t & 3u) != 3u) return;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            bs[r].add(t >> 2, acc[r]);
+            acc[r] = 0.0f;
+        }
+    }
+}
+// A finished row's total; the sums start again.
+template <int KIND>
+__device__ __forceinline__ float row_total(float& acc, BlockSum& bs) {
+    float v = acc;
+    if constexpr (BLOCK_SUMS<KIND>) v = bs.tot + (bs.mid + acc);
+    acc = 0.0f;
+    bs = BlockSum{};
+    return v;
+}
+
 // Row totals of a finished group of R tiles into the workgroup's LDS row
 // buffer (unscaled; tiles r >= nvalid alias T[0] and are skipped).
-template <int R>
-__device__ __forceinline__ void flush_group(float* acc, const uint32_t* T, int nvalid, uint32_t t0, int lane,
-                                            float* ysh) {
+template <int KIND, int R>
+__device__ __forceinline__ void flush_group(float* acc, BlockSum* bs, const uint32_t* T, int nvalid, uint32_t t0,
+                                            int lane, float* ysh) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const float v = tile_row_sum(acc[r]);
+        const float v = tile_row_sum(row_total<KIND>(acc[r], bs[r]));
         if (r < nvalid && lane < 16) ysh[(T[r] - t0) * 16u + (uint32_t)lane] = v;
-        acc[r] = 0.0f;
     }
 }
 
@@ -336,6 +375,7 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
     const float* SX = reinterpret_cast<const float*>(lds + (size_t)o.steps * Kcfg<KIND>::P * A_TILE_STRIDE);
 
     float acc[R];
+    BlockSum bs[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0f;
     ItemStride<D> adv;
@@ -345,7 +385,8 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             compute_step<KIND, R>(f[d], ts[d], A, SX, q, acc);
-            if (ts[d] + 1 == o.steps) flush_group<R>(acc, T[d], nv[d], t0, lane, ysh);
+            end_step<KIND, R>(ts[d], acc, bs);
+            if (ts[d] + 1 == o.steps) flush_group<KIND, R>(acc, bs, T[d], nv[d], t0, lane, ysh);
             adv.next(W, it + D + d, last, T[d], R, &nv[d], &ts[d]);
             if constexpr (KIND == HK_MIXED) {
                 // headers from LDS: the data loads wait for an LDS read, not
@@ -364,7 +405,8 @@ gemv_tiled_kernel(const OrganView* __restrict__ organs, uint32_t n_organs, const
     for (int d = 0; d < D; ++d) {
         if (it + d >= W.n) break;
         compute_step<KIND, R>(f[d], ts[d], A, SX, q, acc);
-        if (ts[d] + 1 == o.steps) flush_group<R>(acc, T[d], nv[d], t0, lane, ysh);
+        end_step<KIND, R>(ts[d], acc, bs);
+        if (ts[d] + 1 == o.steps) flush_group<KIND, R>(acc, bs, T[d], nv[d], t0, lane, ysh);
     }
     __syncthreads();
     const uint32_t nrows = (t1 > t0 ? t1 - t0 : 0u) * 16u;
@@ -460,6 +502,7 @@ struct TileWalk {
         const float* SX = reinterpret_cast<const float*>(img + (size_t)o.steps * Kcfg<KIND>::P * A_TILE_STRIDE);
         const int q = lane >> 4;
         float acc[R];
+        BlockSum bs[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = 0.0f;
         ItemStride<D> adv;
@@ -469,7 +512,8 @@ struct TileWalk {
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 compute_step<KIND, R>(f[d], ts[d], A, SX, q, acc);
-                if (ts[d] + 1 == o.steps) flush_group<R>(acc, T[d], nv[d], t0, lane, ysh);
+                end_step<KIND, R>(ts[d], acc, bs);
+                if (ts[d] + 1 == o.steps) flush_group<KIND, R>(acc, bs, T[d], nv[d], t0, lane, ysh);
                 adv.next(W, it + D + d, last, T[d], R, &nv[d], &ts[d]);
                 fetch_step<KIND, R>(o, T[d], nv[d], ts[d], lane, f[d]);
             }
@@ -478,7 +522,8 @@ struct TileWalk {
         for (int d = 0; d < D; ++d) {
             if (it + d >= W.n) break;
             compute_step<KIND, R>(f[d], ts[d], A, SX, q, acc);
-            if (ts[d] + 1 == o.steps) flush_group<R>(acc, T[d], nv[d], t0, lane, ysh);
+            end_step<KIND, R>(ts[d], acc, bs);
+            if (ts[d] + 1 == o.steps) flush_group<KIND, R>(acc, bs, T[d], nv[d], t0, lane, ysh);
         }
     }
 };
@@ -901,36 +946,45 @@ struct SplitArgs {
 
 constexpr size_t SPLIT_LDS_LIMIT = 128 * 1024;
 
+// Steps of a tile that each of its KS waves runs (past the last: no work).
+template <int KIND>
+__host__ __device__ constexpr uint32_t split_per(uint32_t S, uint32_t ks_log) {
+    return BLOCK_SUMS<KIND> ? (((S + 3u) / 4u + (1u << ks_log) - 1u) >> ks_log) * 4u
+                            : (S + (1u << ks_log) - 1u) >> ks_log;
+}
+
 // LDS: the x image, then (RES) a copy of x and the residual's products, then
-// (KS > 1) the {scale, v} terms of a chunk of steps of every tile of a round,
-// then (RES) the rows' base sums.
+// (KS > 1) the {scale, v} terms or block sums of a chunk of steps of every tile
+// of a round, then (RES) the rows' base sums.
 template <int KIND, bool RES>
 struct SplitLds {
     static constexpr uint32_t TERMS = KIND == HK_MIXED ? 2u : 1u;  // a step's
-    uint32_t chunk;  // items of a wave between barriers
+    // 256-byte words of a wave's item
+    static constexpr uint32_t WORDS = BLOCK_SUMS<KIND> ? 1u : 2u * TERMS;
+    uint32_t chunk;  // items of a wave between barriers (BLOCK_SUMS: one, of four steps)
     size_t xs, vals, terms, ysh, total;
     __host__ __device__ SplitLds(uint32_t S, uint32_t cols, uint32_t tpw, uint32_t waves, uint32_t per, uint32_t bufs)
-        : chunk(per < 4u ? per : 4u) {
+        : chunk(BLOCK_SUMS<KIND> ? 1u : per < 4u ? per : 4u) {
         xs = (x_lds_bytes<KIND>(S) + 15u) & ~(size_t)15;
         vals = xs + (RES ? (size_t)cols * 4u : 0);
         terms = vals + (RES ? (size_t)RICE_BATCH * 4u : 0);
-        ysh = terms + (size_t)bufs * waves * chunk * TERMS * 512u;  // (bufs 0: KS = 1)
+        ysh = terms + (size_t)bufs * waves * chunk * WORDS * 256u;  // (bufs 0: KS = 1)
         total = ysh + (RES ? (size_t)tpw * 64u : 0);
     }
 };
 
-// A row's terms are added in step order whatever KS is, so an organ's sums are
-// the same bits alone, in a set of any size and as an lm_head.  KS = 1: a wave
-// walks its tiles (t0 + its index, + TS, ...).  SPLIT (KS > 1): the workgroup
-// takes TS tiles a round, wave k of a tile its steps k, k + KS, ...; the waves
-// leave each lane's {scale, v} in LDS and, every four items, one wave per tile
-// (another each round) runs the same chain of fused multiply-adds that one
-// wave walking the tile would, while the others are in the next items.  Every
-// wave runs the same number of items, so all meet at each barrier; items past
-// the tile's steps re-read a valid one and leave {-0, 0}, which changes no
-// sum.  (The chain is in the code once: inlined after every item of the
-// unrolled loop it cost up to 1 us of instruction fetches, 20 q8 512 x 2048 5.6
-// against 5.1.)
+// A row's terms are added as one wave walking the row adds them, whatever KS
+// is, so an organ's sums are the same bits alone, in a set of any size and as
+// an lm_head.  KS = 1: a wave walks its tiles (t0 + its index, + TS, ...).
+// SPLIT (KS > 1): the workgroup takes TS tiles a round, wave k of a tile its
+// steps k, k + KS, ... (BLOCK_SUMS: its blocks of four steps, the same way);
+// the waves leave each lane's {scale, v} (the block's sum) in LDS and, every
+// four items, one wave per tile (another each round) adds them in order, while
+// the others are in the next items.  Every wave runs the same number of items,
+// so all meet at each barrier; items past the tile's steps re-read a valid one
+// and leave {-0, 0}, which changes no sum.  (The chain is in the code once:
+// inlined after every item of the unrolled loop it cost up to 1 us of
+// instruction fetches, 20 q8 512 x 2048 5.6 against 5.1.)
 // RES: the HGRAVR02 residual added to the base sums in the same launch (256
 // threads; one round; records loaded before the image build).
 // HEAD: x is the hidden state; the prologue forms RMSNorm(1+w) of it and the
@@ -959,9 +1013,8 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     const uint32_t S = o.steps, KS = 1u << a.ks_log, TS = 1u << a.ts_log;
     const uint32_t ksl = wave & (KS - 1u), tsl = wave >> a.ks_log;
     const uint32_t t0 = part * a.tpw, t1 = min(t0 + a.tpw, o.n_tiles);
-    // SPLIT: item j of a wave is step ksl + KS j of its tile, per items a
-    // tile, D of them in flight
-    const uint32_t per = SPLIT ? (S + KS - 1u) >> a.ks_log : S;
+    // SPLIT: per items a tile and wave, D of them in flight
+    const uint32_t per = SPLIT ? split_per<KIND>(S, a.ks_log) : S;
     // (KS = 1: a wave may have no tile)
     const uint32_t rounds = SPLIT || t0 + tsl < t1 ? (t1 - t0 - (SPLIT ? 0u : tsl) + TS - 1u) >> a.ts_log : 0u;
     const uint32_t n = rounds * per;
@@ -990,7 +1043,10 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
         }
     };
     auto f_tile = [&]() { return min(fT, t1 - 1u); };
-    auto f_step = [&]() { return SPLIT ? min(ksl + (fj << a.ks_log), S - 1u) : fj; };
+    auto nth = [&](uint32_t j) {  // SPLIT: the step of this wave's item j
+        return BLOCK_SUMS<KIND> ? 4u * (ksl + (j >> 2 << a.ks_log)) + (j & 3u) : ksl + (j << a.ks_log);
+    };
+    auto f_step = [&]() { return SPLIT ? min(nth(fj), S - 1u) : fj; };
     Frag<KIND, 1> f[D];
     if constexpr (KIND == HK_MIXED) {
         uint4 h[D];
@@ -1046,6 +1102,7 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
 
     const ImageA A{lds, a_lane_offset(lane)};
     float2* terms = reinterpret_cast<float2*>(lds + M.terms) + (uint32_t)lane * TERMS;  // + 64 TERMS a step
+    float* sums = reinterpret_cast<float*>(lds + M.terms) + lane;                      // BLOCK_SUMS: + 64 a block
     float* ysh = reinterpret_cast<float*>(lds + M.ysh);
     uint64_t best = 0;
     auto put_tile = [&](uint32_t T, float v) {  // v: this lane's part of the tile's row sums
@@ -1061,8 +1118,48 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
         }
     };
     float acc = 0.0f;  // SPLIT: of the tile that this wave sums
+    BlockSum bs;
     if constexpr (SPLIT) {
         uint32_t buf = 0;
+        float blk = 0.0f;
+        // adds up items jb .. jb + 3 of every wave of tile T (k-th of its
+        // round), in order; last: and ends the row
+        auto sum = [&](uint32_t T, uint32_t k, uint32_t jb, bool last) {
+            if constexpr (BLOCK_SUMS<KIND>) {
+                const float* t = sums + (((buf << a.ts_log) + k) << a.ks_log) * 64u;
+                const uint32_t b0 = jb / 4u << a.ks_log;  // (KS > 2: a multiple of 4)
+                auto add = [&](auto count) {
+                    constexpr uint32_t N = decltype(count)::value;
+                    float e[N];
+#pragma unroll
+                    for (uint32_t u = 0; u < N; ++u) e[u] = t[u * 64u];
+#pragma unroll
+                    for (uint32_t u = 0; u < N; ++u) bs.add(N > 2u ? u : b0 + u, e[u]);
+                    t += N * 64u;
+                };
+                if (KS >= 8u)
+                    for (uint32_t i = KS >> 3; i; --i) add(std::integral_constant<uint32_t, 8>{});
+                else if (KS == 4u) add(std::integral_constant<uint32_t, 4>{});
+                else add(std::integral_constant<uint32_t, 2>{});
+            } else {
+                const float2* t = terms + (((buf << a.ts_log) + k) * M.chunk << a.ks_log) * 64u * TERMS;
+                const uint32_t m = (min(4u, per - jb) << a.ks_log) * TERMS;  // a multiple of 2
+                auto add = [&](auto count) {
+                    constexpr uint32_t N = decltype(count)::value;
+                    float2 e[N];
+#pragma unroll
+                    for (uint32_t u = 0; u < N; ++u) e[u] = t[u / TERMS * 64u * TERMS + u % TERMS];
+#pragma unroll
+                    for (uint32_t u = 0; u < N; ++u) acc = __builtin_fmaf(e[u].x, e[u].y, acc);
+                    t += N * 64u;
+                };
+                for (uint32_t i = m >> 4; i; --i) add(std::integral_constant<uint32_t, 16>{});
+                if (m & 8u) add(std::integral_constant<uint32_t, 8>{});
+                if (m & 4u) add(std::integral_constant<uint32_t, 4>{});
+                if (m & 2u) add(std::integral_constant<uint32_t, 2>{});
+            }
+            if (last) put_tile(T, row_total<KIND>(acc, bs));
+        };
         for (uint32_t round = 0; round < rounds; ++round)
             for (uint32_t j0 = 0; j0 < per; j0 += D) {
                 // chunks of 4 items: this group's first slot
@@ -1074,8 +1171,16 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
                 }
                 auto leave = [&](uint32_t d) {
                     if (j0 + d >= per) return;
-                    const uint32_t cs = ksl + ((j0 + d) << a.ks_log);
+                    const uint32_t cs = nth(j0 + d);
                     const bool on = cs < S;
+                    if constexpr (BLOCK_SUMS<KIND>) {  // (D is a block)
+                        if (d == 0) blk = 0.0f;
+                        compute_terms<KIND, 1>(f[d], min(cs, S - 1u), A, sx, q, [&](int, float s, float v) {
+                            blk = __builtin_fmaf(on ? s : -0.0f, on ? v : 0.0f, blk);
+                        });
+                        if (d == D - 1u) sums[((((buf << a.ts_log) + tsl) << a.ks_log) + ksl) * 64u] = blk;
+                        return;
+                    }
                     float2* o2 = terms + (((((buf << a.ts_log) + tsl) * M.chunk + c0 + d) << a.ks_log) + ksl) * 64u * TERMS;
                     compute_terms<KIND, 1>(f[d], min(cs, S - 1u), A, sx, q, [&](int, float s, float v) {
                         *o2++ = make_float2(on ? s : -0.0f, on ? v : 0.0f);
@@ -1096,38 +1201,18 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
                 }
                 if (!last && c0 + D < 4u) continue;
                 __syncthreads();
-                // the chunk's terms of the round's tiles, one tile per wave
+                // the round's tiles, one tile per wave
                 const uint32_t k = (wave - (round << a.ts_log)) & ((nthr >> 6) - 1u), T = t0 + (round << a.ts_log) + k;
-                if (k < TS && T < t1) {
-                    const float2* t = terms + (((buf << a.ts_log) + k) * M.chunk << a.ks_log) * 64u * TERMS;
-                    const uint32_t m = (min(c0 + D, per - (j0 - c0)) << a.ks_log) * TERMS;  // a multiple of 2
-                    auto add = [&](auto count) {
-                        constexpr uint32_t N = decltype(count)::value;
-                        float2 e[N];
-#pragma unroll
-                        for (uint32_t u = 0; u < N; ++u) e[u] = t[u / TERMS * 64u * TERMS + u % TERMS];
-#pragma unroll
-                        for (uint32_t u = 0; u < N; ++u) acc = __builtin_fmaf(e[u].x, e[u].y, acc);
-                        t += N * 64u;
-                    };
-                    for (uint32_t i = m >> 4; i; --i) add(std::integral_constant<uint32_t, 16>{});
-                    if (m & 8u) add(std::integral_constant<uint32_t, 8>{});
-                    if (m & 4u) add(std::integral_constant<uint32_t, 4>{});
-                    if (m & 2u) add(std::integral_constant<uint32_t, 2>{});
-                    if (last) {
-                        put_tile(T, acc);
-                        acc = 0.0f;
-                    }
-                }
+                if (k < TS && T < t1) sum(T, k, j0 - c0, last);
                 buf ^= a.bufs - 1u;
             }
     } else {
         uint32_t cT = t0 + tsl, cj = 0, it = 0;
         auto consume = [&](const Frag<KIND, 1>& fr) {
             compute_step<KIND, 1>(fr, cj, A, sx, q, &acc);
+            end_step<KIND, 1>(cj, &acc, &bs);
             if (++cj < per) return;
-            put_tile(cT, acc);
-            acc = 0.0f;
+            put_tile(cT, row_total<KIND>(acc, bs));
             cj = 0;
             cT += TS;
         };
@@ -1220,40 +1305,49 @@ static uint32_t pow2_ceil(uint32_t v) {
 //   * up to 1,024 row tiles the workgroups are what is scarce: about one per
 //     CU, so tpw = tiles / 256 rounded up to a power of two, and as many waves
 //     as the steps and the image (one chunk of 8 columns a thread) employ.
-//     One Q4 2048 x 7168: 14.2 -> 5.3, q8 4096 x 2048: 7.6 -> 3.7, q8 2048 x
-//     7168: 21.8 -> 5.9, binary 4096 x 2048: 4.1 -> 3.35; 20 mixed organs (640
-//     tiles): 5.35 -> 4.1; 20 Q4 organs: 6.8 -> 4.4.  (Wide rows with 8 waves
-//     instead of 16: 0.3 us more for Q4 2048 x 7168, 0.7 for q8.)
-//   * up to 2,048 tiles one wave per tile, 8 tiles side by side (34 Q4 organs:
-//     6.95 -> 5.1, binary 4.4 -> 3.9, mixed 5.2 -> 4.6; 40 Q4 organs with 7168
-//     columns: 25.4 -> 15.1; steps split over two waves: 6.1 and 17);
-//   * up to 4,096 tiles four waves a tile where the rows have more than 16
-//     steps (80 Q4 organs with 7168 columns: 30.5 -> 26.3; q8 with 4096: 31.2
-//     -> 27.3), the short kinds one wave per tile (mixed 6.05 -> 5.63, binary
-//     5.07 -> 4.88); Q4 of 16 steps walks (80 organs: 9.4 against 9.8);
+//     One Q4 2048 x 7168: 14.2 -> 5.2, q8 4096 x 2048: 7.6 -> 3.6, q8 2048 x
+//     7168: 21.8 -> 5.7, binary 4096 x 2048: 4.1 -> 3.35; 20 mixed organs (640
+//     tiles): 5.35 -> 4.2; 20 Q4 organs: 6.8 -> 4.4.  (Wide rows with 8 waves
+//     instead of 16: 0.3 us more for Q4 2048 x 7168, 0.7 for q8; rows of one
+//     or two blocks with 8 waves instead of 4: 0.1-0.2 more.)
+//   * up to 2,048 tiles one wave per tile, 8 tiles side by side (binary 4.4 ->
+//     3.9, mixed 5.2 -> 4.6; 40 Q4 organs with 7168 columns: 25.4 -> 15.1), or
+//     four waves a tile for Q4 of up to 32 steps in at most five tiles a CU
+//     (20,000 x 2048 5.6 against 6.4; 50 organs 6.3 against 5.9) and for q8
+//     (33 organs 7.55 against 8.3, 64 organs 12.3 against 14.3) but the
+//     longest rows in few tiles (7168 columns, 33 organs 22.5 against 21.1, 64
+//     organs 36.1 against 38);
+//   * up to 4,096 tiles Q4 of more than 16 steps one wave per tile (100 organs
+//     with 7168 columns: 40 -> 31.5, four waves 33.7), q8 four waves (100
+//     organs 18.1), the short kinds one wave per tile, 4 side by side (mixed
+//     6.05 -> 5.63, binary 5.07 -> 4.88); Q4 of 16 steps walks (80 organs: 9.4
+//     against 9.8);
 //   * beyond, q8 (200 organs: 42.7 -> 36.6) and mixed (8.9 -> 8.05) up to the
 //     streamed shapes; the others' walk is faster (binary 320 organs: 9.7
 //     against 10.8; 200 Q4 organs: 20.1 against 19.9, with 7168 columns equal).
 // HEAD: every workgroup ends in one atomic max on the same word, which the
-// memory side takes at about 12 ns each (a binary 151,936 x 2048 lm_head over
-// 1,900 workgroups: 30 us for 44 MB), so one or two balanced workgroups per
-// CU, 8 waves each.  One wave per tile for binary (16.5 us) and for short rows
-// or few tiles (q8 32,000 x 1024 10.9 against 13.3 with four waves a tile; Q4
-// 32,000 x 2048 12.3 against 13.7), four else (q8 151,936 x 2048 49.9 against
-// 52.2, 65,000 rows 26.5 against 29.2; Q4 151,936 x 4096 62.7).  A q8 lm_head
-// larger than the Infinity Cache loads non-temporally with one workgroup per
-// CU (128,256 x 4096: 96.2 -> 84; below, the hint and the fewer loads in flight
-// cost: 65,000 rows 25.9 -> 34.8; Q4 of these sizes fits and gains nothing from
-// it); tile counts that leave a nearly empty last round cost up to 30 %.
+// memory side takes at about 12 ns each (a binary 151,936 x 2048 lm_head: 15.1
+// us over 256 workgroups, 16.2 over 594, 23.2 over 1,187), so one or two
+// balanced workgroups per CU, 8 waves each.  One wave per tile for binary and
+// for short rows (q8 32,000 x 1024 11.3 against 12.2 with four waves a tile; Q4
+// 32,000 x 2048 12.3 against 13), eight waves for long rows in at most three
+// tiles a CU (q8 11,409 x 2048 10.8, four 11.1, one 11.4; Q4 11,409 x 4096 11.5,
+// 11.9, 12.5), four else (q8 151,936 x 2048 49.7; 65,000 rows 25.3; Q4 4096 x
+// 2048 8.2, one 9.0).  A q8 lm_head larger than the Infinity Cache loads
+// non-temporally with one workgroup per CU (128,256 x 4096: 96.2 -> 78; below,
+// the hint and the fewer loads in flight cost: 65,000 rows 25.9 -> 34.8; Q4 of
+// these sizes fits and gains nothing from it); tile counts that leave a nearly
+// empty last round cost up to 30 %.
 // RES (256 threads, at most 4 tiles a workgroup: a row's records are one
 // thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8
 // -> 6.6, 512 x 7168: 35.4 -> 8.7; above 4,096 tiles the two launches are
 // faster (160 organs: 11.0 against 11.8).
 static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uint32_t S, uint32_t cols) {
-    const uint32_t s2 = pow2_ceil(S);
+    const bool wide = kind == HK_Q4 || kind == HK_Q8;
+    const uint32_t s2 = pow2_ceil(wide ? (S + 3u) / 4u : S);  // (a wave's least: a block of four steps)
     if (head) {
-        const bool walk = kind == HK_BIN || S <= 8 || (S <= 16 && tiles <= 2048) || (S <= 32 && tiles > 512 && tiles <= 1024);
-        const uint32_t ks = walk ? 1u : 4u, ts = 8u / ks;
+        const bool walk = kind == HK_BIN || S <= 8 || (S <= 16 && tiles > 512 && tiles <= 2048);
+        const uint32_t ks = walk ? 1u : S >= 32 && tiles <= 768 ? 8u : 4u, ts = 8u / ks;
         const bool past_mall = kind == HK_Q8 && tiles * 16u * cols > MALL_BYTES;
         const uint32_t wgs = kind == HK_BIN || tiles <= 4096 || past_mall ? 256u : 512u;
         const uint32_t even = (uint32_t)((tiles + wgs - 1u) / wgs);
@@ -1266,15 +1360,21 @@ static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uin
         return {4, ks, std::max(tpw, 4u / ks)};
     }
     if (S == 1 || tiles >= 16384) return {0, 0, 0};
-    const bool wide = kind == HK_Q4 || kind == HK_Q8;
     if (tiles <= 1024) {
         const bool w16 = cols > 4096 || (S >= 16 && tpw == 4) || (wide && S >= (tpw == 1 ? 48u : 32u));
-        const uint32_t w = w16 ? 16u : S < 16 && tpw == 1 ? 4u : 8u;
+        const bool w4 = wide ? s2 <= 2u && tpw <= 2u : S < 16 && tpw == 1;
+        const uint32_t w = w16 ? 16u : w4 ? 4u : 8u;
         const uint32_t ks = std::min(w / tpw, s2);
         return {w, ks, std::max(tpw, w / ks)};
     }
-    if (tiles <= 2048) return {8, 1, 8};
-    if (wide && S >= 16 && (tiles <= 4096 ? S > 16 : kind == HK_Q8)) return {8, 4, 2};
+    if (tiles <= 2048) {
+        const bool four = kind == HK_Q8   ? S >= 16 && (S <= 64 || tiles > 1536)
+                          : kind == HK_Q4 ? S >= 16 && S <= 32 && tiles <= 1280
+                                          : false;
+        return four ? SplitShape{8, 4, 2} : SplitShape{8, 1, 8};
+    }
+    if (kind == HK_Q4 && S > 16 && tiles <= 4096) return {8, 1, 8};
+    if (kind == HK_Q8 && S >= (tiles <= 4096 ? 17u : 16u)) return {8, 4, 2};
     if (!wide && (tiles <= 4096 || kind == HK_MIXED)) return {4, 1, 4};
     return {0, 0, 0};
 }
@@ -1286,7 +1386,8 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     *done = false;
     const SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
     if (!c.waves || (!HEAD && vectors_overlap(x, xs, sh.cols, y, ys, sh.rows, n))) return hipSuccess;
-    const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw, ts = waves / ks, per = (sh.steps + ks - 1u) / ks;
+    const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw, ts = waves / ks;
+    const uint32_t per = split_per<KIND>(sh.steps, (uint32_t)__builtin_ctz(ks));
     const uint32_t bufs = ks == 1u ? 0u : tpw == ts && per <= 4u ? 1u : 2u;
     const size_t lds = SplitLds<KIND, RES>(sh.steps, sh.cols, tpw, waves, per, bufs).total;
     if (lds > SPLIT_LDS_LIMIT) return hipSuccess;

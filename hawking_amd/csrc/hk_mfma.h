@@ -646,9 +646,10 @@ __device__ __forceinline__ void fetch_mixed(const OrganView& o, const uint4& h, 
 // 0.74 -> 0.84 of 8 TB/s, binary (with the 2-tile, 5-deep shape) 0.76 ->
 // 0.78; the hint on the 2-byte scale loads, on the mixed kind's loads (its
 // binary lanes re-read their 16 bytes) or on the 3-bit kind's measured
-// slower, and so did the terminal head's q8 launch (its kernel runs NT =
-// false).  The default is off: the batch-1 MoE decode kernels, bound by
-// their latency chains, ran 1-2 % faster with ordinary loads.
+// slower.  The terminal head asks for it only for a q8 lm_head larger than
+// the Infinity Cache (smaller ones are found there by the next token).  The
+// default is off: the batch-1 MoE decode kernels, bound by their latency
+// chains, ran 1-2 % faster with ordinary loads.
 template <int KIND, int R, bool NT = false>
 __device__ __forceinline__ void fetch_one(const OrganView& o, uint32_t T, uint32_t t, int lane, Frag<KIND, R>& f,
                                           int r) {

@@ -71,7 +71,8 @@ def test_small_launches_within_bound(ctx, oracle, kind, rows, cols):
 # ragged organs whose row tiles sit on both sides of each change of shape (the
 # long rows: the shapes of Q4 and q8 organs of more than 16 steps)
 TILES = [(k, t, 1024) for k in ("q4", "q8", "bin", "mixed", "rice") for t in (256, 257, 513, 1025, 2049, 4097)]
-TILES += [("q4", t, 2176) for t in (1024, 1025, 2048, 2049, 4096, 4097)]
+TILES += [("q4", t, 2176) for t in (1024, 1025, 1280, 1281, 2048, 2049, 4096, 4097)]
+TILES += [("q8", t, 4224) for t in (1025, 1536, 1537, 2048)] + [(k, t, 512) for k in ("q4", "q8") for t in (512, 513)]
 TILES += [(k, t, c) for k, c in (("q8", 1088), ("mixed", 1024)) for t in (4096, 16383, 16384)]
 
 
@@ -128,6 +129,30 @@ def test_bits_do_not_depend_on_the_set(ctx, oracle, kind, cols):
         assert np.all(got[:, 509:] == 7.0)
         for i in alone:
             assert i >= n or np.array_equal(got[i, :509], alone[i]), (n, i)
+
+
+@pytest.mark.parametrize("kind,unit", [("q4", 128), ("q8", 64)])
+def test_long_rows_round_like_short_ones(ctx, oracle, kind, unit):
+    """Error against 64 bits of rows of S = 7168 / unit steps.  A row of four
+    steps shows what its terms round (e0); adding the blocks up adds, with a
+    roundoff of 0.41 2^-24 of each partial sum and random signs, that times the
+    square root of 5 + S / 32 (one chain of S steps: of S / 2, 2.1e-7 for Q4 and
+    2.3e-7 for q8, beyond the bound).  8 % for the sample."""
+    from hawking_amd.organs import OrganSet
+    print("[gpu-case] split gemv, long rows in 64 bits", kind, flush=True)
+    sys.stdout.flush()
+
+    def error(cols, n):
+        o = _organ(ctx, oracle, kind, 2048, cols, 0x5000)
+        xs = np.random.default_rng(cols).standard_normal((n, cols)).astype(np.float32)
+        y = ctx.to_device(np.zeros((n, 2048), np.float32))
+        OrganSet(ctx, [o] * n).gemv(ctx.to_device(xs), cols, y, 2048)
+        want = xs.astype(np.float64) @ o.decode().astype(np.float64).T
+        return np.linalg.norm(y.download() - want) / np.linalg.norm(want)
+
+    e0, S = error(4 * unit, 16), 7168 // unit
+    for n in (2, 5, 12):
+        assert error(7168, n) <= 1.08 * np.hypot(e0, 0.41 * 2.0 ** -24 * np.sqrt(5 + S / 32)), n
 
 
 ONE = [(k, 300, 1024) for k in KIND] + [("rice", 8, 128), ("rice", 65536, 128), ("bin", 40, 512)]

@@ -29,6 +29,9 @@ def _organ(ctx, oracle, kind, rows, cols):
 CASES = [(k, v, h, c) for k in sorted(KIND)
          for v, h, c in ((1, 128, 0), (15, 640, 3), (257, 8192, 1), (4101, 1024, 100), (70000, 512, 331))]
 CASES.append(("q8", 140001, 2048, 7))  # weights larger than the Infinity Cache
+# row tiles on both sides of each change of the waves a tile
+CASES += [(k, v, h, 5) for k, h in (("q8", 2048), ("q4", 4096)) for v in (12288, 12289)]
+CASES += [(k, v, h, 5) for k, h in (("q8", 1024), ("q4", 2048)) for v in (8192, 8193, 32768, 32769)]
 
 
 @pytest.mark.parametrize("kind,vocab,hidden,cut", CASES)
