@@ -57,7 +57,7 @@ struct ItemStride {
 };
 
 // How a lane's terms of a row are summed, in every launch shape alike: in step
-// order, and for Q4 and q8 (16 to 128 steps a row) in blocks of four steps,
+// order, and for Q4 and q8 (up to 56 and 112 steps a row) in blocks of four,
 // the blocks' sums added up four at a time and those in order.  The shorter
 // chains round less (relative error against 64 bits at 2048 x 7168, one chain
 // -> blocks: Q4 2.1e-7 -> 1.75e-7, q8 2.3e-7 -> 1.5e-7; the same at 4 steps a

@@ -164,8 +164,8 @@ struct SynthSrc {
 // (G <= 128: at most 16, inside one DPP row), so a wave reads 2 KiB of
 // consecutive bytes and its maximum, sum and codes need no LDS.  With one
 // thread per group (loads 4 G bytes apart, each line fetched again for every
-// element) a 2048 x 7168 Q4 pack took 490 us; it takes 15 us here, 4.3 TB/s of
-// the 4 bytes a weight read and the codes written.
+// element) a 2048 x 7168 Q4 pack took 490 us; it takes 13.7-15.5 us here, 4.3-4.9
+// TB/s of the 4 bytes a weight read and the codes written.
 __device__ __forceinline__ void load8(const float* w, bool v4, float (&v)[8]) {
     if (v4) {
         const float4* p = reinterpret_cast<const float4*>(w);
