@@ -1310,6 +1310,11 @@ static uint32_t pow2_ceil(uint32_t v) {
 //     tiles): 5.35 -> 4.2; 20 Q4 organs: 6.8 -> 4.4.  (Wide rows with 8 waves
 //     instead of 16: 0.3 us more for Q4 2048 x 7168, 0.7 for q8; rows of one
 //     or two blocks with 8 waves instead of 4: 0.1-0.2 more.)
+//   * Q4 and q8 rows of eight blocks or more where three or five tiles a
+//     workgroup give each CU one (a power of two leaves some idle): all waves
+//     on one tile after the other (20 q8 organs 5.14 -> 4.95, 33 organs 7.6 ->
+//     7.25, with 7168 columns 21.3 -> 19.7; Q4 11,000 x 4096 6.7 -> 5.9, 33
+//     organs with 7168 columns 14.5 -> 13.1);
 //   * up to 2,048 tiles one wave per tile, 8 tiles side by side (binary 4.4 ->
 //     3.9, mixed 5.2 -> 4.6; 40 Q4 organs with 7168 columns: 25.4 -> 15.1), or
 //     four waves a tile for Q4 of up to 32 steps in at most five tiles a CU
@@ -1342,7 +1347,8 @@ static uint32_t pow2_ceil(uint32_t v) {
 // thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8
 // -> 6.6, 512 x 7168: 35.4 -> 8.7; above 4,096 tiles the two launches are
 // faster (160 organs: 11.0 against 11.8).
-static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uint32_t S, uint32_t cols) {
+static SplitShape split_shape(int kind, bool res, bool head, uint32_t n, uint32_t n_tiles, uint32_t S, uint32_t cols) {
+    const uint64_t tiles = (uint64_t)n * n_tiles;
     const bool wide = kind == HK_Q4 || kind == HK_Q8;
     const uint32_t s2 = pow2_ceil(wide ? (S + 3u) / 4u : S);  // (a wave's least: a block of four steps)
     if (head) {
@@ -1360,6 +1366,12 @@ static SplitShape split_shape(int kind, bool res, bool head, uint64_t tiles, uin
         return {4, ks, std::max(tpw, 4u / ks)};
     }
     if (S == 1 || tiles >= 16384) return {0, 0, 0};
+    if (wide && S >= 32 && tiles > 512 && tiles <= 1280) {
+        uint32_t even = 3;
+        while (even < 5 && (uint64_t)n * ((n_tiles + even - 1u) / even) > 256u) ++even;
+        const uint32_t w = S >= 48 ? 16u : 8u;
+        if (even != 4 && (uint64_t)n * ((n_tiles + even - 1u) / even) <= 256u) return {w, w, even};
+    }
     if (tiles <= 1024) {
         const bool w16 = cols > 4096 || (S >= 16 && tpw == 4) || (wide && S >= (tpw == 1 ? 48u : 32u));
         const bool w4 = wide ? s2 <= 2u && tpw <= 2u : S < 16 && tpw == 1;
@@ -1384,7 +1396,7 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
                                const OrganView& sh, const float* x, size_t xs, float* y, size_t ys, hipStream_t s,
                                bool* done, const HeadArgs& ha = {}, uint32_t* status = nullptr) {
     *done = false;
-    const SplitShape c = split_shape(KIND, RES, HEAD, (uint64_t)n * sh.n_tiles, sh.steps, sh.cols);
+    const SplitShape c = split_shape(KIND, RES, HEAD, n, sh.n_tiles, sh.steps, sh.cols);
     if (!c.waves || (!HEAD && vectors_overlap(x, xs, sh.cols, y, ys, sh.rows, n))) return hipSuccess;
     const uint32_t waves = c.waves, ks = c.ks, tpw = c.tpw, ts = waves / ks;
     const uint32_t per = split_per<KIND>(sh.steps, (uint32_t)__builtin_ctz(ks));

@@ -72,6 +72,7 @@ def test_small_launches_within_bound(ctx, oracle, kind, rows, cols):
 # long rows: the shapes of Q4 and q8 organs of more than 16 steps)
 TILES = [(k, t, 1024) for k in ("q4", "q8", "bin", "mixed", "rice") for t in (256, 257, 513, 1025, 2049, 4097)]
 TILES += [("q4", t, 2176) for t in (1024, 1025, 1280, 1281, 2048, 2049, 4096, 4097)]
+TILES += [(k, t, c) for k, c in (("q8", 2112), ("q4", 6176)) for t in (512, 513, 768, 769, 1024, 1025, 1280, 1281)]
 TILES += [("q8", t, 4224) for t in (1025, 1536, 1537, 2048)] + [(k, t, 512) for k in ("q4", "q8") for t in (512, 513)]
 TILES += [(k, t, c) for k, c in (("q8", 1088), ("mixed", 1024)) for t in (4096, 16383, 16384)]
 
