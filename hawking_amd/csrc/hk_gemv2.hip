@@ -981,8 +981,8 @@ struct SplitLds {
 // the waves leave each lane's {scale, v} (the block's sum) in LDS and, every
 // four items, one wave per tile (another each round) adds them in order, while
 // the others are in the next items.  Every wave runs the same number of items,
-// so all meet at each barrier; items past the tile's steps re-read a valid one
-// and leave {-0, 0}, which changes no sum.  (The chain is in the code once:
+// so all meet at each barrier; items past the tile's steps load a valid one
+// and leave {-0, 0} (add nothing to the block), which changes no sum.  (The chain is in the code once:
 // inlined after every item of the unrolled loop it cost up to 1 us of
 // instruction fetches, 20 q8 512 x 2048 5.6 against 5.1.)
 // RES: the HGRAVR02 residual added to the base sums in the same launch (256
@@ -1046,7 +1046,7 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
     auto nth = [&](uint32_t j) {  // SPLIT: the step of this wave's item j
         return BLOCK_SUMS<KIND> ? 4u * (ksl + (j >> 2 << a.ks_log)) + (j & 3u) : ksl + (j << a.ks_log);
     };
-    auto f_step = [&]() { return SPLIT ? min(nth(fj), S - 1u) : fj; };
+    auto f_step = [&]() { return SPLIT ? min(nth(min(fj, per - 1u)), S - 1u) : fj; };
     Frag<KIND, 1> f[D];
     if constexpr (KIND == HK_MIXED) {
         uint4 h[D];
@@ -1172,19 +1172,19 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
                 auto leave = [&](uint32_t d) {
                     if (j0 + d >= per) return;
                     const uint32_t cs = nth(j0 + d);
-                    const bool on = cs < S;
                     if constexpr (BLOCK_SUMS<KIND>) {  // (D is a block)
                         if (d == 0) blk = 0.0f;
-                        compute_terms<KIND, 1>(f[d], min(cs, S - 1u), A, sx, q, [&](int, float s, float v) {
-                            blk = __builtin_fmaf(on ? s : -0.0f, on ? v : 0.0f, blk);
-                        });
+                        if (cs < S) compute_step<KIND, 1>(f[d], cs, A, sx, q, &blk);
                         if (d == D - 1u) sums[((((buf << a.ts_log) + tsl) << a.ks_log) + ksl) * 64u] = blk;
                         return;
                     }
                     float2* o2 = terms + (((((buf << a.ts_log) + tsl) * M.chunk + c0 + d) << a.ks_log) + ksl) * 64u * TERMS;
-                    compute_terms<KIND, 1>(f[d], min(cs, S - 1u), A, sx, q, [&](int, float s, float v) {
-                        *o2++ = make_float2(on ? s : -0.0f, on ? v : 0.0f);
-                    });
+                    if (cs < S) {
+                        compute_terms<KIND, 1>(f[d], cs, A, sx, q, [&](int, float s, float v) { *o2++ = make_float2(s, v); });
+                    } else {
+#pragma unroll
+                        for (uint32_t u = 0; u < TERMS; ++u) o2[u] = make_float2(-0.0f, 0.0f);
+                    }
                 };
                 // (two bodies: a load under a condition would have every later
                 // item wait for all loads)
