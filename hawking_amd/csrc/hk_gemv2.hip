@@ -946,6 +946,9 @@ struct SplitArgs {
 
 constexpr size_t SPLIT_LDS_LIMIT = 128 * 1024;
 
+template <int KIND>
+constexpr uint32_t split_depth = KIND == HK_MIXED ? 2 : 4;  // steps in flight per wave
+enum { SPLIT_WALK, SPLIT_CHUNKS, SPLIT_ONCE };              // KS = 1; KS > 1; one round of at most split_depth items
 // Steps of a tile that each of its KS waves runs (past the last: no work).
 template <int KIND>
 __host__ __device__ constexpr uint32_t split_per(uint32_t S, uint32_t ks_log) {
@@ -975,25 +978,30 @@ struct SplitLds {
 
 // A row's terms are added as one wave walking the row adds them, whatever KS
 // is, so an organ's sums are the same bits alone, in a set of any size and as
-// an lm_head.  KS = 1: a wave walks its tiles (t0 + its index, + TS, ...).
-// SPLIT (KS > 1): the workgroup takes TS tiles a round, wave k of a tile its
-// steps k, k + KS, ... (BLOCK_SUMS: its blocks of four steps, the same way);
-// the waves leave each lane's {scale, v} (the block's sum) in LDS and, every
-// four items, one wave per tile (another each round) adds them in order, while
-// the others are in the next items.  Every wave runs the same number of items,
-// so all meet at each barrier; items past the tile's steps load a valid one
-// and leave {-0, 0} (add nothing to the block), which changes no sum.  (The chain is in the code once:
-// inlined after every item of the unrolled loop it cost up to 1 us of
-// instruction fetches, 20 q8 512 x 2048 5.6 against 5.1.)
+// an lm_head.  SPLIT_WALK (KS = 1): a wave walks its tiles (t0 + its index, +
+// TS, ...).  Else (KS > 1) the workgroup takes TS tiles a round, wave k of a
+// tile its steps k, k + KS, ... (BLOCK_SUMS: its blocks of four steps, the same
+// way); the waves leave each lane's {scale, v} (the block's sum) in LDS and,
+// every four items, one wave per tile (another each round) adds them in order,
+// while the others are in the next items.  Every wave runs the same number of
+// items, so all meet at each barrier; items past the tile's steps load a valid
+// one and leave {-0, 0} (add nothing to the block), which changes no sum.  (The
+// chain is in the code once: inlined after every item of the unrolled loop it
+// cost up to 1 us of instruction fetches, 20 q8 512 x 2048 5.6 against 5.1.)
+// SPLIT_ONCE: one round whose items are all in flight from the start
+// (SPLIT_CHUNKS the rest): as straight code instead of the loops' it is 0.1-0.35
+// us faster (20 mixed 512 x 2048 4.30 -> 4.12, 20 Q4 4.35 -> 4.03, 10 q8 4.08 ->
+// 3.80).
 // RES: the HGRAVR02 residual added to the base sums in the same launch (256
 // threads; one round; records loaded before the image build).
 // HEAD: x is the hidden state; the prologue forms RMSNorm(1+w) of it and the
 // epilogue folds the rows' greedy keys (HeadArgs; cols <= 8192, 512 threads).
 // NT: the weight loads carry the non-temporal hint.
-template <int KIND, bool SPLIT, bool RES, bool HEAD, bool NT = false>
+template <int KIND, int MODE, bool RES, bool HEAD, bool NT = false>
 __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs a) {
+    constexpr bool SPLIT = MODE != SPLIT_WALK;
     static_assert(!(RES && HEAD), "an lm_head has no fused residual");
-    constexpr uint32_t D = KIND == HK_MIXED ? 2 : 4;  // steps in flight per wave
+    constexpr uint32_t D = split_depth<KIND>;
     constexpr uint32_t TERMS = SplitLds<KIND, RES>::TERMS;
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ float red[HEAD ? 16 : 1];
@@ -1160,52 +1168,60 @@ __global__ void __launch_bounds__(RES ? 256 : 1024) gemv_split_kernel(SplitArgs 
             }
             if (last) put_tile(T, row_total<KIND>(acc, bs));
         };
-        for (uint32_t round = 0; round < rounds; ++round)
-            for (uint32_t j0 = 0; j0 < per; j0 += D) {
-                // chunks of 4 items: this group's first slot
-                const uint32_t c0 = j0 & 3u;
-                const bool last = j0 + D >= per;  // of the tile
-                if (last) {
-                    fj = 0;
-                    fT += TS;
-                }
-                auto leave = [&](uint32_t d) {
-                    if (j0 + d >= per) return;
-                    const uint32_t cs = nth(j0 + d);
-                    if constexpr (BLOCK_SUMS<KIND>) {  // (D is a block)
-                        if (d == 0) blk = 0.0f;
-                        if (cs < S) compute_step<KIND, 1>(f[d], cs, A, sx, q, &blk);
-                        if (d == D - 1u) sums[((((buf << a.ts_log) + tsl) << a.ks_log) + ksl) * 64u] = blk;
-                        return;
+        auto leave = [&](uint32_t j0, uint32_t d) {  // item j0 + d
+            if (j0 + d >= per) return;
+            const uint32_t cs = nth(j0 + d);
+            if constexpr (BLOCK_SUMS<KIND>) {  // (D is a block)
+                if (d == 0) blk = 0.0f;
+                if (cs < S) compute_step<KIND, 1>(f[d], cs, A, sx, q, &blk);
+                if (d == D - 1u) sums[((((buf << a.ts_log) + tsl) << a.ks_log) + ksl) * 64u] = blk;
+                return;
+            }
+            float2* o2 =
+                terms + (((((buf << a.ts_log) + tsl) * M.chunk + (j0 & 3u) + d) << a.ks_log) + ksl) * 64u * TERMS;
+            if (cs < S) {
+                compute_terms<KIND, 1>(f[d], cs, A, sx, q, [&](int, float s, float v) { *o2++ = make_float2(s, v); });
+            } else {
+#pragma unroll
+                for (uint32_t u = 0; u < TERMS; ++u) o2[u] = make_float2(-0.0f, 0.0f);
+            }
+        };
+        if constexpr (MODE == SPLIT_ONCE) {
+#pragma unroll
+            for (uint32_t d = 0; d < D; ++d) leave(0, d);
+            __syncthreads();
+            if (wave < TS && t0 + wave < t1) sum(t0 + wave, wave, 0, true);
+        } else {
+            for (uint32_t round = 0; round < rounds; ++round)
+                for (uint32_t j0 = 0; j0 < per; j0 += D) {
+                    // chunks of 4 items: this group's first slot
+                    const uint32_t c0 = j0 & 3u;
+                    const bool last = j0 + D >= per;  // of the tile
+                    if (last) {
+                        fj = 0;
+                        fT += TS;
                     }
-                    float2* o2 = terms + (((((buf << a.ts_log) + tsl) * M.chunk + c0 + d) << a.ks_log) + ksl) * 64u * TERMS;
-                    if (cs < S) {
-                        compute_terms<KIND, 1>(f[d], cs, A, sx, q, [&](int, float s, float v) { *o2++ = make_float2(s, v); });
+                    // (two bodies: a load under a condition would have every
+                    // later item wait for all loads)
+                    if (!last || round + 1u < rounds) {
+#pragma unroll
+                        for (uint32_t d = 0; d < D; ++d) {
+                            leave(j0, d);
+                            fetch_one<KIND, 1, NT>(o, f_tile(), f_step(), lane, f[d], 0);
+                            step_on();
+                        }
                     } else {
 #pragma unroll
-                        for (uint32_t u = 0; u < TERMS; ++u) o2[u] = make_float2(-0.0f, 0.0f);
+                        for (uint32_t d = 0; d < D; ++d) leave(j0, d);
                     }
-                };
-                // (two bodies: a load under a condition would have every later
-                // item wait for all loads)
-                if (!last || round + 1u < rounds) {
-#pragma unroll
-                    for (uint32_t d = 0; d < D; ++d) {
-                        leave(d);
-                        fetch_one<KIND, 1, NT>(o, f_tile(), f_step(), lane, f[d], 0);
-                        step_on();
-                    }
-                } else {
-#pragma unroll
-                    for (uint32_t d = 0; d < D; ++d) leave(d);
+                    if (!last && c0 + D < 4u) continue;
+                    __syncthreads();
+                    // the round's tiles, one tile per wave
+                    const uint32_t k = (wave - (round << a.ts_log)) & ((nthr >> 6) - 1u), T = t0 + (round << a.ts_log) + k;
+                    if (k < TS && T < t1) sum(T, k, j0 - c0, last);
+                    buf ^= a.bufs - 1u;
                 }
-                if (!last && c0 + D < 4u) continue;
-                __syncthreads();
-                // the round's tiles, one tile per wave
-                const uint32_t k = (wave - (round << a.ts_log)) & ((nthr >> 6) - 1u), T = t0 + (round << a.ts_log) + k;
-                if (k < TS && T < t1) sum(T, k, j0 - c0, last);
-                buf ^= a.bufs - 1u;
-            }
+        }
     } else {
         uint32_t cT = t0 + tsl, cj = 0, it = 0;
         auto consume = [&](const Frag<KIND, 1>& fr) {
@@ -1305,9 +1321,9 @@ static uint32_t pow2_ceil(uint32_t v) {
 //   * up to 1,024 row tiles the workgroups are what is scarce: about one per
 //     CU, so tpw = tiles / 256 rounded up to a power of two, and as many waves
 //     as the steps and the image (one chunk of 8 columns a thread) employ.
-//     One Q4 2048 x 7168: 14.2 -> 5.2, q8 4096 x 2048: 7.6 -> 3.6, q8 2048 x
-//     7168: 21.8 -> 5.7, binary 4096 x 2048: 4.1 -> 3.35; 20 mixed organs (640
-//     tiles): 5.35 -> 4.2; 20 Q4 organs: 6.8 -> 4.4.  (Wide rows with 8 waves
+//     One Q4 2048 x 7168: 14.2 -> 4.8, q8 4096 x 2048: 7.6 -> 3.4, q8 2048 x
+//     7168: 21.8 -> 5.6, binary 4096 x 2048: 4.1 -> 3.35; 20 mixed organs (640
+//     tiles): 5.35 -> 4.1; 20 Q4 organs: 6.8 -> 4.0.  (Wide rows with 8 waves
 //     instead of 16: 0.3 us more for Q4 2048 x 7168, 0.7 for q8; rows of one
 //     or two blocks with 8 waves instead of 4: 0.1-0.2 more.)
 //   * Q4 and q8 rows of eight blocks or more where three or five tiles a
@@ -1318,7 +1334,7 @@ static uint32_t pow2_ceil(uint32_t v) {
 //   * up to 2,048 tiles one wave per tile, 8 tiles side by side (binary 4.4 ->
 //     3.9, mixed 5.2 -> 4.6; 40 Q4 organs with 7168 columns: 25.4 -> 15.1), or
 //     four waves a tile for Q4 of up to 32 steps in at most five tiles a CU
-//     (20,000 x 2048 5.6 against 6.4; 50 organs 6.3 against 5.9) and for q8
+//     (20,000 x 2048 5.1 against 6.4; 50 organs 6.3 against 5.9) and for q8
 //     (33 organs 7.55 against 8.3, 64 organs 12.3 against 14.3) but the
 //     longest rows in few tiles (7168 columns, 33 organs 22.5 against 21.1, 64
 //     organs 36.1 against 38);
@@ -1425,10 +1441,12 @@ static hipError_t launch_split(const OrganView* organs, const ResView* res, cons
     a.ha = ha;
     a.status = status;
     const bool nt = HEAD && KIND == HK_Q8 && (uint64_t)sh.rows * sh.cols > MALL_BYTES;
-    auto* k = ks > 1 ? nt ? gemv_split_kernel<KIND, true, RES, HEAD, HEAD && KIND == HK_Q8>
-                          : gemv_split_kernel<KIND, true, RES, HEAD>
-              : nt   ? gemv_split_kernel<KIND, false, RES, HEAD, HEAD && KIND == HK_Q8>
-                     : gemv_split_kernel<KIND, false, RES, HEAD>;
+    auto* k = ks > 1 ? nt ? gemv_split_kernel<KIND, SPLIT_CHUNKS, RES, HEAD, HEAD && KIND == HK_Q8>
+                          : gemv_split_kernel<KIND, SPLIT_CHUNKS, RES, HEAD>
+              : nt   ? gemv_split_kernel<KIND, SPLIT_WALK, RES, HEAD, HEAD && KIND == HK_Q8>
+                     : gemv_split_kernel<KIND, SPLIT_WALK, RES, HEAD>;
+    if constexpr (!HEAD)
+        if (ks > 1 && tpw == ts && per <= split_depth<KIND>) k = gemv_split_kernel<KIND, SPLIT_ONCE, RES, HEAD>;
     hipLaunchKernelGGL(k, dim3(a.parts * n), dim3(64u * waves), lds, s, a);
     return hipGetLastError();
 }
