@@ -1316,49 +1316,56 @@ static uint32_t pow2_ceil(uint32_t v) {
 }
 
 // Where the split pays and its shape (us per launch, 20 launches in a graph;
-// against the walk of gemv_tiled_kernel; organs of 512 x 2048 unless stated):
+// against the walk of gemv_tiled_kernel; organs of 512 x 2048 unless stated).
+// A shape is waves / waves a tile / tiles a workgroup.
 //   * one step (<= 512 binary columns): nothing to split (2.95 against 3.1-3.35);
 //   * up to 1,024 row tiles the workgroups are what is scarce: about one per
 //     CU, so tpw = tiles / 256 rounded up to a power of two, and as many waves
-//     as the steps and the image (one chunk of 8 columns a thread) employ.
-//     One Q4 2048 x 7168: 14.2 -> 4.8, q8 4096 x 2048: 7.6 -> 3.4, q8 2048 x
-//     7168: 21.8 -> 5.6, binary 4096 x 2048: 4.1 -> 3.35; 20 mixed organs (640
-//     tiles): 5.35 -> 4.1; 20 Q4 organs: 6.8 -> 4.0.  (Wide rows with 8 waves
-//     instead of 16: 0.3 us more for Q4 2048 x 7168, 0.7 for q8; rows of one
-//     or two blocks with 8 waves instead of 4: 0.1-0.2 more.)
+//     as the steps and the image (one chunk of 8 columns a thread) employ; Q4
+//     and q8: as many waves a tile as the row has blocks (up to 16 / tpw), so
+//     that every step is in flight at once.  One Q4 2048 x 7168: 14.2 -> 4.8, q8
+//     4096 x 2048: 7.6 -> 3.4, q8 2048 x 7168: 21.8 -> 5.6, binary 4096 x 2048:
+//     4.1 -> 3.35; 20 mixed organs (640 tiles): 5.35 -> 4.1; 20 Q4 organs: 6.8
+//     -> 4.0; 10 Q4 organs of 23 steps 16/8/2 4.1, 8/4/2 4.7; one q8 organ of 36
+//     steps 16/16/1 3.7, 8/8/1 4.35.  Rows of five to eight blocks in 513 to 704
+//     tiles: 8/8/1 (23 q8 organs of 22 steps 4.5, 16/4/4 5.0);
 //   * Q4 and q8 rows of eight blocks or more where three or five tiles a
 //     workgroup give each CU one (a power of two leaves some idle): all waves
-//     on one tile after the other (20 q8 organs 5.14 -> 4.95, 33 organs 7.6 ->
-//     7.25, with 7168 columns 21.3 -> 19.7; Q4 11,000 x 4096 6.7 -> 5.9, 33
-//     organs with 7168 columns 14.5 -> 13.1);
-//   * up to 2,048 tiles one wave per tile, 8 tiles side by side (binary 4.4 ->
-//     3.9, mixed 5.2 -> 4.6; 40 Q4 organs with 7168 columns: 25.4 -> 15.1), or
-//     four waves a tile for Q4 of up to 32 steps in at most five tiles a CU
-//     (20,000 x 2048 5.1 against 6.4; 50 organs 6.3 against 5.9) and for q8
-//     (33 organs 7.55 against 8.3, 64 organs 12.3 against 14.3) but the
-//     longest rows in few tiles (7168 columns, 33 organs 22.5 against 21.1, 64
-//     organs 36.1 against 38);
-//   * up to 4,096 tiles Q4 of more than 16 steps one wave per tile (100 organs
-//     with 7168 columns: 40 -> 31.5, four waves 33.7), q8 four waves (100
-//     organs 18.1), the short kinds one wave per tile, 4 side by side (mixed
-//     6.05 -> 5.63, binary 5.07 -> 4.88); Q4 of 16 steps walks (80 organs: 9.4
-//     against 9.8);
-//   * beyond, q8 (200 organs: 42.7 -> 36.6) and mixed (8.9 -> 8.05) up to the
-//     streamed shapes; the others' walk is faster (binary 320 organs: 9.7
+//     on one tile after the other (33 q8 organs 7.6 -> 7.25, with 7168 columns
+//     21.3 -> 19.7; Q4 11,000 x 4096 6.7 -> 5.9, 23 Q4 organs of 36 steps 8.0 ->
+//     6.6);
+//   * up to 2,048 tiles one wave per tile, 8/1/8 (binary 4.4 -> 3.9, mixed 5.2 ->
+//     4.6; 40 Q4 organs with 7168 columns: 25.4 -> 15.1), but up to five tiles a
+//     CU 8/4/2 for rows of four blocks (Q4 20,000 x 2048 5.1 against 6.4) and
+//     for five to eight 16/8/6 (40 Q4 organs of 26 steps 7.2, 8/8/1 8.0) or, q8,
+//     8/8/1 (of 26 steps 6.3, 16/8/6 6.4);
+//   * q8 rows whose blocks divide by eight, or long ones that about fill four
+//     waves: 8/4/2 above 1,280 tiles (64 organs 12.3 against 14.3, with 7168
+//     columns 36.1 against 38, 100 organs 18.1); others leave waves without a
+//     block, 8/1/8 (64 organs of 22 steps 8.4 against 9.3, of 36 steps 12.05
+//     against 13.1; 110 organs of 45 steps 22.8 against 23.7).  Q4 of more than 16 steps 8/1/8 up to 4,096 tiles
+//     (100 organs with 7168 columns: 40 -> 31.5, 8/4/2 33.7); of up to 16 steps it
+//     walks (80 organs: 9.4 against 9.8);
+//   * the short kinds 4/1/4 up to 4,096 tiles (mixed 6.05 -> 5.63, binary 5.07 ->
+//     4.88), mixed (8.9 -> 8.05) and q8 (200 organs: 42.7 -> 36.6) up to the
+//     streamed shapes; the others' walk is faster there (binary 320 organs: 9.7
 //     against 10.8; 200 Q4 organs: 20.1 against 19.9, with 7168 columns equal).
 // HEAD: every workgroup ends in one atomic max on the same word, which the
 // memory side takes at about 12 ns each (a binary 151,936 x 2048 lm_head: 15.1
 // us over 256 workgroups, 16.2 over 594, 23.2 over 1,187), so one or two
-// balanced workgroups per CU, 8 waves each.  One wave per tile for binary and
-// for short rows (q8 32,000 x 1024 11.3 against 12.2 with four waves a tile; Q4
-// 32,000 x 2048 12.3 against 13), eight waves for long rows in at most three
-// tiles a CU (q8 11,409 x 2048 10.8, four 11.1, one 11.4; Q4 11,409 x 4096 11.5,
-// 11.9, 12.5), four else (q8 151,936 x 2048 49.7; 65,000 rows 25.3; Q4 4096 x
-// 2048 8.2, one 9.0).  A q8 lm_head larger than the Infinity Cache loads
-// non-temporally with one workgroup per CU (128,256 x 4096: 96.2 -> 78; below,
-// the hint and the fewer loads in flight cost: 65,000 rows 25.9 -> 34.8; Q4 of
-// these sizes fits and gains nothing from it); tile counts that leave a nearly
-// empty last round cost up to 30 %.
+// balanced workgroups per CU, 8 waves each.  One wave per tile for binary, for
+// short rows (q8 32,000 x 1024 11.3 against 12.2 with four waves a tile) and for
+// rows whose blocks do not divide by four (q8 16,536 x 1408 10.6 against 11.9,
+// 65,000 x 2304 26.9 against 28.5, 151,936 x 3328 77.5 against 83.5; Q4 30,000 x
+// 2304 12.5 against 15.0), four else (q8 151,936 x 2048 49.7 against 52; 65,000
+// rows 25.3).  With at most two tiles a CU four waves, two for 17 to 23 steps
+// (q8 8,000 x 1408 9.6, four 10.2, one 9.9; x 2880 10.7, 11.6, 13.2); eight
+// where three tiles a workgroup give each CU one and the blocks divide (q8
+// 11,409 x 2048 10.8, four 11.1, one 11.4).  A q8 lm_head larger than the
+// Infinity Cache loads non-temporally with one workgroup per CU (128,256 x 4096:
+// 96.2 -> 78; below, the hint and the fewer loads in flight cost: 65,000 rows
+// 25.9 -> 34.8; Q4 of these sizes fits and gains nothing from it); tile counts
+// that leave a nearly empty last round cost up to 30 %.
 // RES (256 threads, at most 4 tiles a workgroup: a row's records are one
 // thread's chain) replaces two launches: one organ 7.8 -> 5.0, 40 organs 8.8
 // -> 6.6, 512 x 7168: 35.4 -> 8.7; above 4,096 tiles the two launches are
@@ -1366,44 +1373,53 @@ static uint32_t pow2_ceil(uint32_t v) {
 static SplitShape split_shape(int kind, bool res, bool head, uint32_t n, uint32_t n_tiles, uint32_t S, uint32_t cols) {
     const uint64_t tiles = (uint64_t)n * n_tiles;
     const bool wide = kind == HK_Q4 || kind == HK_Q8;
-    const uint32_t s2 = pow2_ceil(wide ? (S + 3u) / 4u : S);  // (a wave's least: a block of four steps)
+    const uint32_t nb = (S + 3u) / 4u;  // blocks of a Q4 or q8 row
     if (head) {
-        const bool walk = kind == HK_BIN || S <= 8 || (S <= 16 && tiles > 512 && tiles <= 2048);
-        const uint32_t ks = walk ? 1u : S >= 32 && tiles <= 768 ? 8u : 4u, ts = 8u / ks;
+        const uint32_t even = (uint32_t)((tiles + 255u) / 256u);
+        uint32_t ks = nb % 4u == 0 && (S > 16 || tiles > 2048) ? 4u : 1u;
+        if (tiles <= 512) ks = nb % 4u == 0 || S >= 24 ? 4u : 2u;
+        else if (even == 3 && nb % 8u == 0) ks = 8;
+        if (kind == HK_BIN || S <= 8) ks = 1;
+        const uint32_t ts = 8u / ks;
         const bool past_mall = kind == HK_Q8 && tiles * 16u * cols > MALL_BYTES;
         const uint32_t wgs = kind == HK_BIN || tiles <= 4096 || past_mall ? 256u : 512u;
-        const uint32_t even = (uint32_t)((tiles + wgs - 1u) / wgs);
-        return {8, ks, std::min((even + ts - 1u) / ts * ts, 64u)};
+        const uint32_t per_wg = (uint32_t)((tiles + wgs - 1u) / wgs);
+        return {8, ks, std::min((per_wg + ts - 1u) / ts * ts, 64u)};
     }
     const uint32_t tpw = std::min(pow2_ceil((uint32_t)((tiles + 255) / 256)), 4u);
     if (res) {
         if (tiles > 4096) return {0, 0, 0};
-        const uint32_t ks = std::min(std::max(4u / tpw, 1u), s2);
+        const uint32_t ks = std::min(std::max(4u / tpw, 1u), pow2_ceil(S));
         return {4, ks, std::max(tpw, 4u / ks)};
     }
     if (S == 1 || tiles >= 16384) return {0, 0, 0};
-    if (wide && S >= 32 && tiles > 512 && tiles <= 1280) {
+    if (!wide) {
+        if (tiles <= 1024) {
+            const uint32_t w = cols > 4096 || (S >= 16 && tpw == 4) ? 16u : S < 16 && tpw == 1 ? 4u : 8u;
+            const uint32_t ks = std::min(w / tpw, pow2_ceil(S));
+            return {w, ks, std::max(tpw, w / ks)};
+        }
+        if (tiles <= 2048) return {8, 1, 8};
+        return tiles <= 4096 || kind == HK_MIXED ? SplitShape{4, 1, 4} : SplitShape{0, 0, 0};
+    }
+    if (nb >= 8 && tiles > 512 && tiles <= 1280) {
         uint32_t even = 3;
         while (even < 5 && (uint64_t)n * ((n_tiles + even - 1u) / even) > 256u) ++even;
-        const uint32_t w = S >= 48 ? 16u : 8u;
-        if (even != 4 && (uint64_t)n * ((n_tiles + even - 1u) / even) <= 256u) return {w, w, even};
+        const uint32_t w = nb > 8 ? 16u : 8u;
+        const bool full = nb <= 16 || 4u * ((nb + 15u) / 16u) * 16u <= 5u * nb;  // (a wave's last block used)
+        if (full && even != 4 && (uint64_t)n * ((n_tiles + even - 1u) / even) <= 256u) return {w, w, even};
     }
+    if (nb >= 5 && nb <= 8 && ((tiles > 512 && tiles <= 704) || (tiles > 1024 && tiles <= 1280)))
+        return kind == HK_Q4 && tiles > 1024 ? SplitShape{16, 8, 6} : SplitShape{8, 8, 1};
     if (tiles <= 1024) {
-        const bool w16 = cols > 4096 || (S >= 16 && tpw == 4) || (wide && S >= (tpw == 1 ? 48u : 32u));
-        const bool w4 = wide ? s2 <= 2u && tpw <= 2u : S < 16 && tpw == 1;
-        const uint32_t w = w16 ? 16u : w4 ? 4u : 8u;
-        const uint32_t ks = std::min(w / tpw, s2);
+        const uint32_t w = nb <= 2 ? (tpw <= 2 ? 4u : 8u) : nb <= 4 ? (tpw == 4 ? 16u : 8u) : nb <= 8 && tpw == 1 ? 8u : 16u;
+        const uint32_t ks = std::min(w / tpw, pow2_ceil(nb));
         return {w, ks, std::max(tpw, w / ks)};
     }
-    if (tiles <= 2048) {
-        const bool four = kind == HK_Q8   ? S >= 16 && (S <= 64 || tiles > 1536)
-                          : kind == HK_Q4 ? S >= 16 && S <= 32 && tiles <= 1280
-                                          : false;
-        return four ? SplitShape{8, 4, 2} : SplitShape{8, 1, 8};
-    }
-    if (kind == HK_Q4 && S > 16 && tiles <= 4096) return {8, 1, 8};
-    if (kind == HK_Q8 && S >= (tiles <= 4096 ? 17u : 16u)) return {8, 4, 2};
-    if (!wide && (tiles <= 4096 || kind == HK_MIXED)) return {4, 1, 4};
+    if (nb == 4 && tiles <= 1280) return {8, 4, 2};
+    const bool four = kind == HK_Q8 && (nb % 8u == 0 || (nb >= 16 && (nb + 3u) / 4u * 4u * 8u <= 9u * nb));
+    if (tiles <= 2048 || (S > 16 && tiles <= 4096)) return four ? SplitShape{8, 4, 2} : SplitShape{8, 1, 8};
+    if (kind == HK_Q8 && S >= 16 && tiles > 4096) return {8, 4, 2};
     return {0, 0, 0};
 }
 
